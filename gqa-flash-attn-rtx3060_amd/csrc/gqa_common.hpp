@@ -95,6 +95,11 @@ __device__ constexpr int key_of(int v, int h) { return 16 * (v >> 3) + 8 * h + (
 // pi: M index of S^T -> key inside a 32-key block (swap bits 2 and 3).
 __device__ constexpr int pi_key(int m) { return (m & ~12) | ((m & 4) << 1) | ((m & 8) >> 1); }
 
+// n / d for 0 <= n < 2^31 (FastDiv of d, gqa_params.hpp).
+__device__ inline int fast_div(int n, uint32_t mul, uint32_t shift) {
+  return (int)((__umulhi((uint32_t)n, mul) + (uint32_t)n) >> shift);
+}
+
 // Value of x in lane (l ^ 32), combined with x by `op`.  v_permlane32_swap
 // exchanges the upper half of its first operand with the lower half of its
 // second; feeding x twice leaves {x[l%32], x[l%32+32]} in the two results.
@@ -352,10 +357,15 @@ __device__ inline void store_coherent(float* p, float v) {
 __device__ inline float load_coherent(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Four consecutive floats at byte offset `off` of buffer `r`, read the same
-// way (a 16-byte buffer load with sc1 set: cache-policy bit 4 on gfx950).
-__device__ inline f32x4 load_coherent4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 16));
+// Four consecutive floats at byte offset `off` + `soff` (wave-uniform) of
+// buffer `r`, read and written the same way (16-byte buffer accesses with sc1
+// set: cache-policy bit 4 on gfx950).
+__device__ inline f32x4 load_coherent4(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff = 0) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 16));
+}
+__device__ inline void store_coherent4(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, f32x4 v) {
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), r, off, soff, 16);
 }
 
 // ---------------------------------------------------------------------------

@@ -58,13 +58,6 @@ static_assert(kFusedMaxRowSplitsHost * 4 <= kDecTileBytes, "m (or l) of the fuse
 static_assert(256 * 16 <= kDecTileBytes && 32 * (kDecD / 4) * 16 <= kDecTileBytes,
               "the fused combine's split-group sums fit one LDS stage");
 
-// 16-byte device-coherent store (sc1: written through to the point where
-// all XCDs are coherent), through a buffer descriptor over the workspace.
-__device__ inline void store_coherent4(__amdgpu_buffer_rsrc_t r, uint32_t off, f32x4 v) {
-  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), r, off, 0, 16);
-}
-
 // Fused log-sum-exp combine of the R valid rows of one (b, kv head, 32-row
 // block) over all S splits (gqa_split.py:134-147), by one workgroup:
 //   1. m and l of every (row, split), and the accumulators of this thread's
@@ -638,7 +631,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const uint32_t ob = (uint32_t)((row * D + 32 * (db0 + d) + 4 * hh) * 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        store_coherent4(rw, ob + 32u * j,
+        store_coherent4(rw, ob, 32u * j,
                         f32x4{acc[d][4 * j], acc[d][4 * j + 1], acc[d][4 * j + 2], acc[d][4 * j + 3]});
     }
     // A sequence without keys stores m = 0, l = 0 (never produced otherwise:
@@ -1036,7 +1029,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.ws_acc, 0xFFFFFFF0u);
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
-      store_coherent4(rw, (uint32_t)((row * D + (D / 4) * wave + 16 * db + 4 * lg) * 4), acc[db]);
+      store_coherent4(rw, (uint32_t)((row * D + (D / 4) * wave + 16 * db + 4 * lg) * 4), 0, acc[db]);
     if (wave == 0 && lg == 0) {
       store_coherent(p.ws_m + row, skv == 0 ? 0.f : m_run * c);
       store_coherent(p.ws_l + row, l_tot);

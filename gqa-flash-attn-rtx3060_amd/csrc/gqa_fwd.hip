@@ -255,11 +255,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   const uint32_t kssb = (uint32_t)(2 * p.k.ss), vssb = (uint32_t)(2 * p.v.ss);
   auto decode = [&](int w, int i, int block_m) __attribute__((always_inline)) -> Item {
     Item x;
-    x.bh = w / n_items;
+    x.bh = fast_div(w, p.div_items.mul, p.div_items.shift);
     int idx = w - x.bh * n_items;
     int chunk = 0;
     if constexpr (chunked) {
-      chunk = idx / p.n_mblk;
+      chunk = fast_div(idx, p.div_mblk.mul, p.div_mblk.shift);
       idx -= chunk * p.n_mblk;
     }
     if (idx < p.n_split) {
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
       x.pid_m = dm.causal ? (p.n_mblk - 1 - mrank) : mrank;
       x.part = (x.pid_m >= p.n_mblk - p.n_split) ? 0 : -1;
     }
-    x.b = x.bh / dm.Hkv;
+    x.b = fast_div(x.bh, p.div_hkv.mul, p.div_hkv.shift);
     x.kvh = x.bh - x.b * dm.Hkv;
     // Keys of this sequence (paged: its own length, clamped to [0, Skv]),
     // and its query rows (variable lengths: q_len[b], tokens from q_start[b]).
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     x.tok0 = varlen ? (int64_t)load_uniform(p.q_start + x.b) : 0;
     // This lane's query row.
     const int r = wave * 32 + i;
-    const int g = r / block_m, ml = r - g * block_m;
+    const int g = (int)(__umul24(r, p.bm_mul) >> 16), ml = r - g * block_m;
     x.pos = x.pid_m * block_m + ml;
     x.valid = (g < dm.G) && (x.pos < x.sq);
     x.head = x.kvh * dm.G + (g < dm.G ? g : 0);
@@ -506,15 +506,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   // of stage 2 (tile indices relative to tb), then Q.  The tile loads go
   // first: the Q loads behind them touch 32 rows per instruction and, issued
   // first, held the tile loads back by ~2 us.  An invalid row loads row 0 of
-  // its sequence (always present here) and is zeroed.  Paged: returns the
-  // block(s) of the tile the first softmax phase issues.
+  // its sequence (always present here); it is zeroed once the loads have
+  // landed, so that they are all in flight together (a select beside each load
+  // made the compiler wait for every one of the eight in turn: 1.9-2.4 us per
+  // launch).  Paged: returns the block(s) of the tile the first softmax phase
+  // issues.
   auto prologue_q = [&](const Item& x) __attribute__((always_inline)) {
     const T* qrow = static_cast<const T*>(p.q.ptr) + row_off(x, p.q, x.valid ? x.pos : 0, x.head);
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(qrow + 16 * ks + 8 * hh);
-      qreg[ks] = x.valid ? v : u32x4{0u, 0u, 0u, 0u};
-    }
+    for (int ks = 0; ks < NKS; ++ks) qreg[ks] = *reinterpret_cast<const u32x4*>(qrow + 16 * ks + 8 * hh);
   };
   auto prologue_kv = [&](const Item& x) __attribute__((always_inline)) -> TileBlocks {
     TileBlocks bn = tile_block(x, x.tb);
@@ -664,6 +664,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     m_run = -__builtin_inff();
     l_run = 0.f;
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the prologue loads
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) pin(qreg[ks]);
+    if (__builtin_amdgcn_ballot_w64(!it.valid) != 0) {
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) qreg[ks] = it.valid ? qreg[ks] : u32x4{0u, 0u, 0u, 0u};
+    }
     phase_barrier();
     if (grp == 1) phase_barrier();  // group B runs one phase behind
 
@@ -722,14 +728,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     // slower on short key-split prefills when re-deriving them).
     int w_cur = item_at(k_item), zero = 0, bm = p.block_m;
     if constexpr (!PERSIST) asm volatile("" : "+s"(w_cur), "+s"(zero), "+s"(bm));
+    // The output rows' places are worked out here, not hoisted out of the
+    // item loop (where they delayed the first loads).
+    int wave_e = wave;
+    asm volatile("" : "+s"(wave_e));
     const int lane_e =
         PERSIST ? lane : (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, (unsigned)zero));
     const int t_e = wave * 64 + lane_e, i_e = lane_e & 31, hh_e = lane_e >> 5;
     const Item ie = PERSIST ? it : decode(w_cur, i_e, bm);
 
     // Split query block: publish this half's state (reference max, lane
-    // partial row sum, accumulators, lane-major so each lane of the other
-    // item reads back exactly its own row); the item that completes the
+    // partial row sum, accumulators in groups of four, lane-major so each lane
+    // of the other item reads back exactly its own row with 16-byte loads, all
+    // requested before the first is used); the item that completes the
     // block's counter merges the other half into its registers and writes o.
     // The counter is read first: when the other half has already published
     // (counter 1), this item is the last one and skips publishing its own.
@@ -740,6 +751,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     if (!chunked && ie.part >= 0) {
       constexpr int PF_ = kFwdPartFloats(D);
       constexpr int NA = NDB * 16;  // accumulators per lane
+      constexpr uint32_t kQuad = kFwdThreads * 16;  // bytes of one group of four
       const int slot = ie.bh * p.n_split + (p.n_mblk - 1 - ie.pid_m);
       float* mine = p.part_ws + ((int64_t)slot * 2 + ie.part) * PF_;
       const float* other = p.part_ws + ((int64_t)slot * 2 + (1 - ie.part)) * PF_;
@@ -747,10 +759,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
       __syncthreads();
       bool last = s_last;
       if (!last) {
+        const __amdgpu_buffer_rsrc_t rm = make_rsrc(mine, NDB * 4 * kQuad);
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) store_coherent(mine + (db * 16 + v) * kFwdThreads + t_e, acc[db][v]);
+          for (int j = 0; j < 4; ++j)
+            store_coherent4(rm, 16u * t_e, (db * 4 + j) * kQuad,
+                            f32x4{acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]});
         store_coherent(mine + NA * kFwdThreads + t_e, m_run);
         store_coherent(mine + (NA + 1) * kFwdThreads + t_e, l_run);
         __builtin_amdgcn_s_waitcnt(0);  // this thread's stores are done
@@ -768,8 +783,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
         // contraction included) does not depend on which half finished
         // last: repeated calls give identical outputs.
         const bool lo = ie.part == 0;
+        const __amdgpu_buffer_rsrc_t ro = make_rsrc(other, NDB * 4 * kQuad);
         const float m_o = load_coherent(other + NA * kFwdThreads + t_e);
         const float l_o = load_coherent(other + (NA + 1) * kFwdThreads + t_e);
+        f32x4 xo[NDB * 4];
+#pragma unroll
+        for (int j = 0; j < NDB * 4; ++j) xo[j] = load_coherent4(ro, 16u * t_e, j * kQuad);
+        __builtin_amdgcn_sched_barrier(0);
         const float m0 = lo ? m_run : m_o, m1 = lo ? m_o : m_run;
         const float mm = fmaxf(m0, m1);
         const float mu = (mm == -__builtin_inff()) ? 0.f : mm;
@@ -778,7 +798,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
-            const float x_o = load_coherent(other + (db * 16 + v) * kFwdThreads + t_e);
+            const float x_o = xo[db * 4 + (v >> 2)][v & 3];
             const float x0 = lo ? acc[db][v] : x_o, x1 = lo ? x_o : acc[db][v];
             acc[db][v] = __builtin_fmaf(x0, a0, x1 * a1);
           }
@@ -850,16 +870,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
             *reinterpret_cast<u32x2*>(ot + i_e * (2 * D) + ch * 16 + 8 * hh_e) = x;
           }
         __builtin_amdgcn_s_waitcnt(kLgkm0);  // this wave's LDS writes before its reads
-        const int cc = lane_e % CPR16;
+        const int cc = lane_e % CPR16, r0 = lane_e / CPR16;
+        if ((bm & 31) == 0) {
+          // The wave's 32 rows are consecutive positions of one head: one row
+          // address, advanced by RPI rows per store.
+          const int g2 = (int)(__umul24(wave_e * 32, p.bm_mul) >> 16);
+          const int pos2 = ie.pid_m * bm + (wave_e * 32 - g2 * bm) + r0;
+          T* orow = static_cast<T*>(const_cast<void*>(p.o.ptr)) + row_off(ie, p.o, pos2, ie.kvh * dm.G + g2) + 8 * cc;
+          const int left = g2 < dm.G ? ie.sq - pos2 : 0;  // rows from this one on
 #pragma unroll
-        for (int ri = 0; ri < 32 / RPI; ++ri) {
-          const int rr = RPI * ri + lane_e / CPR16;  // row of the tile
-          const u32x4 x = *reinterpret_cast<const u32x4*>(ot + rr * (2 * D) + ((cc ^ (rr & (CPR16 - 1))) * 16));
-          const int r2 = wave * 32 + rr;
-          const int g2 = r2 / bm, pos2 = ie.pid_m * bm + (r2 - g2 * bm);
-          if (g2 < dm.G && pos2 < ie.sq) {
-            T* orow = static_cast<T*>(const_cast<void*>(p.o.ptr)) + row_off(ie, p.o, pos2, ie.kvh * dm.G + g2);
-            *reinterpret_cast<u32x4*>(orow + 8 * cc) = x;
+          for (int ri = 0; ri < 32 / RPI; ++ri) {
+            const int rr = RPI * ri + r0;  // row of the tile
+            const u32x4 x = *reinterpret_cast<const u32x4*>(ot + rr * (2 * D) + ((cc ^ (rr & (CPR16 - 1))) * 16));
+            if (RPI * ri < left) *reinterpret_cast<u32x4*>(orow + (int64_t)(RPI * ri) * p.o.ss) = x;
+          }
+        } else {
+#pragma unroll 1
+          for (int ri = 0; ri < 32 / RPI; ++ri) {
+            const int rr = RPI * ri + r0;
+            const u32x4 x = *reinterpret_cast<const u32x4*>(ot + rr * (2 * D) + ((cc ^ (rr & (CPR16 - 1))) * 16));
+            const int r2 = wave_e * 32 + rr;
+            const int g2 = (int)(__umul24(r2, p.bm_mul) >> 16), pos2 = ie.pid_m * bm + (r2 - g2 * bm);
+            if (g2 < dm.G && pos2 < ie.sq) {
+              T* orow = static_cast<T*>(const_cast<void*>(p.o.ptr)) + row_off(ie, p.o, pos2, ie.kvh * dm.G + g2);
+              *reinterpret_cast<u32x4*>(orow + 8 * cc) = x;
+            }
           }
         }
       }
@@ -929,6 +964,10 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   const int per_bh = p.kv_splits > 0 ? p.n_mblk * p.kv_splits : p.n_mblk + p.n_split;
   const int total = per_bh * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
+  p.div_items = make_fast_div((uint32_t)per_bh);
+  p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
+  p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
+  p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;
   int grid = total;
   if (PG == 0 && D == 128) {
     const int cus = device_cu_count();

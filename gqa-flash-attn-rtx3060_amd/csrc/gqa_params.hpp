@@ -13,6 +13,21 @@ struct TensorRef {
   int64_t sb, sh, ss;  // batch, head, sequence strides
 };
 
+// Division of 0 <= n < 2^31 by a launch constant d (fast_div in
+// gqa_common.hpp): with l = ceil(log2 d) and m = floor(2^32 (2^l - d) / d) + 1,
+// n / d = (mulhi(m, n) + n) >> l (Granlund and Montgomery, "Division by
+// invariant integers using multiplication").  A kernel's integer divisions by
+// run-time values otherwise cost 25-40 dependent instructions each before its
+// first load is issued.
+struct FastDiv {
+  uint32_t mul, shift;
+};
+inline FastDiv make_fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (l < 32 && ((uint64_t)1 << l) < d) ++l;
+  return FastDiv{(uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - d)) / d + 1), l};
+}
+
 struct Dims {
   int B, Hq, Hkv, Sq, Skv, D, G;
   float c;  // head_dim^-0.5 * log2(e)
@@ -25,6 +40,11 @@ struct FwdParams {
   Dims dm;
   int block_m;  // query positions per workgroup (G * block_m <= kFwdRows packed rows)
   int n_mblk;   // ceil(Sq / block_m)
+  // Set by the launcher: division by the items per (b, kv head), by n_mblk
+  // and by Hkv, and ceil(2^16 / block_m): r / block_m = (r * bm_mul) >> 16 for
+  // r < kFwdRows.
+  FastDiv div_items, div_mblk, div_hkv;
+  uint32_t bm_mul;
   float* lse;   // optional (nullptr): natural-log LSE per row, contiguous (B, Hq, Sq)
   // Key-range split of the n_split heaviest query blocks of every (b, kv
   // head) into two work items (lower and upper half of the block's key

@@ -28,7 +28,8 @@ using gqa::TensorRef;
 // 11: gqa_fwd_chunks_launch (single pass over key chunks + split combine).
 // 12: gqa_paged_fwd_chunks_launch (the same over a paged cache).
 // 13: gqa_paged_fwd_split_launch (the paged single pass with split blocks).
-constexpr int kAbiVersion = 13;
+// 14: gqa_split_flat_launch, gqa_paged_split_flat_launch (flat splits).
+constexpr int kAbiVersion = 14;
 
 int check_dims(int B, int Hq, int Hkv, int Sq, int Skv, int D, int dtype) {
   if (B < 0 || Hq <= 0 || Hkv <= 0 || Sq < 0 || Skv < 0) return GQA_E_SHAPE;
@@ -92,6 +93,9 @@ const char* gqa_strerror(int code) {
       return "gqa_split_noalloc_launch: the split partials exceed its fixed buffer "
              "(GQA_NOALLOC_SCRATCH_BYTES, 16 MiB); use fewer splits or gqa_split_first_launch with a "
              "caller workspace";
+    case GQA_E_FLAT:
+      return "flat split: slots must be in [1, GQA_MAX_SPLITS] and the call one the LDS-DMA first pass takes with "
+             "at most 32 packed rows per kv head (16 at head_dim 64)";
     default: break;
   }
   if (code > 0) return hipGetErrorString(static_cast<hipError_t>(code));
@@ -437,6 +441,45 @@ int reduce_impl(const float* workspace, int splits, void* o, const int64_t o_str
                 int num_heads, int seq_q, int head_dim, int dtype, void* stream, const int* q_start = nullptr,
                 const int* q_len = nullptr);
 
+// A flat split (checked arguments): workspace as SplitParams::slots describes
+// it (acc, m, l, plan), first pass, then the combine unless the first pass
+// writes o.
+int flat_impl(gqa::SplitParams& p, float* workspace, void* o, const int64_t o_stride[4], float* lse, int dtype,
+              void* stream) {
+  const size_t rows = ((size_t)p.slots + p.dm.B) * p.dm.Hq * p.dm.Sq;
+  p.ws_acc = workspace;
+  p.ws_m = workspace + rows * p.dm.D;
+  p.ws_l = p.ws_m + rows;
+  p.plan = reinterpret_cast<int*>(p.ws_l + rows);
+  p.o = ref(o, o_stride);
+  p.lse = lse;
+  if (!gqa::decode_kernel_fits(p)) return GQA_E_FLAT;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int rc = to_code(gqa::launch_decode_first(p, dtype, st));
+  if (rc || p.direct) return rc;
+  gqa::ReduceParams r{};
+  r.ws_acc = p.ws_acc;
+  r.ws_m = p.ws_m;
+  r.ws_l = p.ws_l;
+  r.o = p.o;
+  r.B = p.dm.B;
+  r.Hq = p.dm.Hq;
+  r.Sq = p.dm.Sq;
+  r.D = p.dm.D;
+  r.splits = p.slots;  // at most this many partials per row
+  r.lse = lse;
+  r.q_start = p.q_start;
+  r.q_len = p.q_len;
+  if (p.block_table != nullptr) {
+    r.plan = p.plan;
+  } else {
+    const int unit = gqa::decode_unit(p.dm.D);
+    r.units = (p.dm.Skv + unit - 1) / unit;
+    r.slots = (int)std::min<int64_t>(p.slots, (int64_t)r.units * p.dm.B);
+  }
+  return to_code(gqa::launch_split_reduce(r, dtype, st));
+}
+
 }  // namespace
 
 extern "C" {
@@ -477,6 +520,84 @@ int gqa_split_launch(const void* q, const int64_t q_stride[4], const void* k, co
                               num_kv_heads, seq_q, seq_kv, head_dim, scale_log2, causal, dtype, stream);
   if (rc) return rc;
   return reduce_impl(workspace, splits, o, o_stride, lse, batch, num_heads, seq_q, head_dim, dtype, stream);
+}
+
+size_t gqa_split_flat_workspace_bytes(int batch, int num_heads, int seq_q, int head_dim, int slots) {
+  if (batch <= 0 || num_heads <= 0 || seq_q <= 0 || head_dim <= 0 || slots <= 0) return 0;
+  const size_t rows = ((size_t)slots + batch) * num_heads * seq_q;
+  return rows * ((size_t)head_dim + 2) * sizeof(float) + (size_t)batch * 2 * sizeof(int);
+}
+
+int gqa_split_flat_launch(const void* q, const int64_t q_stride[4], const void* k, const int64_t k_stride[4],
+                          const void* v, const int64_t v_stride[4], void* o, const int64_t o_stride[4], float* lse,
+                          float* workspace, int slots, int batch, int num_heads, int num_kv_heads, int seq_q,
+                          int seq_kv, int head_dim, float scale_log2, int causal, int dtype, void* stream) {
+  int rc = check_dims(batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, dtype);
+  if (rc) return rc;
+  if (slots < 1 || slots > GQA_MAX_SPLITS || seq_kv < 1) return GQA_E_FLAT;
+  if (batch == 0 || seq_q == 0) return GQA_OK;
+  if (workspace == nullptr) return GQA_E_NULL;
+  if (((reinterpret_cast<uintptr_t>(workspace) & 15u) | (reinterpret_cast<uintptr_t>(lse) & 3u)) != 0)
+    return GQA_E_STRIDE;
+  if ((rc = check_tensor(q, q_stride)) || (rc = check_tensor(o, o_stride)) || (rc = check_tensor(k, k_stride)) ||
+      (rc = check_tensor(v, v_stride)))
+    return rc;
+  gqa::SplitParams p{};
+  p.q = ref(q, q_stride);
+  p.k = ref(k, k_stride);
+  p.v = ref(v, v_stride);
+  const int G = num_heads / num_kv_heads;
+  p.dm = Dims{batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, G, scale_log2, causal ? 1 : 0};
+  p.splits = 1;
+  p.slots = slots;
+  p.chunk = seq_kv;  // the longest piece
+  p.n_rblk = (G * seq_q + 31) / 32;
+  p.rotate = p.k.ss == head_dim && p.v.ss == head_dim;
+  // One slot per sequence: each is one piece, written to o by the first pass.
+  p.direct = slots == batch;
+  return flat_impl(p, workspace, o, o_stride, lse, dtype, stream);
+}
+
+int gqa_paged_split_flat_launch(const void* q, const int64_t q_stride[4], const void* k_cache,
+                                const int64_t k_cache_stride[4], const void* v_cache,
+                                const int64_t v_cache_stride[4], const int* block_table, int table_stride,
+                                const int* seq_lens, const int* q_start, const int* q_len, int block_size,
+                                int max_seq_len, void* o, const int64_t o_stride[4], float* lse, float* workspace,
+                                int slots, int batch, int num_heads, int num_kv_heads, int seq_q, int head_dim,
+                                float scale_log2, int causal, int dtype, void* stream) {
+  int rc = check_dims(batch, num_heads, num_kv_heads, seq_q, max_seq_len, head_dim, dtype);
+  if (rc) return rc;
+  if (block_size < 1 || block_size > GQA_MAX_BLOCK_SIZE || (block_size & (block_size - 1)) != 0)
+    return GQA_E_BLOCK;
+  if (table_stride < 0 || (int64_t)table_stride * block_size < (int64_t)max_seq_len) return GQA_E_BLOCK;
+  if (slots < 1 || slots > GQA_MAX_SPLITS || max_seq_len < 1) return GQA_E_FLAT;
+  if (batch == 0 || seq_q == 0) return GQA_OK;
+  if (workspace == nullptr || seq_lens == nullptr || block_table == nullptr) return GQA_E_NULL;
+  if (((reinterpret_cast<uintptr_t>(workspace) & 15u) |
+       ((reinterpret_cast<uintptr_t>(seq_lens) | reinterpret_cast<uintptr_t>(block_table) |
+         reinterpret_cast<uintptr_t>(lse)) & 3u)) != 0)
+    return GQA_E_STRIDE;
+  if ((rc = check_varlen(q_start, q_len))) return rc;
+  if ((rc = check_tensor(q, q_stride)) || (rc = check_tensor(o, o_stride)) ||
+      (rc = check_tensor(k_cache, k_cache_stride)) || (rc = check_tensor(v_cache, v_cache_stride)))
+    return rc;
+  gqa::SplitParams p{};
+  p.q = ref(q, q_stride);
+  p.k = cache_ref(k_cache, k_cache_stride);
+  p.v = cache_ref(v_cache, v_cache_stride);
+  const int G = num_heads / num_kv_heads;
+  p.dm = Dims{batch, num_heads, num_kv_heads, seq_q, max_seq_len, head_dim, G, scale_log2, causal ? 1 : 0};
+  p.splits = 1;
+  p.slots = slots;
+  p.n_rblk = (G * seq_q + 31) / 32;
+  p.block_table = block_table;
+  p.seq_lens = seq_lens;
+  p.table_stride = table_stride;
+  while ((1 << p.block_shift) < block_size) ++p.block_shift;
+  p.rotate = p.k.ss == head_dim && p.v.ss == head_dim;
+  p.q_start = q_start;
+  p.q_len = q_len;
+  return flat_impl(p, workspace, o, o_stride, lse, dtype, stream);
 }
 
 int gqa_split_reduce_launch(const float* workspace, int splits, void* o, const int64_t o_stride[4], int batch,

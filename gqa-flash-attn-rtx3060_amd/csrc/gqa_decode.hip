@@ -38,6 +38,7 @@
 // (b, kv head, row block) to count its partial in combines all splits
 // (gqa_split.py:134-147) with one round of global loads — m and l of every
 // (row, split) and this thread's accumulators are requested together.
+#include <algorithm>
 #include <type_traits>
 
 #include "gqa_common.hpp"
@@ -202,6 +203,154 @@ __device__ void decode_combine(const SplitParams& p, int b, int kvh, int rb, int
   }
 }
 
+// Workspace row of the partial of (b, head, pos) from split (or slot) s.
+__device__ inline int64_t partial_row(const SplitParams& p, bool flat, int b, int head, int pos, int s) {
+  return flat ? ((int64_t)(s + b) * p.dm.Hq + head) * p.dm.Sq + pos
+              : (((int64_t)b * p.dm.Hq + head) * p.dm.Sq + pos) * p.splits + s;
+}
+
+// A row whose only split this was (SplitParams::direct): o = acc / l, and its
+// LSE from one lane (`lse_lane`), as the combine of a single partial gives
+// them: NaN and -inf for a row with no visible key, zeros and -inf for a
+// sequence without keys.  each(put): put(dim, f32x4) for this lane's dims.
+template <int DT, typename F>
+__device__ inline void store_rows_direct(const SplitParams& p, int b, int head, int pos, bool varlen, int64_t tok0,
+                                         int skv, float m2, float l, bool lse_lane, F each) {
+  using E = Elem<DT>;
+  using T = typename E::T;
+  if (p.lse != nullptr && lse_lane)
+    p.lse[varlen ? (tok0 + pos) * p.dm.Hq + head : ((int64_t)b * p.dm.Hq + head) * p.dm.Sq + pos] =
+        (skv == 0 || m2 == -__builtin_inff()) ? -__builtin_inff() : (m2 + __log2f(l)) * kLn2;
+  const float lu = skv == 0 ? __builtin_inff() : l;
+  T* orow = static_cast<T*>(const_cast<void*>(p.o.ptr)) + (int64_t)head * p.o.sh +
+            (varlen ? (tok0 + pos) * p.o.ss : (int64_t)b * p.o.sb + (int64_t)pos * p.o.ss);
+  each([&](int dim, f32x4 a) {
+    u32x2 x;
+    x[0] = E::pack2(a[0] / lu, a[1] / lu);
+    x[1] = E::pack2(a[2] / lu, a[3] / lu);
+    *reinterpret_cast<u32x2*>(orow + dim) = x;
+  });
+}
+
+// Sum of n over the wave's lanes 0..lane (row shifts, then row broadcasts).
+__device__ inline int wave_scan(int n) {
+  n += __builtin_amdgcn_update_dpp(0, n, 0x111, 0xF, 0xF, true);   // row_shr:1
+  n += __builtin_amdgcn_update_dpp(0, n, 0x112, 0xF, 0xF, true);   // row_shr:2
+  n += __builtin_amdgcn_update_dpp(0, n, 0x114, 0xF, 0xF, true);   // row_shr:4
+  n += __builtin_amdgcn_update_dpp(0, n, 0x118, 0xF, 0xF, true);   // row_shr:8
+  n += __builtin_amdgcn_update_dpp(0, n, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  n += __builtin_amdgcn_update_dpp(0, n, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return n;
+}
+
+// The pieces of one slot of a flat split (SplitParams::slots): ranges of
+// consecutive tile steps ("units" of TK keys) of one sequence each, in order.
+// The slot's range is [j * T / slots, (j + 1) * T / slots) of the T units of
+// all sequences (with fewer units than slots, unit j alone, so that no slot
+// between two pieces of a sequence is empty); every value is wave-uniform except a lane's own sequence in
+// the scans (each wave works the ranges out for itself: the lengths live on
+// the device).
+template <int TK, bool PAGED> struct FlatWalk {
+  int at, end;      // units of the flat order still to do
+  int b, u0, n;     // current sequence, its first unit in the flat order, its units
+  int base, carry;  // paged: first sequence of the scanned group of 64, units before it
+  int incl, own;    // paged, per lane: scan over the group, this lane's sequence's units
+  int len, skv;     // ... and keys; keys of the current sequence
+
+  // Units of sequence `s` (per lane): none without query rows.
+  __device__ static int units(const SplitParams& p, int s, int& len) {
+    len = 0;
+    if (s >= p.dm.B) return 0;
+    len = min(max(p.seq_lens[s], 0), p.dm.Skv);
+    return p.q_len != nullptr && p.q_len[s] <= 0 ? 0 : (len + TK - 1) / TK;
+  }
+  __device__ static int units(const SplitParams& p, int s) {
+    int l;
+    return units(p, s, l);
+  }
+  __device__ void scan(const SplitParams& p, int lane) {
+    own = units(p, base + lane, len);
+    incl = wave_scan(own);
+  }
+  __device__ static int last(int v) { return __builtin_amdgcn_readlane(v, 63); }
+
+  __device__ void start(const SplitParams& p, int slot, int lane) {
+    int total = 0;
+    if constexpr (PAGED) {
+      for (int g0 = p.dm.B > 64 ? 64 : p.dm.B; g0 < p.dm.B; g0 += 64) total += last(wave_scan(units(p, g0 + lane)));
+      base = 0;
+      carry = 0;
+      scan(p, lane);
+      total += last(incl);
+    } else {
+      n = (p.dm.Skv + TK - 1) / TK;
+      total = n * p.dm.B;
+    }
+    if (total < p.slots) {
+      at = min(slot, total);
+      end = min(slot + 1, total);
+    } else {
+      at = fast_div(slot * total, p.div_splits.mul, p.div_splits.shift);
+      end = fast_div((slot + 1) * total, p.div_splits.mul, p.div_splits.shift);
+    }
+    if constexpr (PAGED) {
+      b = 0;
+      u0 = 0;
+      n = 0;
+    } else if (at < end) {
+      b = fast_div(at, p.div_units.mul, p.div_units.shift);
+      u0 = b * n;
+    }
+  }
+
+  // Paged: (first partial, number of partials) of every sequence for the
+  // combine, by one wave: unit t lies in slot ((t + 1) * slots - 1) / T.
+  // (Contiguous sequences are equally long: the combine works it out.)
+  __device__ static void plan(const SplitParams& p, int lane) {
+    int total = 0, before = 0;
+    for (int g0 = 0; g0 < p.dm.B; g0 += 64) total += last(wave_scan(units(p, g0 + lane)));
+    const int slots = min(p.slots, total);
+    for (int g0 = 0; g0 < p.dm.B; g0 += 64) {
+      const int s = g0 + lane, mine = units(p, s);
+      const int upto = wave_scan(mine) + before;
+      before = last(upto);
+      if (s < p.dm.B) {
+        int first = 0, count = 0;
+        if (mine > 0) {
+          first = ((upto - mine + 1) * slots - 1) / total;
+          count = (upto * slots - 1) / total - first + 1;
+        }
+        p.plan[2 * s] = first + s;
+        p.plan[2 * s + 1] = count;
+      }
+    }
+  }
+
+  // The next piece: units [from, from + cnt) of sequence b.
+  __device__ bool next(const SplitParams& p, int lane, int& from, int& cnt) {
+    if (at >= end) return false;
+    if constexpr (PAGED) {
+      while (at >= carry + last(incl)) {  // (ends: at < T)
+        carry += last(incl);
+        base += 64;
+        scan(p, lane);
+      }
+      const int l = __builtin_ffsll((long long)__builtin_amdgcn_ballot_w64(carry + incl > at)) - 1;
+      b = base + l;
+      n = __builtin_amdgcn_readlane(own, l);
+      skv = __builtin_amdgcn_readlane(len, l);
+      u0 = carry + __builtin_amdgcn_readlane(incl, l) - n;
+    } else if (at >= u0 + n) {
+      ++b;
+      u0 += n;
+    }
+    from = at - u0;
+    cnt = min(end, u0 + n) - at;
+    at += cnt;
+    return true;
+  }
+};
+
 }  // namespace
 
 // KV: 0 contiguous K/V; 1 a paged cache with pages of >= 64 keys (one
@@ -214,7 +363,7 @@ __device__ void decode_combine(const SplitParams& p, int b, int kvh, int rb, int
 // min(seq_lens[b], Skv) keys.  With q_start / q_len set, q is token-major and
 // sequence b has q_len[b] query rows from token q_start[b].
 // RW: 32-row blocks per workgroup (1, 2 or 4).
-template <int DT, int KV, int RW>
+template <int DT, int KV, int RW, bool FLAT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gqa_decode_kernel(SplitParams p) {
   constexpr int D = kDecD;
   constexpr bool PAGED = KV != 0;
@@ -256,38 +405,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int db0 = ((wave % WPR) / KS) * NDB;
 
   const int n_wblk = (p.n_rblk + RW - 1) / RW;
-  const int total = dm.B * dm.Hkv * n_wblk * p.splits;
+  constexpr bool flat = FLAT;
+  const int per = flat ? p.slots : p.splits;
+  const int total = (flat ? 1 : dm.B) * dm.Hkv * n_wblk * per;
   const int w = xcd_remap(blockIdx.x, total);
-  const int s = w % p.splits;
-  int rest = w / p.splits;
-  const int rbw = rest % n_wblk;
-  rest /= n_wblk;
-  const int kvh = rest % dm.Hkv;
-  const int b = rest / dm.Hkv;
+  int rest = fast_div(w, p.div_splits.mul, p.div_splits.shift);
+  const int s = w - rest * per;
+  const int rest2 = fast_div(rest, p.div_wblk.mul, p.div_wblk.shift);
+  const int rbw = rest - rest2 * n_wblk;
+  int b = flat ? 0 : fast_div(rest2, p.div_hkv.mul, p.div_hkv.shift);
+  const int kvh = rest2 - b * dm.Hkv;
   const int rb = RW * rbw + rh;  // this wave's 32-row block
+  const bool varlen = p.q_len != nullptr;
+  const int wr0 = 32 * RW * rbw;  // the workgroup's first packed row
+  // This lane's query row (position-major packing), the workgroup's first
+  // and last positions.
+  const int r = 32 * rb + i;
+  const int pos = fast_div(r, p.div_g.mul, p.div_g.shift), g = r - pos * dm.G;
+  const int head = kvh * dm.G + g;
+  const int pos_lo = fast_div(wr0, p.div_g.mul, p.div_g.shift);
+  const int pos_end = fast_div(wr0 + 32 * RW - 1, p.div_g.mul, p.div_g.shift);
+  FlatWalk<64, PAGED> walk;
+  bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
+  if constexpr (flat) walk.start(p, s, lane);
+  // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
+  for (;;) {
+  int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
+  if constexpr (flat) {
+    int from, cnt;
+    if (!walk.next(p, lane, from, cnt)) {
+      if (plan_due) walk.plan(p, lane);  // (no sequence has keys)
+      return;
+    }
+    b = walk.b;
+    c0 = from * 64;
+    len = cnt * 64;
+  }
   // Keys of this sequence (paged: its own length, clamped to [0, Skv], so no
   // key past the block table's covered range is addressed) and its query
   // rows (variable lengths: q_len[b] rows from token q_start[b]).
-  const int skv = PAGED ? min(max(load_uniform(p.seq_lens + b), 0), dm.Skv) : dm.Skv;
-  const bool varlen = p.q_len != nullptr;
+  const int skv = !PAGED ? dm.Skv : flat ? walk.skv : min(max(load_uniform(p.seq_lens + b), 0), dm.Skv);
   const int sq = varlen ? min(max(load_uniform(p.q_len + b), 0), dm.Sq) : dm.Sq;
   const int64_t tok0 = varlen ? (int64_t)load_uniform(p.q_start + b) : 0;
-  const int wr0 = 32 * RW * rbw;        // the workgroup's first packed row
-  if (wr0 / dm.G >= sq) return;          // a row block past this sequence's queries
-
-  // This lane's query row (position-major packing).
-  const int r = 32 * rb + i;
-  const int pos = r / dm.G, g = r - pos * dm.G;
+  if (pos_lo >= sq) {  // a row block past this sequence's queries
+    if (flat) continue;
+    return;
+  }
   const bool valid = pos < sq;
-  const int head = kvh * dm.G + g;
   const int qpos = pos + (skv - sq);
 
-  // Keys of this chunk (gqa_split.py:55-60), clamped to the block's last
+  // Keys of this piece (gqa_split.py:55-60), clamped to the block's last
   // visible key under causal.
-  const int c0 = s * p.chunk;
-  int c1 = min(c0 + p.chunk, skv);
-  const int pos_lo = wr0 / dm.G;
-  const int pos_hi = min(sq - 1, (wr0 + 32 * RW - 1) / dm.G);
+  int c1 = min(c0 + len, skv);
+  const int pos_hi = min(sq - 1, pos_end);
   if (dm.causal) c1 = min(c1, pos_hi + (skv - sq) + 1);
   const int nk = max(c1 - c0, 0);
   const int ntiles = (nk + 63) >> 6;
@@ -415,6 +585,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       qreg[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 32u * ks, 0, 0));
   }
   issue(1, lds_c_k1, lds_d_v1);
+  // (While the first piece's loads are in flight.)
+  if (plan_due) walk.plan(p, lane);
+  plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).  Waiting here,
   // explicitly, also settles Q for the compiler: otherwise it waits for
   // every load in flight before entering the tile loop.
@@ -566,15 +739,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   using I1 = std::integral_constant<int, 1>;
   using BT = std::true_type;
   using BF = std::false_type;
-  // Tiles in pairs (stage 0, stage 1); an odd count is padded with one tile
-  // past the chunk (zeros, every key masked: it adds nothing).
-  const int ne = (ntiles + 1) & ~1;
+  // Tiles in pairs (stage 0, stage 1); the last one or two refill nothing.
   int it = 0;
-  for (; it + 4 <= ne; it += 2) {
+  for (; it + 4 <= ((ntiles + 1) & ~1); it += 2) {
     step(I0{}, BT{}, BF{}, it);
     step(I1{}, BT{}, BF{}, it + 1);
   }
-  if (it < ne) {
+  if (it + 1 == ntiles) {
+    step(I0{}, BF{}, BT{}, it);
+  } else if (it < ntiles) {
     step(I0{}, BF{}, BF{}, it);
     step(I1{}, BF{}, BT{}, it + 1);
   }
@@ -623,8 +796,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // 32 * (db0 + d) + 8 * j + 4 * hh + 0..3 in acc[d][4j .. 4j + 3].  With
   // two key groups, group 0 holds the merged state.
   const float l_tot = xhalf_sum(l_run);
+  if (FLAT && p.direct) {
+    if (valid && kh == 0)
+      store_rows_direct<DT>(p, b, head, pos, varlen, tok0, skv, m_run * c, l_tot, db0 == 0 && hh == 0,
+                            [&](auto put) {
+#pragma unroll
+                              for (int d = 0; d < NDB; ++d)
+#pragma unroll
+                                for (int j = 0; j < 4; ++j)
+                                  put(32 * (db0 + d) + 8 * j + 4 * hh,
+                                      f32x4{acc[d][4 * j], acc[d][4 * j + 1], acc[d][4 * j + 2], acc[d][4 * j + 3]});
+                            });
+    return;
+  }
   if (valid && kh == 0) {
-    const int64_t row = (((int64_t)b * dm.Hq + head) * dm.Sq + pos) * p.splits + s;
+    const int64_t row = partial_row(p, flat, b, head, pos, s);
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.ws_acc, 0xFFFFFFF0u);
 #pragma unroll
     for (int d = 0; d < NDB; ++d) {
@@ -643,6 +829,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
 
+  if constexpr (FLAT) continue;
   if (PAGED || p.counters == nullptr) return;
   // Fused combine: count this partial once its stores have completed; the
   // workgroup completing the count for this (b, kv head, row block) combines
@@ -662,11 +849,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // One call site in a loop (a second inlined copy of the combine would
   // put its register arrays on the stack).
 #pragma unroll 1
-  for (int rbc = RW * rbw; rbc < RW * rbw + RW && rbc < p.n_rblk && (32 * rbc) / dm.G < sq; ++rbc) {
+  for (int rbc = RW * rbw; rbc < RW * rbw + RW && rbc < p.n_rblk &&
+                           fast_div(32 * rbc, p.div_g.mul, p.div_g.shift) < sq; ++rbc) {
     if (rbc > RW * rbw) __syncthreads();  // the previous combine's LDS reads are done
     decode_combine<DT>(p, b, kvh, rbc, t, reinterpret_cast<float*>(lds_a_k0), reinterpret_cast<float*>(lds_b_v0),
                        reinterpret_cast<float*>(lds_d_v1), reinterpret_cast<f32x4*>(lds_c_k1));
   }
+  return;
+  }  // pieces
 }
 
 // ---------------------------------------------------------------------------
@@ -698,7 +888,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // and r & 6 gives their four 32-byte pieces four distinct bank groups); the
 // fused combine is not built for it (its callers take the two-launch form).
 // ---------------------------------------------------------------------------
-template <int DT, int KV, int D = kDecD>
+template <int DT, int KV, bool FLAT, int D = kDecD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gqa_decode16_kernel(SplitParams p) {
   static_assert(D == 128 || D == 64, "head_dim 64 or 128");
   constexpr bool PAGED = KV != 0;
@@ -729,29 +919,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6) & 3;
   const int i16 = lane & 15, lg = lane >> 4;
 
-  const int total = dm.B * dm.Hkv * p.splits;  // one row block per (b, kv head)
+  // One row block per (b, kv head): work item (kv head or (b, kv head), split
+  // or slot).
+  constexpr bool flat = FLAT;
+  const int per = flat ? p.slots : p.splits;
+  const int total = (flat ? 1 : dm.B) * dm.Hkv * per;
   const int w = xcd_remap(blockIdx.x, total);
-  const int s = w % p.splits;
-  const int rest = w / p.splits;
-  const int kvh = rest % dm.Hkv;
-  const int b = rest / dm.Hkv;
-  const int skv = PAGED ? min(max(load_uniform(p.seq_lens + b), 0), dm.Skv) : dm.Skv;
+  const int rest = fast_div(w, p.div_splits.mul, p.div_splits.shift);
+  const int s = w - rest * per;
+  int b = flat ? 0 : fast_div(rest, p.div_hkv.mul, p.div_hkv.shift);
+  const int kvh = rest - b * dm.Hkv;
   const bool varlen = p.q_len != nullptr;
+  // This lane's query row (position-major packing).
+  const int pos = fast_div(i16, p.div_g.mul, p.div_g.shift), g = i16 - pos * dm.G;
+  const int head = kvh * dm.G + g;
+  FlatWalk<TK, PAGED> walk;
+  bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
+  if constexpr (flat) walk.start(p, s, lane);
+  // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
+  for (;;) {
+  int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
+  if constexpr (flat) {
+    int from, cnt;
+    if (!walk.next(p, lane, from, cnt)) {
+      if (plan_due) walk.plan(p, lane);  // (no sequence has keys)
+      return;
+    }
+    b = walk.b;
+    c0 = from * TK;
+    len = cnt * TK;
+  }
+  const int skv = !PAGED ? dm.Skv : flat ? walk.skv : min(max(load_uniform(p.seq_lens + b), 0), dm.Skv);
   const int sq = varlen ? min(max(load_uniform(p.q_len + b), 0), dm.Sq) : dm.Sq;
   const int64_t tok0 = varlen ? (int64_t)load_uniform(p.q_start + b) : 0;
   if (sq <= 0) return;  // a sequence without query rows (variable lengths)
-
-  // This lane's query row (position-major packing).
-  const int pos = i16 / dm.G, g = i16 - pos * dm.G;
   const bool valid = pos < sq;
-  const int head = kvh * dm.G + g;
   const int qpos = pos + (skv - sq);
 
-  // Keys of this chunk (gqa_split.py:55-60), clamped to the block's last
+  // Keys of this piece (gqa_split.py:55-60), clamped to the block's last
   // visible key under causal.
-  const int c0 = s * p.chunk;
-  int c1 = min(c0 + p.chunk, skv);
-  const int pos_hi = min(sq - 1, 15 / dm.G);
+  int c1 = min(c0 + len, skv);
+  const int pos_hi = min(sq - 1, fast_div(15, p.div_g.mul, p.div_g.shift));
   if (dm.causal) c1 = min(c1, pos_hi + (skv - sq) + 1);
   const int nk = max(c1 - c0, 0);
   const int ntiles = (nk + TK - 1) / TK;
@@ -864,6 +1072,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       qreg[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 64u * ks, 0, 0));
   }
   issue(1, lds_c_k1, lds_d_v1);
+  // (While the first piece's loads are in flight.)
+  if (plan_due) walk.plan(p, lane);
+  plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * NI * NSUB));
 
@@ -1005,27 +1216,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   using I1 = std::integral_constant<int, 1>;
   using BT = std::true_type;
   using BF = std::false_type;
-  // Tiles in pairs; an odd count is padded with one tile past the chunk
-  // (zeros, every key masked); the last pair refills nothing.
-  const int ne = (ntiles + 1) & ~1;
+  // Tiles in pairs; the last one or two refill nothing.
   int it = 0;
-  for (; it + 4 <= ne; it += 2) {
+  for (; it + 4 <= ((ntiles + 1) & ~1); it += 2) {
     step(I0{}, BT{}, BF{}, it);
     step(I1{}, BT{}, BF{}, it + 1);
   }
-  if (it < ne) {
+  if (it + 1 == ntiles) {
+    step(I0{}, BF{}, BT{}, it);
+  } else if (it < ntiles) {
     step(I0{}, BF{}, BF{}, it);
     step(I1{}, BF{}, BT{}, it + 1);
   }
   __builtin_amdgcn_s_setprio(0);
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 
-  // This wave's dims of the valid rows' partials: lane (i16, lg) holds dims
-  // (D / 4) wave + 16 db + 4 lg + 0..3 in acc[db]; l is summed over the 4 lane
-  // groups (each holds the sum over its own keys).
+  // This wave's dims of the valid rows: lane (i16, lg) holds dims (D / 4) wave
+  // + 16 db + 4 lg + 0..3 in acc[db]; l is summed over the 4 lane groups (each
+  // holds the sum over its own keys).
   const float l_tot = xhalf_sum(xquad_sum(l_run));
+  if (FLAT && p.direct) {
+    if (valid)
+      store_rows_direct<DT>(p, b, head, pos, varlen, tok0, skv, m_run * c, l_tot, wave == 0 && lg == 0,
+                            [&](auto put) {
+#pragma unroll
+                              for (int db = 0; db < NDB; ++db) put((D / 4) * wave + 16 * db + 4 * lg, acc[db]);
+                            });
+    return;
+  }
   if (valid) {
-    const int64_t row = (((int64_t)b * dm.Hq + head) * dm.Sq + pos) * p.splits + s;
+    const int64_t row = partial_row(p, flat, b, head, pos, s);
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.ws_acc, 0xFFFFFFF0u);
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -1035,8 +1255,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       store_coherent(p.ws_l + row, l_tot);
     }
   }
+  if constexpr (!FLAT) break;
+  }  // pieces
 
-  if (PAGED || D != kDecD || p.counters == nullptr) return;
+  if (FLAT || PAGED || D != kDecD || p.counters == nullptr) return;
   // Fused combine, as gqa_decode_kernel.
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -1054,6 +1276,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 bool decode_kernel_fits(const SplitParams& p) {
   const int D = p.dm.D;
+  // Flat splits: one 32-row block per kv head (two or four with the walk's
+  // state spill registers); 32-bit products of units and slots.
+  const bool flat = p.slots > 0;
+  if (flat && (p.n_rblk != 1 || p.counters != nullptr)) return false;
+  const int unit = decode_unit(D);
+  if (flat && ((int64_t)((p.dm.Skv + unit - 1) / unit) * p.dm.B + 1) * (p.slots + 1) >= ((int64_t)1 << 31)) return false;
   // Head_dim 64: the 16-row first pass only (at most 16 packed rows per kv
   // head), in the two-launch form (no fused combine at that width).
   if (D == 64) {
@@ -1070,7 +1298,8 @@ bool decode_kernel_fits(const SplitParams& p) {
   // 64-row sub-tile; the whole accumulator workspace.
   const int64_t span = paged ? 64 : (int64_t)p.chunk + (D == 64 ? 256 : 128);
   if (span * p.k.ss * 2 >= ((int64_t)1 << 31) || span * p.v.ss * 2 >= ((int64_t)1 << 31)) return false;
-  const int64_t acc_bytes = (int64_t)p.dm.B * p.dm.Hq * p.dm.Sq * p.splits * D * 4;
+  const int64_t acc_bytes =
+      (flat ? (int64_t)p.slots + p.dm.B : (int64_t)p.dm.B * p.splits) * p.dm.Hq * p.dm.Sq * D * 4;
   // ... and a kv head's query group (its G heads x Sq rows).
   const int64_t q_bytes = 2 * ((int64_t)(p.dm.G - 1) * p.q.sh + (int64_t)(p.dm.Sq - 1) * p.q.ss + D);
   return acc_bytes <= 0xFFFFFFF0ll && q_bytes < ((int64_t)1 << 31);
@@ -1078,27 +1307,39 @@ bool decode_kernel_fits(const SplitParams& p) {
 
 // Every 32-row block of a kv head in one workgroup up to four (each K/V
 // chunk is then streamed once per 64 or 128 rows, not per 32).
-template <int DT, int KV>
-static hipError_t launch_decode_t(const SplitParams& p, hipStream_t stream) {
+template <int DT, int KV, bool FLAT>
+static hipError_t launch_decode_t(SplitParams p, hipStream_t stream) {
   const int rw = p.n_rblk >= 3 ? 4 : p.n_rblk == 2 ? 2 : 1;
-  const int64_t total = (int64_t)p.dm.B * p.dm.Hkv * ((p.n_rblk + rw - 1) / rw) * p.splits;
+  const int n_wblk = (p.n_rblk + rw - 1) / rw, per = p.slots > 0 ? p.slots : p.splits;
+  const int64_t total = (int64_t)(p.slots > 0 ? 1 : p.dm.B) * p.dm.Hkv * n_wblk * per;
   if (total <= 0) return hipSuccess;
+  const int unit = decode_unit(p.dm.D);
+  p.div_splits = make_fast_div((uint32_t)per);
+  p.div_wblk = make_fast_div((uint32_t)n_wblk);
+  p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
+  p.div_g = make_fast_div((uint32_t)p.dm.G);
+  p.div_units = make_fast_div((uint32_t)std::max((p.dm.Skv + unit - 1) / unit, 1));
+  const dim3 grid((unsigned)total), block(256);
   if (p.dm.D == 64)  // decode_kernel_fits: at most 16 packed rows
-    hipLaunchKernelGGL((gqa_decode16_kernel<DT, KV, 64>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gqa_decode16_kernel<DT, KV, FLAT, 64>), grid, block, 0, stream, p);
   else if (p.dm.G * p.dm.Sq <= 16)
-    hipLaunchKernelGGL((gqa_decode16_kernel<DT, KV>), dim3((unsigned)total), dim3(256), 0, stream, p);
-  else if (rw == 4)
-    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 4>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gqa_decode16_kernel<DT, KV, FLAT>), grid, block, 0, stream, p);
+  else if (rw == 1)
+    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 1, FLAT>), grid, block, 0, stream, p);
+  else if constexpr (FLAT)
+    return hipErrorInvalidValue;  // decode_kernel_fits: one 32-row block
   else if (rw == 2)
-    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 2>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 2, false>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 1>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((gqa_decode_kernel<DT, KV, 4, false>), grid, block, 0, stream, p);
   return hipGetLastError();
 }
 
 template <int KV>
 static hipError_t launch_decode_kv(const SplitParams& p, int dtype, hipStream_t stream) {
-  return dtype == 0 ? launch_decode_t<0, KV>(p, stream) : launch_decode_t<1, KV>(p, stream);
+  if (p.slots > 0)
+    return dtype == 0 ? launch_decode_t<0, KV, true>(p, stream) : launch_decode_t<1, KV, true>(p, stream);
+  return dtype == 0 ? launch_decode_t<0, KV, false>(p, stream) : launch_decode_t<1, KV, false>(p, stream);
 }
 
 hipError_t launch_decode_first(const SplitParams& p, int dtype, hipStream_t stream) {

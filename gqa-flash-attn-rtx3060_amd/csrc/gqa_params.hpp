@@ -120,6 +120,22 @@ struct SplitParams {
   // Stagger the tile order of the splits (set when each head's K and V rows
   // are consecutive: key stride == head_dim).
   int rotate;
+  // One split per (b, kv head) whose rows the first pass writes to o (and
+  // lse) itself: no partials, no combine.
+  int direct;
+  // Flat split (slots > 0; splits is ignored): the keys of all sequences, in
+  // units of one tile step, are laid end to end and cut into `slots` equal
+  // ranges, one per workgroup of a (kv head, row block); a workgroup works
+  // through the pieces of the sequences in its range, one partial each.
+  // Piece (slot j, sequence b) is partial j + b, so a sequence's partials are
+  // consecutive: ws_acc (slots + B, Hq, Sq, D), ws_m and ws_l (slots + B, Hq,
+  // Sq).  Paged: plan receives (first partial, number of partials) per
+  // sequence for the combine.
+  int slots;
+  int* plan;
+  // Set by the launcher: division by the splits (or slots), the row blocks
+  // per workgroup column, Hkv, G and (contiguous) a sequence's units.
+  FastDiv div_splits, div_wblk, div_hkv, div_g, div_units;
 };
 
 // Split-KV combine: one workgroup per (b, q head, query row).
@@ -132,6 +148,12 @@ struct ReduceParams {
   float* lse;  // optional: as FwdParams::lse
   const int* q_start;  // optional: as FwdParams::q_start / q_len
   const int* q_len;
+  // Flat split (splits is ignored): the plan of SplitParams, or over
+  // contiguous K/V (plan nullptr, units > 0) `units` units per sequence in
+  // `slots` <= B * units slots.
+  const int* plan;
+  int slots, units;
+  FastDiv div_sq, div_hq, div_total;  // set by the launcher (div_total: B * units)
 };
 
 // Packed query rows per single-pass workgroup (8 waves x 32 rows).
@@ -189,6 +211,8 @@ hipError_t launch_paged_cache_write(const CacheWriteParams& p, hipStream_t strea
 hipError_t launch_split_reduce(const ReduceParams& p, int dtype, hipStream_t stream);
 // Decode-shaped first pass (gqa_decode.hip): head_dim 128, contiguous K/V,
 // fixed query lengths, 32-bit chunk and workspace offsets.
+// Keys of one of its tile steps, the unit of a flat split.
+constexpr int decode_unit(int head_dim) { return head_dim == 64 ? 128 : 64; }
 bool decode_kernel_fits(const SplitParams& p);
 hipError_t launch_decode_first(const SplitParams& p, int dtype, hipStream_t stream);  // fused if p.counters
 

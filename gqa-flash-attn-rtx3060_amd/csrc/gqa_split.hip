@@ -29,6 +29,7 @@
 // 64-key sub-tile is one strided run inside one page and loads like a
 // contiguous tile after one table lookup; smaller pages (KV = 2) resolve the
 // page of every row, from a copy of the chunk's table slice in LDS.
+#include <algorithm>
 #include <type_traits>
 
 #include "gqa_common.hpp"
@@ -437,18 +438,29 @@ __global__ __launch_bounds__(256) void gqa_split_reduce_kernel(ReduceParams p) {
   // 8192 keys 10.89 -> 10.72 us, a 16-token verify step at 131072 keys
   // 92.25 -> 91.28 us, bit-identical).
   const int row = xcd_remap(blockIdx.x, gridDim.x);
-  const int S = p.splits;
-  const int pos = row % p.Sq;
-  const int bh = row / p.Sq;
-  const int h = bh % p.Hq, b = bh / p.Hq;
+  const int bh = fast_div(row, p.div_sq.mul, p.div_sq.shift), pos = row - bh * p.Sq;
+  const int b = fast_div(bh, p.div_hq.mul, p.div_hq.shift), h = bh - b * p.Hq;
   // Variable query lengths: rows past this sequence's queries hold no
   // partials; o and lse are token-major.
   const bool varlen = p.q_len != nullptr;
   if (varlen && pos >= p.q_len[b]) return;
   const int64_t tok = varlen ? (int64_t)load_uniform(p.q_start + b) + pos : 0;
-  const float* wm = p.ws_m + (int64_t)row * S;
-  const float* wl = p.ws_l + (int64_t)row * S;
-  const float* wa = p.ws_acc + (int64_t)row * S * D;
+  // This row's partials: S of them, `step` workspace rows apart.
+  const bool flat = p.plan != nullptr || p.units > 0;
+  int S = p.splits, first = 0;
+  if (p.plan != nullptr) {
+    first = load_uniform(p.plan + 2 * b);
+    S = load_uniform(p.plan + 2 * b + 1);
+  } else if (flat) {
+    first = fast_div((b * p.units + 1) * p.slots - 1, p.div_total.mul, p.div_total.shift);
+    S = fast_div((b + 1) * p.units * p.slots - 1, p.div_total.mul, p.div_total.shift) - first + 1;
+    first += b;
+  }
+  const int64_t step = flat ? (int64_t)p.Hq * p.Sq : 1;
+  const int64_t row0 = flat ? first * step + (int64_t)h * p.Sq + pos : (int64_t)row * S;
+  const float* wm = p.ws_m + row0;
+  const float* wl = p.ws_l + row0;
+  const float* wa = p.ws_acc + row0 * D;
 
   const int d4 = t % ND4, sg = t / ND4;
   float m_loc = -__builtin_inff(), l_loc = 0.f;
@@ -463,9 +475,9 @@ __global__ __launch_bounds__(256) void gqa_split_reduce_kernel(ReduceParams p) {
       lv[k] = 0.f;
       av[k] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (s < S) {
-        mv[k] = wm[s];
-        lv[k] = wl[s];
-        av[k] = *reinterpret_cast<const f32x4*>(wa + (int64_t)s * D + 4 * d4);
+        mv[k] = wm[s * step];
+        lv[k] = wl[s * step];
+        av[k] = *reinterpret_cast<const f32x4*>(wa + s * step * D + 4 * d4);
       }
     }
     float mb = m_loc;
@@ -510,7 +522,12 @@ __global__ __launch_bounds__(256) void gqa_split_reduce_kernel(ReduceParams p) {
     T* orow = static_cast<T*>(const_cast<void*>(p.o.ptr)) +
               (varlen ? tok * p.o.ss + (int64_t)h * p.o.sh
                       : (int64_t)b * p.o.sb + (int64_t)h * p.o.sh + (int64_t)pos * p.o.ss);
-    // A sequence without keys (finite m*, l* = 0, o = 0): 0 / inf = 0.
+    // A sequence without keys (finite m*, l* = 0, o = 0; flat: no partials):
+    // 0 / inf = 0.
+    if (flat && S == 0) {
+      l = __builtin_inff();
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     if (l == 0.f && mstar > -__builtin_inff()) l = __builtin_inff();
     u32x2 x;
     x[0] = E::pack2(acc[0] / l, acc[1] / l);
@@ -528,9 +545,12 @@ static hipError_t launch_split_first_t(const SplitParams& p, hipStream_t stream)
 }
 
 template <int DT, int D>
-static hipError_t launch_split_reduce_t(const ReduceParams& p, hipStream_t stream) {
+static hipError_t launch_split_reduce_t(ReduceParams p, hipStream_t stream) {
   const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
   if (rows <= 0) return hipSuccess;
+  p.div_sq = make_fast_div((uint32_t)p.Sq);
+  p.div_hq = make_fast_div((uint32_t)p.Hq);
+  p.div_total = make_fast_div((uint32_t)std::max(p.B * p.units, 1));
   if (p.splits <= 256 / (D / 4))  // at most one split per thread
     hipLaunchKernelGGL((gqa_split_reduce_kernel<DT, D, 1>), dim3((unsigned)rows), dim3(256), 0, stream, p);
   else

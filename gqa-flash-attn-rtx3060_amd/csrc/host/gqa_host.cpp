@@ -68,22 +68,55 @@ py::object split_decode(const at::Tensor& q, const at::Tensor& k, const at::Tens
   return py::cast(o);
 }
 
+// gqa_split_flat_launch into a fresh o (and lse): ws of at least
+// gqa_split_flat_workspace_bytes(...) bytes.  None when the call is not one the
+// flat split takes (GQA_E_FLAT).
+py::object split_flat(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& ws,
+                      int64_t slots, bool causal, double scale_log2, int64_t dtype, bool return_lse) {
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) throw std::invalid_argument("split_flat: 4-d q, k, v expected");
+  if (ws.scalar_type() != at::kFloat) throw std::invalid_argument("split_flat: fp32 workspace expected");
+  at::Tensor o = at::empty_like(q);
+  at::Tensor lse;
+  if (return_lse) lse = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+  int64_t qs[4], ks[4], vs[4], os[4];
+  strides_of(q, qs);
+  strides_of(k, ks);
+  strides_of(v, vs);
+  strides_of(o, os);
+  hipStream_t stream = c10::hip::getCurrentHIPStream(q.get_device()).stream();
+  const int rc = gqa_split_flat_launch(
+      q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os,
+      return_lse ? lse.data_ptr<float>() : nullptr, ws.data_ptr<float>(), static_cast<int>(slots),
+      static_cast<int>(q.size(0)), static_cast<int>(q.size(1)), static_cast<int>(k.size(1)),
+      static_cast<int>(q.size(2)), static_cast<int>(k.size(2)), static_cast<int>(q.size(3)),
+      static_cast<float>(scale_log2), causal ? 1 : 0, static_cast<int>(dtype), stream);
+  if (rc == GQA_E_FLAT) return py::none();
+  if (rc != GQA_OK) {
+    py::module_::import("gqa_kernels._lib").attr("check")(rc);
+    throw std::runtime_error(std::string("gqa_split_flat_launch failed: ") + gqa_strerror(rc));
+  }
+  if (return_lse) return py::make_tuple(o, lse);
+  return py::cast(o);
+}
+
 [[noreturn]] void raise_rc(int rc, const char* what) {
   py::module_::import("gqa_kernels._lib").attr("check")(rc);
   throw std::runtime_error(std::string(what) + " failed: " + gqa_strerror(rc));
 }
 
-// The three kernel routes of paged attention (gqa_kernels.paged.paged_attention,
+// The kernel routes of paged attention (gqa_kernels.paged.paged_attention,
 // after its checks and route choice), launched from the tensors:
 //   route 0: gqa_paged_split_first_launch into ws, then the combine into out
 //            (gqa_split_reduce_varlen_launch with variable query lengths,
 //            else gqa_split_reduce_lse_launch or gqa_split_reduce_launch);
 //   route 1: gqa_paged_fwd_launch, or with `splits` > 0 split query blocks
 //            gqa_paged_fwd_split_launch (ws, zeroed counters);
-//   route 2: gqa_paged_fwd_chunks_launch (ws, `splits` key chunks).
+//   route 2: gqa_paged_fwd_chunks_launch (ws, `splits` key chunks);
+//   route 3: gqa_paged_split_flat_launch (ws, `splits` slots).
+// Returns false (nothing launched) when route 3 does not take the call.
 // q and out are (batch, heads, seq_q, head_dim), or token-major
 // (tokens, heads, head_dim) when q_start / q_len are given.
-void paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
+bool paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                    const at::Tensor& block_table, int64_t table_stride, const at::Tensor& seq_lens,
                    const std::optional<at::Tensor>& q_start, const std::optional<at::Tensor>& q_len,
                    int64_t max_seq_len, const at::Tensor& out, const std::optional<at::Tensor>& lse,
@@ -125,23 +158,31 @@ void paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache
                                     lens, qst, qln, bs, ms, out.data_ptr(), os, lse_p, ws_p,
                                     counters->data_ptr<int>(), S, B, H, Hkv, Sq, D, sl2, causal ? 1 : 0, dt, stream);
     if (rc != GQA_OK) raise_rc(rc, "gqa_paged_fwd_split_launch");
-    return;
+    return true;
   }
   if (route == 1) {
     rc = gqa_paged_fwd_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts, lens,
                               qst, qln, bs, ms, out.data_ptr(), os, lse_p, B, H, Hkv, Sq, D, sl2, causal ? 1 : 0,
                               dt, stream);
     if (rc != GQA_OK) raise_rc(rc, "gqa_paged_fwd_launch");
-    return;
+    return true;
   }
   if (route == 2) {
     rc = gqa_paged_fwd_chunks_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts,
                                      lens, qst, qln, bs, ms, out.data_ptr(), os, lse_p, ws_p, S, B, H, Hkv, Sq, D,
                                      sl2, causal ? 1 : 0, dt, stream);
     if (rc != GQA_OK) raise_rc(rc, "gqa_paged_fwd_chunks_launch");
-    return;
+    return true;
   }
-  if (route != 0) throw std::invalid_argument("paged_forward: route must be 0, 1 or 2");
+  if (route == 3) {
+    rc = gqa_paged_split_flat_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts,
+                                     lens, qst, qln, bs, ms, out.data_ptr(), os, lse_p, ws_p, S, B, H, Hkv, Sq, D,
+                                     sl2, causal ? 1 : 0, dt, stream);
+    if (rc == GQA_E_FLAT) return false;
+    if (rc != GQA_OK) raise_rc(rc, "gqa_paged_split_flat_launch");
+    return true;
+  }
+  if (route != 0) throw std::invalid_argument("paged_forward: route must be 0, 1, 2 or 3");
   rc = gqa_paged_split_first_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts,
                                     lens, qst, qln, bs, ms, ws_p, S, B, H, Hkv, Sq, D, sl2, causal ? 1 : 0, dt,
                                     stream);
@@ -153,6 +194,7 @@ void paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache
   else
     rc = gqa_split_reduce_launch(ws_p, S, out.data_ptr(), os, B, H, Sq, D, dt, stream);
   if (rc != GQA_OK) raise_rc(rc, "gqa_split_reduce_launch");
+  return true;
 }
 
 // gqa_paged_cache_write_launch from the tensors (gqa_kernels.paged.write_kv
@@ -181,7 +223,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("split_decode", &split_decode, "split-KV decode: first pass and combine through gqa_split_launch",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("ws"), py::arg("splits"), py::arg("causal"),
         py::arg("scale_log2"), py::arg("dtype"), py::arg("return_lse"));
-  m.def("paged_forward", &paged_forward, "paged attention: one of the three kernel routes from tensors",
+  m.def("split_flat", &split_flat, "flat split-KV forward through gqa_split_flat_launch", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("ws"), py::arg("slots"), py::arg("causal"), py::arg("scale_log2"), py::arg("dtype"),
+        py::arg("return_lse"));
+  m.def("paged_forward", &paged_forward, "paged attention: one of the kernel routes from tensors",
         py::arg("route"), py::arg("q"), py::arg("k_cache"), py::arg("v_cache"), py::arg("block_table"),
         py::arg("table_stride"), py::arg("seq_lens"), py::arg("q_start"), py::arg("q_len"), py::arg("max_seq_len"),
         py::arg("out"), py::arg("lse"), py::arg("ws"), py::arg("counters"), py::arg("splits"), py::arg("batch"),

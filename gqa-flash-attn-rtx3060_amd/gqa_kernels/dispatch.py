@@ -16,7 +16,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .gqa_split import _counter_buffer, _workspace_buffer, decode_forward, stream_handle
+from .gqa_split import _counter_buffer, _workspace_buffer, decode_forward, flat_forward, stream_handle
 
 __all__ = ["gqa_flash_attn", "Route", "choose_route"]
 
@@ -68,6 +68,17 @@ SPLIT_WG_PER_CU = 2
 # 46.5, 4 tokens at 131072 keys 32 45.7 / 64 47.1, B = 16 x 8192 2 45.7 / 4
 # 46.5, 8192 keys 16 11.2 / 32 11.6.
 DEC16_ROWS = 16
+# Flat splits (gqa_split_flat_launch): for batches whose workgroups, at every
+# power-of-two split count that gives each compute unit up to
+# SPLIT_WG_PER_CU, would keep the fullest CU busy while the others idle more
+# than this share of the time.  Measured on MI355X (bf16, one token, G = 4, 8
+# kv heads, us, best fixed count / flat with one slot per CU): B = 5 x 8192
+# keys (0.63 used) 33.9 / 32.1, B = 20 x 3000 (0.63) 47.6 / 43.2, B = 33 x 3000
+# (0.52) 79.9 / 68.4, B = 9 x 3000 at head_dim 64 (0.56) 17.0 / 17.1; B = 3 x
+# 8192 (0.75) 20.9 / 22.1, B = 12 x 6000 (0.75) 51.6 / 50.7, B = 7 x 2000 (0.88)
+# 14.3 / 16.5, powers of two 0.2-1.5 us the other way (a workgroup that
+# crosses into the next sequence drains and refills its pipeline).
+FLAT_MIN_USED = 0.7
 # Single pass with key-range split of the heaviest causal query blocks: only
 # considered while there are fewer than this many workgroups per CU, and
 # taken when the modelled run time drops by at least FWD_SPLIT_GAIN.
@@ -110,7 +121,9 @@ _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 
 @dataclass(frozen=True)
 class Route:
-    kind: str  # "single", "split" or "chunks" (splits: key chunks per query block)
+    # "single", "split", "chunks" (splits: key chunks per query block) or
+    # "flat" (splits: slots of the flat split)
+    kind: str
     splits: int = 1
     workgroups: int = 0
     fwd_split: int = 0  # single pass: query blocks per (b, kv head) run as two key halves
@@ -412,7 +425,46 @@ def choose_route(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_
     return Route("single", 1, single_wgs + ns * num_kv_heads * batch, ns)
 
 
+def flat_max_rows(head_dim: int = 128) -> int:
+    """Packed rows per kv head up to which the flat split is built."""
+    return DEC16_ROWS if head_dim == 64 else SPLIT_ROWS
+
+
+def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int,
+                cu_count: int, causal: bool = True, head_dim: int = 128) -> Route:
+    """What gqa_flash_attn launches: choose_route's route, refined for at most
+    flat_max_rows(head_dim) packed rows per kv head (a token or a few).
+
+    * Caches below SPLIT_MIN_KV keys are split as longer ones are (the single
+      pass would give each kv head one workgroup of 256 rows, of which 4 hold
+      a query): 700 keys, us, single pass / split: B = 1 20.2 / 8.7, B = 16
+      20.8 / 12.7, B = 64 45.6 / 30.5; 300 keys, B = 1 14.1 / 7.4.
+    * With one split per sequence the first pass writes the output itself
+      (the flat split with one slot per sequence): B = 32 x 700 keys 19.5 ->
+      17.6, B = 64 x 700 32.6 -> 30.5.
+    * Batches that no power-of-two split count spreads evenly over the
+      compute units take the flat split (FLAT_MIN_USED)."""
+    route = choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
+    rows = num_heads // num_kv_heads * seq_q
+    if not 0 < rows <= flat_max_rows(head_dim) or seq_kv <= 0 or batch <= 0:
+        return route
+    base = num_kv_heads * batch
+    splits = split_count(base, seq_kv, cu_count, split_rows_per_workgroup(rows, head_dim), head_dim,
+                         rows16=rows <= DEC16_ROWS)
+
+    def used(wgs: int) -> float:
+        return wgs / (cu_count * _cdiv(wgs, cu_count))
+
+    slots = max(1, cu_count // num_kv_heads)
+    if batch > 1 and slots <= _lib.GQA_MAX_SPLITS and used(base * splits) < FLAT_MIN_USED and base * splits > cu_count:
+        return Route("flat", slots, slots * num_kv_heads)
+    if splits == 1 and batch <= _lib.GQA_MAX_SPLITS:
+        return Route("flat", batch, base)
+    return Route("split", splits, base * splits)
+
+
 _route_cached = functools.lru_cache(maxsize=4096)(choose_route)
+_plan_cached = functools.lru_cache(maxsize=4096)(choose_plan)
 
 
 @functools.lru_cache(maxsize=None)
@@ -470,7 +522,7 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
     dev = q.get_device()  # device index (an int: no torch.device objects on this path)
     assert k.get_device() == dev and v.get_device() == dev, "q, k, v must be on one device"
 
-    route = _route_cached(batch, num_heads, num_kv_heads, seq_q, seq_kv, _cu_count(dev), bool(causal), head_dim)
+    route = _plan_cached(batch, num_heads, num_kv_heads, seq_q, seq_kv, _cu_count(dev), bool(causal), head_dim)
     if dev == torch.cuda.current_device():
         return _launch(route, q, k, v, causal, return_lse, dev)
     with torch.cuda.device(dev):  # launch on q's device
@@ -487,6 +539,12 @@ def _launch(route, q_in, k, v, causal, return_lse, dev):
         q = q_in
     else:
         q, k, v = _kernel_ready(q_in), _kernel_ready(k), _kernel_ready(v)
+    if route.kind == "flat":
+        out = flat_forward(q, k, v, causal, route.splits, return_lse, dev)
+        if out is not None:
+            return out
+        batch, num_heads, seq_q, head_dim = q.shape
+        route = _route_cached(batch, num_heads, k.shape[1], seq_q, k.shape[2], _cu_count(dev), bool(causal), head_dim)
     if route.kind == "split":
         return decode_forward(q, k, v, causal, route.splits, return_lse, dev)
     o = torch.empty_like(q_in)  # as dispatch.py:47; contiguous if unusable

@@ -17,7 +17,8 @@ import torch
 
 from . import _lib
 
-__all__ = ["split_kv_forward", "decode_forward", "workspace_bytes", "stream_handle"]
+__all__ = ["split_kv_forward", "decode_forward", "flat_forward", "workspace_bytes", "flat_workspace_bytes",
+           "stream_handle"]
 
 # Zeroed int32 counters for the fused combine, one buffer per (device,
 # stream): the kernel leaves them zero, so a buffer is reused by every call on
@@ -107,6 +108,13 @@ def workspace_bytes(batch: int, num_heads: int, seq_q: int, head_dim: int, split
     return batch * num_heads * seq_q * splits * (head_dim + 2) * 4
 
 
+def flat_workspace_bytes(batch: int, num_heads: int, seq_q: int, head_dim: int, slots: int) -> int:
+    """Workspace of a flat split (gqa_split_flat_workspace_bytes): fp32 acc,
+    m and l of slots + batch partials per query row, then two int32 per
+    sequence."""
+    return (slots + batch) * num_heads * seq_q * (head_dim + 2) * 4 + batch * 8
+
+
 _SCALE_LOG2 = {64: 64 ** -0.5 * LOG2E, 128: 128 ** -0.5 * LOG2E}
 
 
@@ -167,6 +175,33 @@ def decode_forward(q, k, v, causal, splits, return_lse, dev):
         return _split_launch_ctypes(q, k, v, ws, splits, causal, _SCALE_LOG2[head_dim], return_lse, stream)
     return host.split_decode(q, k, v, ws, splits, bool(causal), _SCALE_LOG2[head_dim], _DTYPES[q.dtype],
                              bool(return_lse))
+
+
+def flat_forward(q, k, v, causal, slots, return_lse, dev):
+    """The flat split-KV forward (gqa_split_flat_launch) of kernel-ready q, k,
+    v on the current device `dev`, or None when it does not take the call
+    (GQA_E_FLAT: more packed rows, or strides past its 32-bit offsets)."""
+    batch, num_heads, seq_q, head_dim = q.shape
+    stream = stream_handle(q.device)
+    need = flat_workspace_bytes(batch, num_heads, seq_q, head_dim, slots)
+    ws = _workspaces.get((dev, stream))
+    if ws is None or ws.numel() * 4 < need:
+        ws = _workspace_buffer(q.device, stream, need)
+    host = _lib._host if _lib._host is not None else _decode_host()
+    if host is not None:
+        return host.split_flat(q, k, v, ws, slots, bool(causal), _SCALE_LOG2[head_dim], _DTYPES[q.dtype],
+                               bool(return_lse))
+    o = torch.empty_like(q)
+    lse = torch.empty(batch, num_heads, seq_q, dtype=torch.float32, device=q.device) if return_lse else None
+    rc = _lib.load().gqa_split_flat_launch(
+        q.data_ptr(), _lib.strides(q), k.data_ptr(), _lib.strides(k), v.data_ptr(), _lib.strides(v),
+        o.data_ptr(), _lib.strides(o), None if lse is None else lse.data_ptr(), ws.data_ptr(), slots,
+        batch, num_heads, k.shape[1], seq_q, k.shape[2], head_dim, _SCALE_LOG2[head_dim], int(bool(causal)),
+        _DTYPES[q.dtype], stream)
+    if rc == _lib.GQA_E_FLAT:
+        return None
+    _lib.check(rc)
+    return o if lse is None else (o, lse)
 
 
 def split_kv_forward(q, k, v, causal, splits, workspace=None, fused=False, return_lse=False):

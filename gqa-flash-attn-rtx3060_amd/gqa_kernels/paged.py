@@ -40,15 +40,17 @@ from typing import Dict, Hashable, List, Optional, Sequence
 import torch
 
 from . import _lib
-from .dispatch import (FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks,
+from .dispatch import (FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
                        fwd_split_makespan)
-from .gqa_split import _counter_buffer, _decode_host, _workspace_buffer, stream_handle, workspace_bytes
+from .gqa_split import (_counter_buffer, _decode_host, _workspace_buffer, flat_workspace_bytes, stream_handle,
+                        workspace_bytes)
 
 __all__ = [
     "paged_attention",
     "write_kv",
     "paged_chunk",
     "paged_splits",
+    "paged_flat_slots",
     "paged_kv_chunks",
     "paged_single_plan",
     "PagedKVCache",
@@ -178,7 +180,31 @@ def paged_splits(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_
     return splits
 
 
-_ROUTE_IDS = {"split": 0, "single": 1, "chunks": 2}
+@functools.lru_cache(maxsize=4096)
+def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_seq_len: int, cu_count: int,
+                     block_size: int = 64, head_dim: int = 128) -> int:
+    """Slots of the flat split (gqa_paged_split_flat_launch) for a paged call,
+    0 for the fixed split count of ``paged_splits``.
+
+    Cutting every sequence alike leaves a batch of unequal lengths waiting
+    for its longest sequences; the flat split gives every workgroup the same
+    number of keys, read from the lengths on the device.  One workgroup per
+    compute unit (two or four measured the same or slower).  Measured on
+    MI355X (bf16, one token, G = 4, 8 kv heads, us, fixed -> flat): 16-key
+    token-major pages, B = 32 of 100-8000 keys 111.7 -> 94.2, B = 16 of
+    500-16000 112.0 -> 93.5, B = 64 of 100-4000 114.4 -> 97.8, B = 14 of
+    600-6000 45.2 -> 37.5, 4 tokens B = 8 of 100-8000 37.2 -> 28.9; head-major
+    64-key pages, B = 8 of 1000-30000 114.7 -> 80.9; equal lengths B = 16 x 8192
+    84.4 -> 83.7, B = 4 x 32768 85.1 -> 88.3.  One sequence (10.3 against 12.4
+    at 8192 keys) keeps the fixed count."""
+    rows = num_heads // num_kv_heads * seq_q
+    if batch < 2 or max_seq_len < 1 or block_size < single_pass_min_block(head_dim):
+        return 0
+    slots = cu_count // num_kv_heads
+    return slots if 0 < rows <= flat_max_rows(head_dim) and 1 <= slots <= _lib.GQA_MAX_SPLITS else 0
+
+
+_ROUTE_IDS = {"split": 0, "single": 1, "chunks": 2, "flat": 3}
 
 
 def _paged_host():
@@ -201,6 +227,12 @@ def _rows_ready(t: torch.Tensor) -> bool:
     for x in st[:-1]:
         bits |= x
     return (t.data_ptr() | bits * t.element_size()) % 16 == 0
+
+
+def _row_strides(t: torch.Tensor, varlen: bool):
+    """q / o strides as the kernels address them; token-major: (unused, head,
+    token, d)."""
+    return _lib._i64x4(0, t.stride(1), t.stride(0), 1) if varlen else _lib.strides(t)
 
 
 def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor) -> int:
@@ -297,7 +329,8 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             keys past it are not read).  Default: the table's capacity,
             max_blocks_per_seq * block_size, which needs no device read.
         scale: score scale (default head_dim ** -0.5, the reference's).
-        splits: split count of the split route (default: ``paged_splits``),
+        splits: split count of the split route (default: the flat split of
+            ``paged_flat_slots``, or ``paged_splits``),
             key chunks per query block of the "chunks" route (default:
             ``paged_kv_chunks``, at least 2), or query blocks run as two key
             halves on the "single" route (default: none when "single" is
@@ -360,6 +393,10 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     assert 0 <= max_seq_len <= capacity, "max_seq_len exceeds the block table's capacity"
     dev = qdev.index if qdev.index is not None else torch.cuda.current_device()
     splits_given = splits is not None
+    flat_slots = 0
+    if splits is None and route in (None, "split"):
+        flat_slots = paged_flat_slots(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
+                                      head_dim)
     if splits is None:
         interleaved = k_cache.stride(1) != head_dim or v_cache.stride(1) != head_dim
         splits = paged_splits(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
@@ -393,6 +430,27 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     assert route == "split" or block_size >= single_pass_min_block(head_dim)
     lse = torch.empty(lse_shape, dtype=torch.float32, device=qdev) if return_lse else None
     counters = None
+    host = _paged_host()
+    if route == "split" and flat_slots:
+        workspace = _workspace_buffer(qdev, stream, flat_workspace_bytes(batch, num_heads, seq_q, head_dim, flat_slots))
+        if host is not None:
+            done = host.paged_forward(_ROUTE_IDS["flat"], q, k_cache, v_cache, block_table, table_stride, seq_lens,
+                                      query_start if varlen else None, query_lens if varlen else None, max_seq_len,
+                                      out, lse, workspace, None, flat_slots, batch, seq_q, scale * LOG2E,
+                                      bool(causal), dtype)
+        else:
+            rc = lib.gqa_paged_split_flat_launch(
+                q.data_ptr(), _row_strides(q, varlen), k_cache.data_ptr(), _lib.strides(k_cache),
+                v_cache.data_ptr(), _lib.strides(v_cache), block_table.data_ptr(), table_stride,
+                seq_lens.data_ptr(), query_start.data_ptr() if varlen else None,
+                query_lens.data_ptr() if varlen else None, block_size, max_seq_len, out.data_ptr(),
+                _row_strides(out, varlen), None if lse is None else lse.data_ptr(), workspace.data_ptr(), flat_slots,
+                batch, num_heads, num_kv_heads, seq_q, head_dim, scale * LOG2E, int(bool(causal)), dtype, stream)
+            done = rc != _lib.GQA_E_FLAT
+            if done:
+                _lib.check(rc)
+        if done:
+            return out if lse is None else (out, lse)
     if route == "single":
         # Split query blocks: their halves' fp32 state and the stream's
         # zeroed merge counters (left zero by the kernel).
@@ -404,15 +462,12 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     else:
         n_parts = kv_chunks if route == "chunks" else splits
         workspace = _workspace_buffer(qdev, stream, workspace_bytes(batch, num_heads, seq_q, head_dim, n_parts))
-    host = _paged_host()
     if host is not None:
         host.paged_forward(_ROUTE_IDS[route], q, k_cache, v_cache, block_table, table_stride, seq_lens,
                            query_start if varlen else None, query_lens if varlen else None, max_seq_len, out, lse,
                            workspace, counters, n_parts, batch, seq_q, scale * LOG2E, bool(causal), dtype)
         return out if lse is None else (out, lse)
-    # Token-major q / o as the kernels address them: (unused, head, token, d).
-    qst = _lib._i64x4(0, q.stride(1), q.stride(0), 1) if varlen else _lib.strides(q)
-    ost = _lib._i64x4(0, out.stride(1), out.stride(0), 1) if varlen else _lib.strides(out)
+    qst, ost = _row_strides(q, varlen), _row_strides(out, varlen)
     qs_p = query_start.data_ptr() if varlen else None
     ql_p = query_lens.data_ptr() if varlen else None
     lse_p = None if lse is None else lse.data_ptr()

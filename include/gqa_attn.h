@@ -52,6 +52,8 @@ extern "C" {
                                  512 / head_dim), or table too short */
 #define GQA_E_SCRATCH (-9)    /* gqa_split_noalloc_launch: partials larger than
                                  GQA_NOALLOC_SCRATCH_BYTES */
+#define GQA_E_FLAT (-10)      /* flat split: slots out of [1, GQA_MAX_SPLITS], no keys, or a call
+                                 the LDS-DMA first pass does not take (see gqa_split_flat_launch) */
 
 #define GQA_MAX_SPLITS 1024
 #define GQA_MAX_BLOCK_SIZE 65536
@@ -249,6 +251,41 @@ int gqa_split_launch(const void* q, const int64_t q_stride[4],
                      int batch, int num_heads, int num_kv_heads,
                      int seq_q, int seq_kv, int head_dim,
                      float scale_log2, int causal, int dtype, void* stream);
+
+/* Flat split-KV forward (no counterpart in the reference, whose splits cut
+ * every sequence alike): the keys of all sequences are laid end to end in
+ * tile steps (64 keys, 128 at head_dim 64) and cut into `slots` equal ranges
+ * per kv head, one workgroup each, so batches of unequal lengths or of a
+ * size that does not divide the compute units keep them equally busy.  The
+ * paged form reads the lengths from seq_lens on the device.  First pass, then
+ * combine (slots == batch over contiguous K/V: one range is one sequence, the
+ * first pass writes o and lse itself).  For at most 32 packed rows
+ * (num_heads / num_kv_heads * seq_q) at head_dim 128, 16 at head_dim 64, and
+ * pages of at least 512 / head_dim keys; GQA_E_FLAT otherwise.
+ * workspace: 16-byte aligned, gqa_split_flat_workspace_bytes() bytes. */
+size_t gqa_split_flat_workspace_bytes(int batch, int num_heads, int seq_q,
+                                      int head_dim, int slots);
+int gqa_split_flat_launch(const void* q, const int64_t q_stride[4],
+                          const void* k, const int64_t k_stride[4],
+                          const void* v, const int64_t v_stride[4],
+                          void* o, const int64_t o_stride[4], float* lse,
+                          float* workspace, int slots,
+                          int batch, int num_heads, int num_kv_heads,
+                          int seq_q, int seq_kv, int head_dim,
+                          float scale_log2, int causal, int dtype,
+                          void* stream);
+int gqa_paged_split_flat_launch(const void* q, const int64_t q_stride[4],
+                                const void* k_cache, const int64_t k_cache_stride[4],
+                                const void* v_cache, const int64_t v_cache_stride[4],
+                                const int* block_table, int table_stride,
+                                const int* seq_lens, const int* q_start,
+                                const int* q_len, int block_size,
+                                int max_seq_len, void* o,
+                                const int64_t o_stride[4], float* lse,
+                                float* workspace, int slots, int batch,
+                                int num_heads, int num_kv_heads, int seq_q,
+                                int head_dim, float scale_log2, int causal,
+                                int dtype, void* stream);
 
 /* Split-KV forward that allocates nothing.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory or hand in a

@@ -29,7 +29,9 @@ using gqa::TensorRef;
 // 12: gqa_paged_fwd_chunks_launch (the same over a paged cache).
 // 13: gqa_paged_fwd_split_launch (the paged single pass with split blocks).
 // 14: gqa_split_flat_launch, gqa_paged_split_flat_launch (flat splits).
-constexpr int kAbiVersion = 14;
+// 15: gqa_fwd_short_launch, gqa_paged_fwd_short_launch (the single pass of
+// short calls).
+constexpr int kAbiVersion = 15;
 
 int check_dims(int B, int Hq, int Hkv, int Sq, int Skv, int D, int dtype) {
   if (B < 0 || Hq <= 0 || Hkv <= 0 || Sq < 0 || Skv < 0) return GQA_E_SHAPE;
@@ -122,12 +124,13 @@ namespace {
 int fwd_impl(const void* q, const int64_t q_stride[4], const void* k, const int64_t k_stride[4], const void* v,
              const int64_t v_stride[4], void* o, const int64_t o_stride[4], float* lse, int batch, int num_heads,
              int num_kv_heads, int seq_q, int seq_kv, int head_dim, float scale_log2, int causal, int dtype,
-             void* stream, int n_split = 0, float* part_ws = nullptr, int* part_cnt = nullptr) {
+             void* stream, int n_split = 0, float* part_ws = nullptr, int* part_cnt = nullptr,
+             bool short_form = false) {
   int rc = check_dims(batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, dtype);
   if (rc) return rc;
-  const int G = num_heads / num_kv_heads;
-  if (G > gqa::kFwdRows) return GQA_E_GROUP;
-  const int block_m = gqa::kFwdRows / G;
+  const int G = num_heads / num_kv_heads, rows = short_form ? gqa::kShortRows : gqa::kFwdRows;
+  if (G > rows) return GQA_E_GROUP;
+  const int block_m = rows / G;
   const int n_mblk = (seq_q + block_m - 1) / block_m;
   if (n_split < 0 || n_split > n_mblk) return GQA_E_SPLITS;
   if (batch == 0 || seq_q == 0) return GQA_OK;
@@ -154,7 +157,8 @@ int fwd_impl(const void* q, const int64_t q_stride[4], const void* k, const int6
   p.part_cnt = part_cnt;
   // The scheduling counters follow the split blocks' counters.
   p.sched = part_cnt != nullptr ? part_cnt + (size_t)batch * num_kv_heads * n_split : nullptr;
-  return to_code(gqa::launch_fwd(p, dtype, static_cast<hipStream_t>(stream)));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return to_code(short_form ? gqa::launch_short(p, dtype, st) : gqa::launch_fwd(p, dtype, st));
 }
 
 // Variable query lengths: q_start and q_len both NULL (uniform seq_q) or
@@ -176,7 +180,7 @@ int paged_fwd_impl(const void* q, const int64_t q_stride[4], const void* k_cache
                    const int* q_len, int block_size, int max_seq_len, void* o, const int64_t o_stride[4],
                    float* lse, float* workspace, int kv_splits, int batch, int num_heads, int num_kv_heads,
                    int seq_q, int head_dim, float scale_log2, int causal, int dtype, void* stream,
-                   int n_split = 0, float* part_ws = nullptr, int* part_cnt = nullptr);
+                   int n_split = 0, float* part_ws = nullptr, int* part_cnt = nullptr, bool short_form = false);
 
 }  // namespace
 
@@ -218,6 +222,28 @@ int gqa_fwd_split_launch(const void* q, const int64_t q_stride[4], const void* k
   if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return GQA_E_STRIDE;
   return fwd_impl(q, q_stride, k, k_stride, v, v_stride, o, o_stride, lse, batch, num_heads, num_kv_heads, seq_q,
                   seq_kv, head_dim, scale_log2, causal, dtype, stream, n_split, workspace, counters);
+}
+
+int gqa_fwd_short_launch(const void* q, const int64_t q_stride[4], const void* k, const int64_t k_stride[4],
+                         const void* v, const int64_t v_stride[4], void* o, const int64_t o_stride[4], float* lse,
+                         int batch, int num_heads, int num_kv_heads, int seq_q, int seq_kv, int head_dim,
+                         float scale_log2, int causal, int dtype, void* stream) {
+  if ((reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return GQA_E_STRIDE;
+  return fwd_impl(q, q_stride, k, k_stride, v, v_stride, o, o_stride, lse, batch, num_heads, num_kv_heads, seq_q,
+                  seq_kv, head_dim, scale_log2, causal, dtype, stream, 0, nullptr, nullptr, true);
+}
+
+int gqa_paged_fwd_short_launch(const void* q, const int64_t q_stride[4], const void* k_cache,
+                               const int64_t k_cache_stride[4], const void* v_cache,
+                               const int64_t v_cache_stride[4], const int* block_table, int table_stride,
+                               const int* seq_lens, const int* q_start, const int* q_len, int block_size,
+                               int max_seq_len, void* o, const int64_t o_stride[4], float* lse, int batch,
+                               int num_heads, int num_kv_heads, int seq_q, int head_dim, float scale_log2, int causal,
+                               int dtype, void* stream) {
+  return paged_fwd_impl(q, q_stride, k_cache, k_cache_stride, v_cache, v_cache_stride, block_table, table_stride,
+                        seq_lens, q_start, q_len, block_size, max_seq_len, o, o_stride, lse, nullptr, 0, batch,
+                        num_heads, num_kv_heads, seq_q, head_dim, scale_log2, causal, dtype, stream, 0, nullptr,
+                        nullptr, true);
 }
 
 int gqa_split_first_launch(const void* q, const int64_t q_stride[4], const void* k, const int64_t k_stride[4],
@@ -709,17 +735,17 @@ int paged_fwd_impl(const void* q, const int64_t q_stride[4], const void* k_cache
                    const int* q_len, int block_size, int max_seq_len, void* o, const int64_t o_stride[4],
                    float* lse, float* workspace, int kv_splits, int batch, int num_heads, int num_kv_heads,
                    int seq_q, int head_dim, float scale_log2, int causal, int dtype, void* stream,
-                   int n_split, float* part_ws, int* part_cnt) {
+                   int n_split, float* part_ws, int* part_cnt, bool short_form) {
   int rc = check_dims(batch, num_heads, num_kv_heads, seq_q, max_seq_len, head_dim, dtype);
   if (rc) return rc;
-  const int G = num_heads / num_kv_heads;
-  if (G > gqa::kFwdRows) return GQA_E_GROUP;
+  const int G = num_heads / num_kv_heads, block_rows = short_form ? gqa::kShortRows : gqa::kFwdRows;
+  if (G > block_rows) return GQA_E_GROUP;
   // Each LDS-DMA instruction loads 512 / head_dim rows, which must lie in
   // one block.
   if (block_size < 512 / head_dim || block_size > GQA_MAX_BLOCK_SIZE || (block_size & (block_size - 1)) != 0)
     return GQA_E_BLOCK;
   if (table_stride < 0 || (int64_t)table_stride * block_size < (int64_t)max_seq_len) return GQA_E_BLOCK;
-  const int block_m = gqa::kFwdRows / G;
+  const int block_m = block_rows / G;
   const int n_mblk = (seq_q + block_m - 1) / block_m;
   if (n_split < 0 || n_split > n_mblk || (n_split > 0 && kv_splits > 0)) return GQA_E_SPLITS;
   if (batch == 0 || seq_q == 0) return GQA_OK;
@@ -765,6 +791,7 @@ int paged_fwd_impl(const void* q, const int64_t q_stride[4], const void* k_cache
   p.block_shift = shift;
   p.q_start = q_start;
   p.q_len = q_len;
+  if (short_form) return to_code(gqa::launch_short(p, dtype, static_cast<hipStream_t>(stream)));
   if (kv_splits == 0) return to_code(gqa::launch_paged_fwd(p, dtype, static_cast<hipStream_t>(stream)));
   // Key chunks: chunk c of every query block covers key tiles [c * ct,
   // (c + 1) * ct) of the longest sequence's range; the partials go to the

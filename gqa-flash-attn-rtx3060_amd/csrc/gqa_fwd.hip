@@ -37,106 +37,13 @@
 #include <type_traits>
 
 #include "gqa_common.hpp"
+#include "gqa_fwd_parts.hpp"
 #include "gqa_lds.hpp"
 #include "gqa_params.hpp"
 
 namespace gqa {
 
-// ---------------------------------------------------------------------------
-// Online softmax of one 64-key S^T tile held as two 32-key blocks (16 values
-// per lane and block; the two lane halves hold the other 16 keys of the
-// same row), exp2 domain.
-//
-// Lazy rescaling: the reference point m_ref of a row is kept as long as the
-// probabilities computed against it stay at most 2^kRescaleLog2, which
-// bf16/fp16 P and fp32 l/acc hold as exactly as probabilities <= 1.  A tile's
-// exponentials are first computed against the current m_ref, with no row
-// max; a lane's partial row sum bounds each of its probabilities, so only
-// when some lane's sum exceeds 2^kRescaleLog2 (or is NaN / inf), or some row
-// has no reference yet, does the wave take the tile's exact row max, raise
-// m_ref to it, rescale l and the accumulators, and recompute the tile's
-// exponentials.  The decision is wave-uniform, so in steady state neither a
-// max tree nor the O accumulators cost VALU work.  The result o = acc / l is
-// unchanged (both are relative to the same m_ref).  A row whose m_ref is
-// still -inf after the exact pass (every key masked so far) uses 0 as the
-// reference, so a fully masked tile contributes p = 0, never NaN.
-// ---------------------------------------------------------------------------
-constexpr float kRescaleSum = 256.0f;  // 2^8
-
-// Exact pass: the tile's row max (a max3 tree), m_ref raised to it, l and the
-// accumulators rescaled.  Returns -m_ref * c, the offset of the exponent.
-template <int NACC>
-__device__ inline float softmax_rebase(const f32x16 (&s)[2], float& m_ref, float& l_run, f32x16 (&acc)[NACC],
-                                       float c) {
-  float m1[11];
-#pragma unroll
-  for (int k = 0; k < 10; ++k) {
-    const int i0 = 3 * k, i1 = 3 * k + 1, i2 = 3 * k + 2;
-    m1[k] = vmax3(s[i0 >> 4][i0 & 15], s[i1 >> 4][i1 & 15], s[i2 >> 4][i2 & 15]);
-  }
-  m1[10] = vmax3(s[1][14], s[1][15], s[1][15]);
-  const float n0 = vmax3(m1[0], m1[1], m1[2]), n1 = vmax3(m1[3], m1[4], m1[5]);
-  const float n2 = vmax3(m1[6], m1[7], m1[8]), n3 = vmax3(m1[9], m1[10], m1[10]);
-  const float mx = xhalf_max(vmax3(vmax3(n0, n1, n2), n3, n3));
-  const float m_new = fmaxf(m_ref, mx);
-  const float m_new_use = (m_new == -__builtin_inff()) ? 0.f : m_new;
-  const float alpha = fast_exp2((m_ref - m_new_use) * c);
-  l_run *= alpha;
-#pragma unroll
-  for (int db = 0; db < NACC; ++db)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[db][v] *= alpha;
-  m_ref = m_new;
-  return -m_new_use * c;
-}
-
-// One 32-key block: p = 2^(s*c - m_ref*c) in fp32, rounded to the input type
-// and packed as the P^T operand; returns the fp32 row sum (a tree).
-template <int DT>
-__device__ inline float softmax_exp(const f32x16& s, float nmc, float c, u32x4 (&pk)[2]) {
-  using E = Elem<DT>;
-  float pv[16];
-#pragma unroll
-  for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(__builtin_fmaf(s[v], c, nmc));
-  float s8[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) s8[j] = pv[2 * j] + pv[2 * j + 1];
-#pragma unroll
-  for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) pk[kk][e] = E::pack2(pv[8 * kk + 2 * e], pv[8 * kk + 2 * e + 1]);
-  return ((s8[0] + s8[1]) + (s8[2] + s8[3])) + ((s8[4] + s8[5]) + (s8[6] + s8[7]));
-}
-
-// ---------------------------------------------------------------------------
-// Instruction schedule of an MFMA phase: slot j is one MFMA; the LDS reads of
-// slot j + P are issued right after MFMA j (P slots ahead, to cover the LDS
-// latency).  Slots [0, NRD2) are P*V MFMAs with two transposing reads each,
-// the rest S^T MFMAs with one 16-byte read each.
-// ---------------------------------------------------------------------------
-template <int NRD2, int NSLOT, int P, int J>
-__device__ __forceinline__ void mphase_prefetch() {
-  if constexpr (J < P && J < NSLOT) {
-    __builtin_amdgcn_sched_group_barrier(0x100, (J < NRD2) ? 2 : 1, 0);  // LDS reads
-    mphase_prefetch<NRD2, NSLOT, P, J + 1>();
-  }
-}
-template <int NRD2, int NSLOT, int P, int J>
-__device__ __forceinline__ void mphase_pipe() {
-  if constexpr (J < NSLOT) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-    if constexpr (J + P < NSLOT) __builtin_amdgcn_sched_group_barrier(0x100, (J + P < NRD2) ? 2 : 1, 0);
-    mphase_pipe<NRD2, NSLOT, P, J + 1>();
-  }
-}
-
-// PG: 0 contiguous K/V; 1 a paged cache through the block table with pages
-// of >= 64 keys (one buffer descriptor per 64-key tile, ending at the
-// sequence's last key); 2 pages of RPI..8 keys (RPI = 512 / D rows per
-// LDS-DMA instruction: each instruction's rows lie in one page, and every
-// instruction gets its own descriptor); 3 pages of 16 or 32 keys (each wave
-// loads 16 consecutive rows of a tile, which lie in one page: one table
-// read and one descriptor per wave and tile).
+// PG: the form of K and V (gqa_fwd_parts.hpp).
 // D = 64 keeps to 128 VGPRs (four waves per SIMD): two workgroups share a
 // compute unit, which outweighs the shorter LDS-read lookahead it needs.
 //
@@ -157,12 +64,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   using ST = FwdStage<D>;
   constexpr int CPR = ST::CPR;
   constexpr bool PAGED = PG != 0;
-  constexpr bool SMALL = PG == 2;
-  constexpr bool MEDIUM = PG == 3;
   constexpr bool PERSIST = PG == 0 && D == 128;
-  // Block ids a wave needs per tile: one, or (small pages) one per LDS-DMA
-  // instruction it issues.
-  struct TileBlocks { int id[SMALL ? ST::NI : 1]; };
+  using TileBlocks = FwdTileBlocks<D, PG>;
   constexpr int NDB = D / 32;  // 32-wide d blocks of O^T
   constexpr int NKS = D / 16;  // k-steps of S^T
   constexpr int PF = (D == 64) ? 3 : 6;  // MFMA slots of LDS-read lookahead
@@ -245,7 +148,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     int b, kvh, bh, pid_m, part;  // part: -1 whole key range, 0 lower half, 1 upper half
     int skv, sq, tb, ntiles, qpos_lo;
     int64_t tok0;
-    int pos, head, qpos;  // this lane's query row
+    int pos, head, vis;  // this lane's query row; the keys it sees, as mask_tile counts them
     bool valid;
     const char* kbh;
     const char* vbh;
@@ -283,7 +186,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     x.pos = x.pid_m * block_m + ml;
     x.valid = (g < dm.G) && (x.pos < x.sq);
     x.head = x.kvh * dm.G + (g < dm.G ? g : 0);
-    x.qpos = x.pos + (x.skv - x.sq);
+    x.vis = (dm.causal ? min(x.skv, x.pos + (x.skv - x.sq) + 1) : x.skv) - 8 * hh;
     // Key range of this item: tiles [tb, tb + ntiles).
     const int pos_lo = x.pid_m * block_m;
     const int pos_hi = min(pos_lo + block_m, x.sq) - 1;
@@ -329,118 +232,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
       (uint32_t)(lrow * kssb) + 16u * (uint32_t)((lane % CPR) ^ ST::gk((gw * ST::RPI + lrow) & 15));
   const uint32_t voff = (uint32_t)(lrow * vssb) + 16u * (uint32_t)((lane % CPR) ^ ST::sv(lrow));
 
-  // Issue this wave's share of K or V tile `tile` (absolute index) into LDS.
-  // Paged, blocks of >= 64 keys: the tile's 64 rows are one run inside one
-  // block; its descriptor starts at the tile's first row and ends at the
-  // sequence's last key, so rows past the sequence (and whole tiles past it,
-  // which read no table entry) load as zeros.  Smaller blocks: the same per
-  // LDS-DMA instruction (RPI rows, one run inside one block).
-  // Paged: the block(s) holding a tile, or this wave's instructions of it
-  // (read only for rows that start inside the sequence).  The softmax phases
-  // use block ids read one phase ahead (blk_next), so the table reads'
-  // latency is off the issue path.
-  auto tile_block = [&](const Item& x, int tile) -> TileBlocks {
-    TileBlocks tbk;
-    const int key0 = tile * ST::kKeys;
-    if constexpr (SMALL) {
-#pragma unroll
-      for (int j = 0; j < ST::NI; ++j) {
-        const int key = key0 + (j * 4 + gw) * ST::RPI;  // first row of instruction j
-        tbk.id[j] = key < x.skv ? load_uniform(x.table_row + (key >> p.block_shift)) : 0;
-      }
-    } else if constexpr (MEDIUM) {
-      const int key = key0 + 16 * gw;  // first of this wave's 16 rows
-      tbk.id[0] = key < x.skv ? load_uniform(x.table_row + (key >> p.block_shift)) : 0;
-    } else {
-      tbk.id[0] = (PAGED && key0 < x.skv) ? load_uniform(x.table_row + (key0 >> p.block_shift)) : 0;
-    }
-    return tbk;
+  // Issue this wave's share of K or V tile `tile` (absolute index) into LDS
+  // (gqa_fwd_parts.hpp).  The softmax phases use block ids read one phase
+  // ahead (blk_next), so the table reads' latency is off the issue path.
+  auto tile_block = [&](const Item& x, int tile) __attribute__((always_inline)) -> TileBlocks {
+    return tile_blocks<D, PG>(x.table_row, p.block_shift, x.skv, tile, gw);
   };
   auto issue_tile = [&](const Item& x, char* lds, const char* head, __amdgpu_buffer_rsrc_t rsrc, uint32_t rowb,
-                        uint32_t off, int64_t blk_stride, int tile, const TileBlocks& blk, bool is_k) {
-    const int key0 = tile * ST::kKeys;
-    if constexpr (MEDIUM) {
-      // This wave's rows [key, key + 16) of the tile, one run in one page:
-      // instruction j loads rows key + j * RPI + 0..RPI-1 (scalar offset) into
-      // LDS rows 16 gw + j * RPI + ...  Both swizzles are linear in the row
-      // bits: V's depends on the lane's row lrow alone (off as given); K's
-      // chunk is (lane % CPR) ^ gk(lrow) ^ gk(j * RPI).
-      (void)rsrc;
-      typedef __attribute__((address_space(3))) void lds_void;
-      const int key = key0 + 16 * gw;
-      const int rows = x.skv - key;
-      __amdgpu_buffer_rsrc_t rt = make_rsrc(head, 0u);
-      if (rows > 0) {
-        const char* base = head + 2 * ((int64_t)blk.id[0] * blk_stride +
-                                       (int64_t)(key & ((1 << p.block_shift) - 1)) * (rowb >> 1));
-        rt = make_rsrc(base, (uint32_t)(min(rows, 16) - 1) * rowb + 2 * D);
-      }
-      if constexpr (D == 64) {
-        // Derived from `off` (the lane's offset for LDS rows gw * RPI + lr),
-        // so no offsets of their own stay live across the loop: sv depends
-        // on lr alone, so V's is `off` for both instructions; gk(gw * RPI +
-        // lr) = gk(lr) ^ gk(8 (gw & 1)) with gk(8) = 2, so K's is `off` for
-        // instruction j = gw & 1 and `off` with chunk bit 1 flipped (byte
-        // offset ^ 32, as lr * rowb is a multiple of 64: the host takes
-        // this path only for such row strides) for the other.
-        // The empty asm keeps the XOR here: hoisted out of the tile loop, its
-        // result would hold a register across the loop.
-        (void)lane;
-        uint32_t flip = off;
-        if (is_k) {
-          asm volatile("" : "+v"(flip));
-          flip ^= 32u;
-        }
-        const uint32_t other = flip;
-#pragma unroll
-        for (int j = 0; j < ST::NI; ++j) {
-          const uint32_t o = (j == (gw & 1)) ? off : other;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_void*)(lds + (gw * ST::NI + j) * 1024), 16, o,
-                                                   (uint32_t)(j * ST::RPI) * rowb, 0, 0);
-        }
-      } else {
-        (void)off;
-        const int lr = lane / CPR, lc = lane % CPR;
-#pragma unroll
-        for (int j = 0; j < ST::NI; ++j) {
-          const int sw = is_k ? (ST::gk(lr) ^ ST::gk(j * ST::RPI)) : ST::sv(lr);
-          const uint32_t o = (uint32_t)(lr * rowb) + 16u * (uint32_t)(lc ^ sw);
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_void*)(lds + (gw * ST::NI + j) * 1024), 16, o,
-                                                   (uint32_t)(j * ST::RPI) * rowb, 0, 0);
-        }
-      }
-    } else if constexpr (SMALL) {
-      // Instruction j loads rows [key, key + RPI) of the tile, one run in
-      // one page (key is a multiple of RPI and pages hold >= RPI keys); its
-      // descriptor ends at the sequence's last key.
-      typedef __attribute__((address_space(3))) void lds_void;
-#pragma unroll
-      for (int j = 0; j < ST::NI; ++j) {
-        const int step = j * 4 + gw;
-        const int key = key0 + step * ST::RPI;
-        const int rows = x.skv - key;
-        __amdgpu_buffer_rsrc_t rt = make_rsrc(head, 0u);
-        if (rows > 0) {
-          const char* base = head + 2 * ((int64_t)blk.id[j] * blk_stride +
-                                         (int64_t)(key & ((1 << p.block_shift) - 1)) * (rowb >> 1));
-          rt = make_rsrc(base, (uint32_t)(min(rows, ST::RPI) - 1) * rowb + 2 * D);
-        }
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (lds_void*)(lds + step * 1024), 16, off, 0, 0, 0);
-      }
-    } else if constexpr (PAGED) {
-      const int rows = x.skv - key0;
-      __amdgpu_buffer_rsrc_t rt = make_rsrc(head, 0u);
-      if (rows > 0) {
-        const char* base =
-            head + 2 * ((int64_t)blk.id[0] * blk_stride + (int64_t)(key0 & ((1 << p.block_shift) - 1)) * (rowb >> 1));
-        rt = make_rsrc(base, (uint32_t)(min(rows, ST::kKeys) - 1) * rowb + 2 * D);
-      }
-      issue_tile_dma<D>(lds, rt, 0u, rowb, off, gw);
-    } else {
-      (void)blk;
-      (void)head;
-      issue_tile_dma<D>(lds, rsrc, (uint32_t)key0 * rowb, rowb, off, gw);
-    }
+                        uint32_t off, int64_t blk_stride, int tile, const TileBlocks& blk, bool is_k)
+                        __attribute__((always_inline)) {
+    issue_fwd_tile<D, PG>(lds, head, rsrc, rowb, off, blk_stride, p.block_shift, x.skv, tile, blk, is_k, gw, lane);
   };
   auto issue_k = [&](const Item& x, char* lds, int tile, const TileBlocks& blk) {
     issue_tile(x, lds, x.kbh, x.rk, kssb, koff, p.k.sb, tile, blk, true);
@@ -510,7 +311,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   // landed, so that they are all in flight together (a select beside each load
   // made the compiler wait for every one of the eight in turn: 1.9-2.4 us per
   // launch).  Paged: returns the block(s) of the tile the first softmax phase
-  // issues.
+  // issues.  (Q in whole rows through LDS, as gqa_short.hip loads it, left
+  // 2048 tokens at 42.2 us and 16384 0.6 % slower here.)
   auto prologue_q = [&](const Item& x) __attribute__((always_inline)) {
     const T* qrow = static_cast<const T*>(p.q.ptr) + row_off(x, p.q, x.valid ? x.pos : 0, x.head);
 #pragma unroll
@@ -603,8 +405,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   // issues this wave's share of the loads two tiles ahead (group A: K(tt+2)
   // into stage tt+2; group B: V(tt+2) into stage tt+3), last waits for the
   // loads it issued one softmax phase earlier.
-  auto vphase = [&](auto s3, int tt) {
+  auto vphase = [&](auto s3, int tt, auto first_c) {
     constexpr int S3 = decltype(s3)::value;
+    constexpr bool FIRST = decltype(first_c)::value;  // the item's first tile: nothing to keep or rescale
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
     __builtin_amdgcn_sched_barrier(0);
@@ -617,21 +420,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     blk_next = tile_block(it, ta + 3);
     const int key0 = ta * ST::kKeys;
     const bool need_mask = (key0 + ST::kKeys > it.skv) || (dm.causal && key0 + ST::kKeys - 1 > it.qpos_lo);
-    if (need_mask) {
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int key = key0 + 32 * mb + key_of(v, hh);
-          const bool off = key >= it.skv || (dm.causal && key > it.qpos);
-          sc[mb][v] = off ? -__builtin_inff() : sc[mb][v];
-        }
-    }
+    if (need_mask) mask_tile(sc, it.vis - key0);
     // Exponentials against the current reference; the exact pass when a
     // row has none yet or a lane's partial sum leaves the bound (not
     // `> kRescaleSum`: NaN and inf sums take the exact pass too).
     float rs0 = 0.f, rs1 = 0.f;
-    bool keep = __builtin_amdgcn_ballot_w64(m_run == -__builtin_inff()) == 0;
+    bool keep = false;
+    if constexpr (!FIRST) keep = __builtin_amdgcn_ballot_w64(m_run == -__builtin_inff()) == 0;
     if (keep) {
       const float nmc = -m_run * c;
       rs0 = softmax_exp<DT>(sc[0], nmc, c, pk[0]);
@@ -639,7 +434,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
       keep = __builtin_amdgcn_ballot_w64(!(rs0 + rs1 <= kRescaleSum)) == 0;
     }
     if (!keep) {
-      const float nmc = softmax_rebase<NDB>(sc, m_run, l_run, acc, c);
+      float nmc;
+      if constexpr (FIRST) {
+        f32x16 none[1] = {f32x16{}};
+        nmc = softmax_rebase<1>(sc, m_run, l_run, none, c);
+      } else {
+        nmc = softmax_rebase<NDB>(sc, m_run, l_run, acc, c);
+      }
       rs0 = softmax_exp<DT>(sc[0], nmc, c, pk[0]);
       rs1 = softmax_exp<DT>(sc[1], nmc, c, pk[1]);
     }
@@ -676,23 +477,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
     const int ntiles = it.ntiles;
     if (ntiles > 0) {
       mphase(I0{}, BF{}, BT{});
-      vphase(I0{}, 0);
+      vphase(I0{}, 0, BT{});
       int tt = 1;
       for (; tt + 3 <= ntiles; tt += 3) {
         mphase(I1{}, BT{}, BT{});
-        vphase(I1{}, tt);
+        vphase(I1{}, tt, BF{});
         mphase(I2{}, BT{}, BT{});
-        vphase(I2{}, tt + 1);
+        vphase(I2{}, tt + 1, BF{});
         mphase(I0{}, BT{}, BT{});
-        vphase(I0{}, tt + 2);
+        vphase(I0{}, tt + 2, BF{});
       }
       if (tt < ntiles) {
         mphase(I1{}, BT{}, BT{});
-        vphase(I1{}, tt);
+        vphase(I1{}, tt, BF{});
         ++tt;
         if (tt < ntiles) {
           mphase(I2{}, BT{}, BT{});
-          vphase(I2{}, tt);
+          vphase(I2{}, tt, BF{});
           ++tt;
         }
       }

@@ -159,6 +159,8 @@ struct ReduceParams {
 // Packed query rows per single-pass workgroup (8 waves x 32 rows).
 constexpr int kFwdRows = 256;
 constexpr int kFwdThreads = 512;
+// ... and per workgroup of the short-call form (4 x 32 rows, two key groups).
+constexpr int kShortRows = 128;
 // One partial state of a split query block: per lane of the 8 waves, D/2
 // accumulators, the reference max and the lane's partial row sum.
 constexpr int kFwdPartFloats(int D) { return kFwdThreads * (D / 2 + 2); }
@@ -205,6 +207,9 @@ inline int device_cu_count() {
 
 hipError_t launch_fwd(const FwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_paged_fwd(const FwdParams& p, int dtype, hipStream_t stream);
+// Single pass of short calls (gqa_short.hip): contiguous, or paged when
+// p.block_table is set; no split blocks, no key chunks.
+hipError_t launch_short(const FwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_split_first(const SplitParams& p, int dtype, hipStream_t stream);  // fused if p.counters
 hipError_t launch_paged_split_first(const SplitParams& p, int dtype, hipStream_t stream);
 hipError_t launch_paged_cache_write(const CacheWriteParams& p, hipStream_t stream);

@@ -112,7 +112,8 @@ py::object split_flat(const at::Tensor& q, const at::Tensor& k, const at::Tensor
 //   route 1: gqa_paged_fwd_launch, or with `splits` > 0 split query blocks
 //            gqa_paged_fwd_split_launch (ws, zeroed counters);
 //   route 2: gqa_paged_fwd_chunks_launch (ws, `splits` key chunks);
-//   route 3: gqa_paged_split_flat_launch (ws, `splits` slots).
+//   route 3: gqa_paged_split_flat_launch (ws, `splits` slots);
+//   route 4: gqa_paged_fwd_short_launch.
 // Returns false (nothing launched) when route 3 does not take the call.
 // q and out are (batch, heads, seq_q, head_dim), or token-major
 // (tokens, heads, head_dim) when q_start / q_len are given.
@@ -127,7 +128,7 @@ bool paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache
   const bool varlen = q_start.has_value() && q_len.has_value();
   if (varlen ? q.dim() != 3 || out.dim() != 3 : q.dim() != 4 || out.dim() != 4)
     throw std::invalid_argument("paged_forward: q / out rank does not match the query layout");
-  if ((route != 1 || splits > 0) && !ws.has_value()) throw std::invalid_argument("paged_forward: workspace expected");
+  if (route != 4 && (route != 1 || splits > 0) && !ws.has_value()) throw std::invalid_argument("paged_forward: workspace expected");
   if (route == 1 && splits > 0 && !counters.has_value())
     throw std::invalid_argument("paged_forward: counters expected");
   const int H = static_cast<int>(q.size(1)), D = static_cast<int>(q.size(-1));
@@ -182,7 +183,14 @@ bool paged_forward(int64_t route, const at::Tensor& q, const at::Tensor& k_cache
     if (rc != GQA_OK) raise_rc(rc, "gqa_paged_split_flat_launch");
     return true;
   }
-  if (route != 0) throw std::invalid_argument("paged_forward: route must be 0, 1, 2 or 3");
+  if (route == 4) {
+    rc = gqa_paged_fwd_short_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts, lens,
+                                    qst, qln, bs, ms, out.data_ptr(), os, lse_p, B, H, Hkv, Sq, D, sl2,
+                                    causal ? 1 : 0, dt, stream);
+    if (rc != GQA_OK) raise_rc(rc, "gqa_paged_fwd_short_launch");
+    return true;
+  }
+  if (route != 0) throw std::invalid_argument("paged_forward: route must be 0 to 4");
   rc = gqa_paged_split_first_launch(q.data_ptr(), qs, k_cache.data_ptr(), ks, v_cache.data_ptr(), vs, table, ts,
                                     lens, qst, qln, bs, ms, ws_p, S, B, H, Hkv, Sq, D, sl2, causal ? 1 : 0, dt,
                                     stream);

@@ -22,7 +22,7 @@ GQA_PAGED_CHUNK_PAGES = 2048
 GQA_NOALLOC_SCRATCH_BYTES = 16 << 20
 GQA_E_SCRATCH = -9
 GQA_E_FLAT = -10
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _i64x4 = ctypes.c_int64 * 4
 _i64x3 = ctypes.c_int64 * 3
@@ -102,6 +102,15 @@ SIGNATURES = {
         _i,
         [_p, _i64x4, _p, _i64x4, _p, _i64x4, _p, _i64x4, _p, _p, _i,
          _i, _i, _i, _i, _i, _i, _f, _i, _i, _p],
+    ),
+    "gqa_fwd_short_launch": (
+        _i,
+        [_p, _i64x4, _p, _i64x4, _p, _i64x4, _p, _i64x4, _p, _i, _i, _i, _i, _i, _i, _f, _i, _i, _p],
+    ),
+    "gqa_paged_fwd_short_launch": (
+        _i,
+        [_p, _i64x4, _p, _i64x4, _p, _i64x4, _p, _i, _p, _p, _p, _i, _i, _p, _i64x4, _p,
+         _i, _i, _i, _i, _i, _f, _i, _i, _p],
     ),
     "gqa_split_flat_workspace_bytes": (ctypes.c_size_t, [_i, _i, _i, _i, _i]),
     "gqa_split_flat_launch": (

@@ -16,7 +16,8 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .gqa_split import _counter_buffer, _workspace_buffer, decode_forward, flat_forward, stream_handle
+from .gqa_split import (_counter_buffer, _workspace_buffer, decode_forward, flat_forward, stream_handle,
+                        workspace_bytes)
 
 __all__ = ["gqa_flash_attn", "Route", "choose_route"]
 
@@ -79,6 +80,33 @@ DEC16_ROWS = 16
 # 14.3 / 16.5, powers of two 0.2-1.5 us the other way (a workgroup that
 # crosses into the next sequence drains and refills its pipeline).
 FLAT_MIN_USED = 0.7
+# The short form of the single pass (gqa_fwd_short_launch: workgroups of
+# SHORT_ROWS packed rows, two key tiles a step), considered for at most
+# SHORT_MAX_WG_PER_CU workgroups per CU.  Its run time in us, fitted within
+# 10 % to 34 shapes at head_dim 128 and 34 at 64 (64-4096 tokens, new tokens
+# over caches up to 8192 keys, B = 1-8, causal and not): SHORT_BASE_US + the
+# longest CU's sum of SHORT_ITEM_US + steps x the step time (_step_us).  The
+# other routes' models count 64-key tile steps; OTHER_STEP_US is what those
+# come to on these shapes.  Measured, us, other route
+# -> short form: 333 tokens 17.0 -> 9.8, 1024 23.4 -> 17.4, 2048 42.1 -> 40.0
+# (29.9 -> 25.8 at head_dim 64), 4 x 300 18.1 -> 15.9, 512 bidirectional
+# 17.7 -> 11.2, 512 over 4096 keys 49.9 -> 44.7; 3000 tokens (three
+# workgroups per CU) 77.4 / 80.4, 2048 bidirectional 62.2 / 66.1, 2 x 512 over 8192 keys
+# 118.9 / 118.9, over 16384 224.9 / 232.0.
+SHORT_ROWS = 128
+SHORT_MAX_WG_PER_CU = 2
+SHORT_BASE_US = 2.5
+SHORT_ITEM_US = {128: 3.5, 64: 2.6}
+SHORT_STEP_US = {128: (1.2, 1.8), 64: (0.86, 1.08)}
+OTHER_STEP_US = {"single": {128: (1.25, 1.65), 64: (1.0, 1.0)}, "chunks": {128: 1.3, 64: 1.1}}
+# Against the split-KV pass (33-128 packed rows, 17-64 at head_dim 64): the
+# longest cache, in keys, that the short form streams faster is this times
+# the root of its workgroups.  Measured, us, short / best split count, G = 4,
+# 8 kv heads: 16 tokens, B = 1 300 keys 9.8 / 10.4, 600 11.9 / 10.7; B = 4 600
+# 12.5 / 13.1, 1000 16.5 / 13.9; B = 16 1500 23.9 / 29.6, 3000 43.0 / 45.9;
+# head_dim 64, 8 tokens, B = 1 600 9.1 / 10.2, 1000 12.1 / 10.3; B = 4 1000
+# 12.1 / 12.5; B = 16 3000 28.1 / 30.6.
+SHORT_SPLIT_KEYS = {128: 160.0, 64: 220.0}
 # Single pass with key-range split of the heaviest causal query blocks: only
 # considered while there are fewer than this many workgroups per CU, and
 # taken when the modelled run time drops by at least FWD_SPLIT_GAIN.
@@ -121,12 +149,16 @@ _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 
 @dataclass(frozen=True)
 class Route:
-    # "single", "split", "chunks" (splits: key chunks per query block) or
-    # "flat" (splits: slots of the flat split)
+    # "single", "split", "chunks" (splits: key chunks per query block),
+    # "flat" (splits: slots of the flat split) or "short"
     kind: str
     splits: int = 1
     workgroups: int = 0
     fwd_split: int = 0  # single pass: query blocks per (b, kv head) run as two key halves
+    # short: bytes of stream workspace choose_route's route takes.  The short
+    # form uses none, but a call whose rows lie too far apart for it falls
+    # back to that route, so the stream's buffer is as large either way.
+    reserve: int = 0
 
 
 def _cdiv(a: int, b: int) -> int:
@@ -425,15 +457,73 @@ def choose_route(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_
     return Route("single", 1, single_wgs + ns * num_kv_heads * batch, ns)
 
 
+def _fwd_split_bytes(batch: int, num_kv_heads: int, head_dim: int, n_split: int) -> int:
+    """gqa_fwd_split_workspace_bytes: two fp32 states of 512 lanes x (D / 2 + 2) per split block."""
+    return batch * num_kv_heads * n_split * 2 * 512 * (head_dim // 2 + 2) * 4
+
+
 def flat_max_rows(head_dim: int = 128) -> int:
     """Packed rows per kv head up to which the flat split is built."""
     return DEC16_ROWS if head_dim == 64 else SPLIT_ROWS
 
 
+def _step_us(lo: float, hi: float, work: int, longest: int, cu_count: int) -> float:
+    """A step's time between `lo`, while the longest item runs with less than
+    half the CUs busy on average, and `hi` with all of them."""
+    return lo + (hi - lo) * min(1.0, max(0.0, 2.0 * work / (max(1, longest) * cu_count) - 1.0))
+
+
+def short_us(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int, cu_count: int,
+             causal: bool, head_dim: int = 128) -> float:
+    """Modelled run time (us) of the short form (constants above): blocks
+    heavy-first under causal, each CU taking the next when free."""
+    block_m = SHORT_ROWS // (num_heads // num_kv_heads)
+    n_mblk, n_bh = _cdiv(seq_q, block_m), batch * num_kv_heads
+    tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
+    step = _step_us(*SHORT_STEP_US[head_dim], sum(tiles) * n_bh, max(tiles), cu_count)
+    runs = []
+    for t in (reversed(tiles) if causal else tiles):
+        _push_run(runs, SHORT_ITEM_US[head_dim] + step * _cdiv(t, 2), 1)
+    return SHORT_BASE_US + _list_makespan(runs, n_bh, cu_count)
+
+
+def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int, cu_count: int,
+              causal: bool, head_dim: int, kv_chunks: int, fwd_split: int, persistent: bool) -> bool:
+    """Whether the short form beats the route it would replace: the split-KV
+    pass for at most split_max_rows(head_dim) packed rows per kv head, else
+    the single pass with `fwd_split` split blocks, or over `kv_chunks` key
+    chunks (`persistent` as chunks_makespan)."""
+    group = num_heads // num_kv_heads
+    if group > SHORT_ROWS or seq_q <= 0 or batch <= 0:
+        return False
+    wgs = _cdiv(seq_q, SHORT_ROWS // group) * num_kv_heads * batch
+    if wgs > SHORT_MAX_WG_PER_CU * cu_count:
+        return False
+    if group * seq_q <= split_max_rows(head_dim):
+        return seq_kv <= SHORT_SPLIT_KEYS[head_dim] * math.sqrt(wgs)
+    block_m = max(1, FWD_ROWS // group)
+    n_mblk, n_bh = _cdiv(seq_q, block_m), batch * num_kv_heads
+    tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
+    if kv_chunks:
+        other = OTHER_STEP_US["chunks"][head_dim] * chunks_makespan(
+            tiles, kv_chunks, n_bh, cu_count, batch * num_heads * seq_q, head_dim, causal, persistent)
+    else:
+        # (The split blocks, the last fwd_split, are two items of half their tiles.)
+        longest = max(max(tiles[:n_mblk - fwd_split], default=0), _cdiv(max(tiles[n_mblk - fwd_split:], default=0), 2))
+        lo, hi = OTHER_STEP_US["single"][head_dim]
+        other = _step_us(lo, hi, sum(tiles) * n_bh, longest, cu_count) * fwd_split_makespan(
+            tiles, fwd_split, n_bh, cu_count, causal, persistent)
+    return short_us(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim) < other
+
+
 def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int,
                 cu_count: int, causal: bool = True, head_dim: int = 128) -> Route:
-    """What gqa_flash_attn launches: choose_route's route, refined for at most
-    flat_max_rows(head_dim) packed rows per kv head (a token or a few).
+    """What gqa_flash_attn launches: choose_route's route, refined.
+
+    More than flat_max_rows(head_dim) packed rows per kv head: the short form
+    of the single pass where use_short says so, and the split-KV pass for the
+    remaining caches below SPLIT_MIN_KV keys.  At most that many (a token or a
+    few):
 
     * Caches below SPLIT_MIN_KV keys are split as longer ones are (the single
       pass would give each kv head one workgroup of 256 rows, of which 4 hold
@@ -446,11 +536,24 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
       compute units take the flat split (FLAT_MIN_USED)."""
     route = choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
     rows = num_heads // num_kv_heads * seq_q
-    if not 0 < rows <= flat_max_rows(head_dim) or seq_kv <= 0 or batch <= 0:
+    if rows <= 0 or seq_kv <= 0 or batch <= 0:
         return route
-    base = num_kv_heads * batch
-    splits = split_count(base, seq_kv, cu_count, split_rows_per_workgroup(rows, head_dim), head_dim,
-                         rows16=rows <= DEC16_ROWS)
+    if rows > flat_max_rows(head_dim) and use_short(
+            batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
+            route.splits if route.kind == "chunks" else 0, route.fwd_split, head_dim == 128):
+        wgs = _cdiv(seq_q, SHORT_ROWS // (num_heads // num_kv_heads)) * num_kv_heads * batch
+        if route.kind == "single":
+            need = _fwd_split_bytes(batch, num_kv_heads, head_dim, route.fwd_split)
+        else:
+            need = workspace_bytes(batch, num_heads, seq_q, head_dim, route.splits)
+        return Route("short", 1, wgs, reserve=need)
+    if rows > split_max_rows(head_dim):
+        return route
+    rpw = split_rows_per_workgroup(rows, head_dim)
+    base = _cdiv(rows, rpw) * num_kv_heads * batch
+    splits = split_count(base, seq_kv, cu_count, rpw, head_dim, rows16=rows <= DEC16_ROWS)
+    if rows > flat_max_rows(head_dim):
+        return Route("split", splits, base * splits)
 
     def used(wgs: int) -> float:
         return wgs / (cu_count * _cdiv(wgs, cu_count))
@@ -529,6 +632,11 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
         return _launch(route, q, k, v, causal, return_lse, dev)
 
 
+def _base_route(q, k, causal, dev):
+    batch, num_heads, seq_q, head_dim = q.shape
+    return _route_cached(batch, num_heads, k.shape[1], seq_q, k.shape[2], _cu_count(dev), bool(causal), head_dim)
+
+
 def _launch(route, q_in, k, v, causal, return_lse, dev):
     # One test for the usual case (all three kernel-ready; 2-byte elements:
     # the dtype is asserted), the per-tensor copies otherwise.
@@ -539,12 +647,15 @@ def _launch(route, q_in, k, v, causal, return_lse, dev):
         q = q_in
     else:
         q, k, v = _kernel_ready(q_in), _kernel_ready(k), _kernel_ready(v)
+    if route.kind != "single" and (k.shape[2] + 192) * max(k.stride(2), v.stride(2)) >= 1 << 30:
+        # Rows so far apart that 32-bit byte offsets cannot span the keys:
+        # the route by shape alone, whose split-KV pass takes them.
+        route = _base_route(q, k, causal, dev)
     if route.kind == "flat":
         out = flat_forward(q, k, v, causal, route.splits, return_lse, dev)
         if out is not None:
             return out
-        batch, num_heads, seq_q, head_dim = q.shape
-        route = _route_cached(batch, num_heads, k.shape[1], seq_q, k.shape[2], _cu_count(dev), bool(causal), head_dim)
+        route = _base_route(q, k, causal, dev)
     if route.kind == "split":
         return decode_forward(q, k, v, causal, route.splits, return_lse, dev)
     o = torch.empty_like(q_in)  # as dispatch.py:47; contiguous if unusable
@@ -552,6 +663,10 @@ def _launch(route, q_in, k, v, causal, return_lse, dev):
         o = torch.empty_like(q_in, memory_format=torch.contiguous_format)
     if route.kind == "chunks":
         return chunks_forward(q, k, v, o, causal, route.splits, return_lse)
+    if route.kind == "short":
+        if route.reserve:
+            _workspace_buffer(q.device, stream_handle(q.device), route.reserve)
+        return short_forward(q, k, v, o, causal, return_lse)
     return single_pass_forward(q, k, v, o, causal, route.fwd_split, return_lse)
 
 
@@ -580,6 +695,20 @@ def single_pass_forward(q, k, v, o, causal, fwd_split=0, return_lse=False):
                                lib.gqa_fwd_split_workspace_bytes(batch, num_kv_heads, head_dim, fwd_split))
     _lib.check(lib.gqa_fwd_split_launch(*qkvo, None if lse is None else lse.data_ptr(),
                                         None if ws is None else ws.data_ptr(), cnt.data_ptr(), fwd_split, *common))
+    return o if lse is None else (o, lse)
+
+
+def short_forward(q, k, v, o, causal, return_lse=False):
+    """Launch the short form of the single pass (gqa_fwd_short_launch) on
+    kernel-ready q, k, v and output o."""
+    batch, num_heads, seq_q, head_dim = q.shape
+    _, num_kv_heads, seq_kv, _ = k.shape
+    lse = torch.empty(batch, num_heads, seq_q, dtype=torch.float32, device=q.device) if return_lse else None
+    _lib.check(_lib.load().gqa_fwd_short_launch(
+        q.data_ptr(), _lib.strides(q), k.data_ptr(), _lib.strides(k), v.data_ptr(), _lib.strides(v),
+        o.data_ptr(), _lib.strides(o), None if lse is None else lse.data_ptr(), batch, num_heads, num_kv_heads,
+        seq_q, seq_kv, head_dim, (head_dim ** -0.5) * LOG2E, int(bool(causal)), _DTYPES[q.dtype],
+        stream_handle(q.device)))
     return o if lse is None else (o, lse)
 
 

@@ -41,7 +41,7 @@ import torch
 
 from . import _lib
 from .dispatch import (FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
-                       fwd_split_makespan)
+                       fwd_split_makespan, use_short)
 from .gqa_split import (_counter_buffer, _decode_host, _workspace_buffer, flat_workspace_bytes, stream_handle,
                         workspace_bytes)
 
@@ -204,7 +204,7 @@ def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     return slots if 0 < rows <= flat_max_rows(head_dim) and 1 <= slots <= _lib.GQA_MAX_SPLITS else 0
 
 
-_ROUTE_IDS = {"split": 0, "single": 1, "chunks": 2, "flat": 3}
+_ROUTE_IDS = {"split": 0, "single": 1, "chunks": 2, "flat": 3, "short": 4}
 
 
 def _paged_host():
@@ -297,6 +297,20 @@ def paged_single_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int,
     return 0, n_split
 
 
+@functools.lru_cache(maxsize=4096)
+def paged_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_seq_len: int, cu_count: int,
+                causal: bool = True, block_size: int = 64, head_dim: int = 128) -> bool:
+    """Whether a paged call takes the short form of the single pass
+    (gqa_paged_fwd_short_launch, dispatch.use_short) in place of
+    paged_route's split-KV pass over more rows than the flat split takes, or
+    of paged_single_plan's single pass."""
+    rows = num_heads // num_kv_heads * seq_q
+    if rows <= flat_max_rows(head_dim) or max_seq_len < 1 or block_size < single_pass_min_block(head_dim):
+        return False
+    kc, ns = paged_single_plan(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, causal, head_dim)
+    return use_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, causal, head_dim, kc, ns, False)
+
+
 def paged_kv_chunks(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_seq_len: int,
                     cu_count: int, causal: bool = True, head_dim: int = 128) -> int:
     """Key chunks per query block for the paged single pass (0: none; see
@@ -339,10 +353,12 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             (batch, num_heads, seq_q).
         out: optional (batch, num_heads, seq_q, head_dim) tensor of q's dtype
             (any strides with 16-byte aligned rows) to write o into.
-        route: "split", "single" or "chunks" to force a kernel (default:
-            paged_route, and "chunks" in place of "single" when
-            paged_kv_chunks finds few query blocks against long sequences;
-            "single" and "chunks" need block_size >= 512 / head_dim).
+        route: "split", "single", "chunks" or "short" to force a kernel
+            (default: paged_route, "chunks" in place of "single" when
+            paged_kv_chunks finds few query blocks against long sequences, and
+            "short", the short form of the single pass, where paged_short
+            finds it faster; all but "split" need block_size >= 512 /
+            head_dim).
         query_start, query_lens, max_query_len: variable query lengths.  q
             is then token-major (num_tokens, num_heads, head_dim); sequence
             b's queries are tokens query_start[b] .. + query_lens[b] - 1
@@ -417,7 +433,12 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     kv_chunks = fwd_split = 0
     if route is None:
         route = paged_route(num_heads, num_kv_heads, seq_q, block_size, head_dim)
-        if route == "single":
+        # (The short form spans a tile's 64 rows with 32-bit byte offsets.)
+        if (not splits_given and max(k_cache.stride(1), v_cache.stride(1)) < 1 << 24
+                and paged_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), bool(causal),
+                                block_size, head_dim)):
+            route = "short"
+        elif route == "single":
             kv_chunks, fwd_split = paged_single_plan(batch, num_heads, num_kv_heads, seq_q, max_seq_len,
                                                      _cu_count(dev), bool(causal), head_dim)
             route = "chunks" if kv_chunks else route
@@ -426,7 +447,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     elif route == "chunks":
         kv_chunks = splits if splits_given else max(2, paged_kv_chunks(
             batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), causal, head_dim))
-    assert route in ("split", "single", "chunks")
+    assert route in ("split", "single", "chunks", "short")
     assert route == "split" or block_size >= single_pass_min_block(head_dim)
     lse = torch.empty(lse_shape, dtype=torch.float32, device=qdev) if return_lse else None
     counters = None
@@ -451,7 +472,9 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
                 _lib.check(rc)
         if done:
             return out if lse is None else (out, lse)
-    if route == "single":
+    if route == "short":
+        n_parts, workspace = 0, None
+    elif route == "single":
         # Split query blocks: their halves' fp32 state and the stream's
         # zeroed merge counters (left zero by the kernel).
         n_parts = fwd_split
@@ -477,6 +500,14 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             v_cache.data_ptr(), _lib.strides(v_cache), block_table.data_ptr(), table_stride,
             seq_lens.data_ptr(), qs_p, ql_p, block_size, max_seq_len, out.data_ptr(), ost,
             lse_p, workspace.data_ptr(), kv_chunks, batch, num_heads, num_kv_heads, seq_q, head_dim,
+            scale * LOG2E, int(bool(causal)), dtype, stream))
+        return out if lse is None else (out, lse)
+    if route == "short":
+        _lib.check(lib.gqa_paged_fwd_short_launch(
+            q.data_ptr(), qst, k_cache.data_ptr(), _lib.strides(k_cache),
+            v_cache.data_ptr(), _lib.strides(v_cache), block_table.data_ptr(), table_stride,
+            seq_lens.data_ptr(), qs_p, ql_p, block_size, max_seq_len, out.data_ptr(), ost,
+            lse_p, batch, num_heads, num_kv_heads, seq_q, head_dim,
             scale * LOG2E, int(bool(causal)), dtype, stream))
         return out if lse is None else (out, lse)
     if route == "single" and fwd_split:
@@ -804,12 +835,7 @@ class GQAPagedAttention(torch.nn.Module):
             else:
                 tables, lens = md.block_tables.index_select(0, sel), md.seq_lens.index_select(0, sel)
             max_q = max(md.query_lens[b] for b in idx)
-            route, splits = kind, None
-            if kind == "single":
-                dev = query.device.index if query.device.index is not None else torch.cuda.current_device()
-                kc, ns = paged_single_plan(n, H, Hkv, max_q, max_seq_len, _cu_count(dev), bool(self.causal), D)
-                route, splits = ("chunks", kc) if kc else ("single", ns)
+            # (paged_attention routes the longest query block as `kind`.)
             paged_attention(q3, k_cache, v_cache, tables, lens, self.causal, max_seq_len=max_seq_len,
-                            scale=self.scale, out=o3, route=route, splits=splits, query_start=qs,
-                            query_lens=ql, max_query_len=max_q)
+                            scale=self.scale, out=o3, query_start=qs, query_lens=ql, max_query_len=max_q)
         return output

@@ -252,6 +252,32 @@ int gqa_split_launch(const void* q, const int64_t q_stride[4],
                      int seq_q, int seq_kv, int head_dim,
                      float scale_log2, int causal, int dtype, void* stream);
 
+/* The single pass in the form for short calls: workgroups of 128 packed rows
+ * whose two wave groups split the keys (merged before o is written), twice as
+ * many of them with half as long a chain of key tiles each as
+ * gqa_fwd_lse_launch / gqa_paged_fwd_launch, whose arguments they take (lse may
+ * be NULL) and whose results they give up to rounding.  num_heads /
+ * num_kv_heads at most 128 (GQA_E_GROUP). */
+int gqa_fwd_short_launch(const void* q, const int64_t q_stride[4],
+                         const void* k, const int64_t k_stride[4],
+                         const void* v, const int64_t v_stride[4],
+                         void* o, const int64_t o_stride[4], float* lse,
+                         int batch, int num_heads, int num_kv_heads,
+                         int seq_q, int seq_kv, int head_dim,
+                         float scale_log2, int causal, int dtype,
+                         void* stream);
+int gqa_paged_fwd_short_launch(const void* q, const int64_t q_stride[4],
+                               const void* k_cache, const int64_t k_cache_stride[4],
+                               const void* v_cache, const int64_t v_cache_stride[4],
+                               const int* block_table, int table_stride,
+                               const int* seq_lens, const int* q_start,
+                               const int* q_len, int block_size,
+                               int max_seq_len, void* o,
+                               const int64_t o_stride[4], float* lse, int batch,
+                               int num_heads, int num_kv_heads, int seq_q,
+                               int head_dim, float scale_log2, int causal,
+                               int dtype, void* stream);
+
 /* Flat split-KV forward (no counterpart in the reference, whose splits cut
  * every sequence alike): the keys of all sequences are laid end to end in
  * tile steps (64 keys, 128 at head_dim 64) and cut into `slots` equal ranges

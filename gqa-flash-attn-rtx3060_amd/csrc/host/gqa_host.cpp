@@ -20,10 +20,19 @@
 // libgqa_hip.so, which it links against.
 #include <torch/extension.h>
 
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/python_arg_parser.h>
 
+#include <algorithm>
+#include <array>
 #include <stdexcept>
 #include <string>
+#include <unordered_map>
 
 #include "gqa_attn.h"
 
@@ -224,6 +233,320 @@ void cache_write(const at::Tensor& key, const at::Tensor& value, const at::Tenso
   if (rc != GQA_OK) raise_rc(rc, "gqa_paged_cache_write_launch");
 }
 
+// ---------------------------------------------------------------------------
+// Whole calls.  gqa_flash_attn and paged_attention spend 10-20 us per call in
+// Python on checks, the route and the launch arguments, more than the kernels
+// of a short call take on the GPU (333 tokens: 16 us of host time beside 9.9
+// us).  These entries do the usual case natively: every check passes, the
+// route of these shapes is known (set_plan, from Python's rules) and the
+// stream's buffers are large enough.  Anything else returns None before
+// allocating or launching, and Python takes the call: it raises, copies,
+// chooses the route (and registers it here) or grows the buffer.
+// ---------------------------------------------------------------------------
+enum Kind : int { kSplit = 0, kSingle = 1, kChunks = 2, kFlat = 3, kShort = 4 };
+
+struct Plan {
+  int kind, n;         // n: splits, split blocks, key chunks or slots
+  int64_t reserve;     // bytes of stream workspace the call keeps
+  float scale_log2;    // gqa_flash_attn: head_dim^-0.5 * log2(e)
+};
+
+using Key = std::array<int64_t, 12>;
+struct KeyHash {
+  size_t operator()(const Key& k) const {
+    uint64_t h = 1469598103934665603ull;
+    for (int64_t v : k) h = (h ^ (uint64_t)v) * 1099511628211ull;
+    return (size_t)(h ^ (h >> 32));
+  }
+};
+// Calls hold the GIL throughout, which guards the table; bounded as Python's
+// own route caches are.
+std::unordered_map<Key, Plan, KeyHash> g_plans;
+
+void set_plan(const std::vector<int64_t>& key, int64_t kind, int64_t n, int64_t reserve, double scale_log2) {
+  Key k{};
+  if (key.size() != k.size()) throw std::invalid_argument("set_plan: key length");
+  std::copy(key.begin(), key.end(), k.begin());
+  if (g_plans.size() >= 8192) g_plans.clear();
+  g_plans[k] = Plan{static_cast<int>(kind), static_cast<int>(n), reserve, static_cast<float>(scale_log2)};
+}
+
+// A plain tensor (no subclass, wrapper or active mode that would have to see
+// the call), or nullptr.
+const at::Tensor* plain(const py::handle& h) {
+  if (!THPVariable_CheckExact(h.ptr())) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(h.ptr());
+  if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || at::isTensorSubclassLike(t)) return nullptr;
+  return &t;
+}
+bool modes_active() {
+  return at::impl::torch_function_mode_enabled() || c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
+bool half_type(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
+int dtype_code(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? GQA_DTYPE_BF16 : GQA_DTYPE_FP16; }
+
+// Unit last stride, every other stride and the pointer multiples of 16 bytes
+// (2-byte elements).
+bool rows_ready(const at::Tensor& t) {
+  const int64_t d = t.dim();
+  if (t.stride(d - 1) != 1) return false;
+  uint64_t bits = reinterpret_cast<uintptr_t>(t.data_ptr());
+  for (int64_t i = 0; i < d - 1; ++i) bits |= 2 * static_cast<uint64_t>(t.stride(i));
+  return (bits & 15) == 0;
+}
+
+// The stream's buffer of at least `bytes` bytes from gqa_split's dictionary,
+// or nullptr.
+void* stream_buffer(const py::dict& buffers, int64_t dev, hipStream_t stream, size_t bytes) {
+  const py::tuple key = py::make_tuple(dev, reinterpret_cast<intptr_t>(stream));
+  PyObject* v = PyDict_GetItemWithError(buffers.ptr(), key.ptr());
+  if (v == nullptr) {
+    PyErr_Clear();
+    return nullptr;
+  }
+  if (!THPVariable_Check(v)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(v);
+  return t.nbytes() >= bytes ? t.data_ptr() : nullptr;
+}
+
+bool capturing() {
+  return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
+
+void check_rc(int rc, const char* what) {
+  if (rc != GQA_OK) raise_rc(rc, what);
+}
+
+// gqa_flash_attn(q, k, v, causal, return_lse), or None.  workspaces, counters:
+// gqa_split's per-stream buffers.
+py::object flash_attn(const py::handle& hq, const py::handle& hk, const py::handle& hv, bool causal, bool return_lse,
+                      const py::dict& workspaces, const py::dict& counters) {
+  const at::Tensor *pq = plain(hq), *pk = plain(hk), *pv = plain(hv);
+  if (pq == nullptr || pk == nullptr || pv == nullptr || modes_active()) return py::none();
+  const at::Tensor &q = *pq, &k = *pk, &v = *pv;
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || !half_type(q) || k.scalar_type() != q.scalar_type() ||
+      v.scalar_type() != q.scalar_type() || v.sizes() != k.sizes())
+    return py::none();
+  const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3), Hkv = k.size(1), Skv = k.size(2);
+  const int64_t dev = q.get_device();
+  if (k.size(0) != B || k.size(3) != D || k.get_device() != dev || v.get_device() != dev ||
+      c10::hip::current_device() != dev)
+    return py::none();
+  const auto found = g_plans.find(Key{0, B, Hq, Hkv, Sq, Skv, D, causal, dev});
+  if (found == g_plans.end() || !rows_ready(q) || !rows_ready(k) || !rows_ready(v)) return py::none();
+  const Plan p = found->second;
+  if (p.kind != kSingle && (Skv + 192) * std::max(k.stride(2), v.stride(2)) >= ((int64_t)1 << 30)) return py::none();
+  hipStream_t stream = c10::hip::getCurrentHIPStream(dev).stream();
+
+  void *ws = nullptr, *cnt = nullptr;
+  size_t need = static_cast<size_t>(p.reserve);
+  if (p.kind == kSplit || p.kind == kChunks)
+    need = gqa_split_workspace_bytes(B, Hq, Sq, D, p.n);
+  else if (p.kind == kFlat)
+    need = gqa_split_flat_workspace_bytes(B, Hq, Sq, D, p.n);
+  else if (p.kind == kSingle)
+    need = gqa_fwd_split_workspace_bytes(B, Hkv, D, p.n);
+  if (need > 0 && (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr) return py::none();
+  if (p.kind == kSingle || p.kind == kChunks) {
+    // (A captured call gets counters of its own.)
+    const size_t n = gqa_fwd_split_counters_count(B, Hkv, p.kind == kSingle ? p.n : 0);
+    if (capturing() || (cnt = stream_buffer(counters, dev, stream, n * sizeof(int))) == nullptr) return py::none();
+  }
+  at::Tensor o = at::empty_like(q);
+  if (!rows_ready(o)) return py::none();
+  at::Tensor lse;
+  if (return_lse) lse = at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat));
+  float* lse_p = return_lse ? lse.data_ptr<float>() : nullptr;
+  int64_t qs[4], ks[4], vs[4], os[4];
+  strides_of(q, qs);
+  strides_of(k, ks);
+  strides_of(v, vs);
+  strides_of(o, os);
+  const int b = B, hq_ = Hq, hkv = Hkv, sq = Sq, skv = Skv, d = D, c = causal ? 1 : 0, dt = dtype_code(q);
+  const float sl2 = p.scale_log2;
+  float* wsf = static_cast<float*>(ws);
+  int* cnti = static_cast<int*>(cnt);
+  const void *qp = q.data_ptr(), *kp = k.data_ptr(), *vp = v.data_ptr();
+  void* op = o.data_ptr();
+  if (p.kind == kSplit) {
+    check_rc(gqa_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2, c, dt,
+                              stream), "gqa_split_launch");
+  } else if (p.kind == kFlat) {
+    const int rc = gqa_split_flat_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2,
+                                         c, dt, stream);
+    if (rc == GQA_E_FLAT) return py::none();
+    check_rc(rc, "gqa_split_flat_launch");
+  } else if (p.kind == kShort) {
+    check_rc(gqa_fwd_short_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, b, hq_, hkv, sq, skv, d, sl2, c, dt, stream),
+             "gqa_fwd_short_launch");
+  } else if (p.kind == kChunks) {
+    check_rc(gqa_fwd_chunks_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2,
+                                   c, dt, stream), "gqa_fwd_chunks_launch");
+  } else {
+    check_rc(gqa_fwd_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2,
+                                  c, dt, stream), "gqa_fwd_split_launch");
+  }
+  if (return_lse) return py::make_tuple(o, lse);
+  return py::cast(o);
+}
+
+// (num_blocks, block_size, Hkv, D) caches paged_attention and write_kv accept.
+bool caches_ready(const at::Tensor& kc, const at::Tensor& vc) {
+  if (kc.dim() != 4 || vc.dim() != 4 || kc.sizes() != vc.sizes() || kc.scalar_type() != vc.scalar_type() ||
+      kc.get_device() != vc.get_device() || !half_type(kc))
+    return false;
+  const int64_t bs = kc.size(1);
+  return bs >= 1 && bs <= GQA_MAX_BLOCK_SIZE && (bs & (bs - 1)) == 0 && rows_ready(kc) && rows_ready(vc);
+}
+bool int_rows(const at::Tensor* t, int64_t n, int64_t dev) {
+  return t != nullptr && t->scalar_type() == at::kInt && t->dim() == 1 && t->size(0) == n && t->is_contiguous() &&
+         t->get_device() == dev;
+}
+
+// paged_attention on its default route, or None.  max_seq_len and
+// max_query_len < 0: not given; qstart None: uniform query lengths.
+py::object paged_attn(const py::handle& hq, const py::handle& hkc, const py::handle& hvc, const py::handle& htab,
+                      const py::handle& hlens, bool causal, int64_t max_seq_len, double scale_log2, bool return_lse,
+                      const py::handle& hout, const py::handle& hqs, const py::handle& hql, int64_t max_query_len,
+                      const py::dict& workspaces, const py::dict& counters) {
+  const at::Tensor *pq = plain(hq), *pkc = plain(hkc), *pvc = plain(hvc), *ptab = plain(htab), *plens = plain(hlens);
+  if (pq == nullptr || pkc == nullptr || pvc == nullptr || ptab == nullptr || plens == nullptr || modes_active())
+    return py::none();
+  const at::Tensor &q = *pq, &kc = *pkc, &vc = *pvc, &tab = *ptab, &lens = *plens;
+  const bool varlen = !hqs.is_none();
+  if (q.dim() != (varlen ? 3 : 4) || !caches_ready(kc, vc) || q.scalar_type() != kc.scalar_type() || !rows_ready(q))
+    return py::none();
+  const int64_t dev = q.get_device(), H = q.size(1), D = q.size(-1), Hkv = kc.size(2), bs = kc.size(1);
+  const int64_t B = varlen ? (lens.dim() == 1 ? lens.size(0) : -1) : q.size(0);
+  const int64_t Sq = varlen ? max_query_len : q.size(2);
+  const at::Tensor *qst = nullptr, *qln = nullptr;
+  if (varlen) {
+    qst = plain(hqs);
+    qln = plain(hql);
+    if (Sq < 0 || !int_rows(qst, B, dev) || !int_rows(qln, B, dev)) return py::none();
+  }
+  if (kc.get_device() != dev || kc.size(3) != D || !int_rows(&lens, B, dev) || tab.scalar_type() != at::kInt ||
+      tab.dim() != 2 || tab.size(0) != B || tab.get_device() != dev || tab.stride(1) != 1 ||
+      (B > 1 && tab.stride(0) < tab.size(1)) || c10::hip::current_device() != dev)
+    return py::none();
+  const int64_t capacity = tab.size(1) * bs;
+  if (max_seq_len < 0) max_seq_len = capacity;
+  if (max_seq_len > capacity) return py::none();
+  const bool interleaved = kc.stride(1) != D || vc.stride(1) != D;
+  const auto found = g_plans.find(Key{1, B, H, Hkv, Sq, max_seq_len, D, causal, dev, bs, interleaved, varlen});
+  if (found == g_plans.end()) return py::none();
+  const Plan p = found->second;
+  if (p.kind == kShort && std::max(kc.stride(1), vc.stride(1)) >= ((int64_t)1 << 24)) return py::none();
+  hipStream_t stream = c10::hip::getCurrentHIPStream(dev).stream();
+  void *ws = nullptr, *cnt = nullptr;
+  size_t need = 0;
+  if (p.kind == kSplit || p.kind == kChunks)
+    need = gqa_split_workspace_bytes(B, H, Sq, D, p.n);
+  else if (p.kind == kFlat)
+    need = gqa_split_flat_workspace_bytes(B, H, Sq, D, p.n);
+  else if (p.kind == kSingle)
+    need = gqa_fwd_split_workspace_bytes(B, Hkv, D, p.n);
+  if (need > 0 && (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr) return py::none();
+  if (p.kind == kSingle && p.n > 0) {
+    const size_t n = gqa_fwd_split_counters_count(B, Hkv, p.n);
+    if (capturing() || (cnt = stream_buffer(counters, dev, stream, n * sizeof(int))) == nullptr) return py::none();
+  }
+  at::Tensor out;
+  if (hout.is_none()) {
+    out = at::empty(q.sizes(), q.options());
+  } else {
+    const at::Tensor* po = plain(hout);
+    if (po == nullptr || po->sizes() != q.sizes() || po->scalar_type() != q.scalar_type() || po->get_device() != dev ||
+        !rows_ready(*po))
+      return py::none();
+    out = *po;
+  }
+  at::Tensor lse;
+  if (return_lse)
+    lse = varlen ? at::empty({q.size(0), H}, q.options().dtype(at::kFloat))
+                 : at::empty({B, H, Sq}, q.options().dtype(at::kFloat));
+  float* lse_p = return_lse ? lse.data_ptr<float>() : nullptr;
+  int64_t qs[4], os[4], ks[4], vs[4];
+  if (varlen) {
+    const int64_t qv[4] = {0, q.stride(1), q.stride(0), 1}, ov[4] = {0, out.stride(1), out.stride(0), 1};
+    std::copy(qv, qv + 4, qs);
+    std::copy(ov, ov + 4, os);
+  } else {
+    strides_of(q, qs);
+    strides_of(out, os);
+  }
+  strides_of(kc, ks);
+  strides_of(vc, vs);
+  const int b = B, h = H, hkv = Hkv, sq = Sq, d = D, c = causal ? 1 : 0, dt = dtype_code(q), bsz = bs;
+  const int ms = max_seq_len, ts = B > 1 ? tab.stride(0) : tab.size(1);
+  const float sl2 = scale_log2;
+  const int *tp = tab.data_ptr<int>(), *lp = lens.data_ptr<int>();
+  const int* qsp = varlen ? qst->data_ptr<int>() : nullptr;
+  const int* qlp = varlen ? qln->data_ptr<int>() : nullptr;
+  float* wsf = static_cast<float*>(ws);
+  const void *qp = q.data_ptr(), *kp = kc.data_ptr(), *vp = vc.data_ptr();
+  void* op = out.data_ptr();
+  if (p.kind == kFlat) {
+    const int rc = gqa_paged_split_flat_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, op, os, lse_p,
+                                               wsf, p.n, b, h, hkv, sq, d, sl2, c, dt, stream);
+    if (rc == GQA_E_FLAT) return py::none();
+    check_rc(rc, "gqa_paged_split_flat_launch");
+  } else if (p.kind == kShort) {
+    check_rc(gqa_paged_fwd_short_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, op, os, lse_p, b, h,
+                                        hkv, sq, d, sl2, c, dt, stream), "gqa_paged_fwd_short_launch");
+  } else if (p.kind == kChunks) {
+    check_rc(gqa_paged_fwd_chunks_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, op, os, lse_p, wsf,
+                                         p.n, b, h, hkv, sq, d, sl2, c, dt, stream), "gqa_paged_fwd_chunks_launch");
+  } else if (p.kind == kSingle && p.n > 0) {
+    check_rc(gqa_paged_fwd_split_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, op, os, lse_p, wsf,
+                                        static_cast<int*>(cnt), p.n, b, h, hkv, sq, d, sl2, c, dt, stream),
+             "gqa_paged_fwd_split_launch");
+  } else if (p.kind == kSingle) {
+    check_rc(gqa_paged_fwd_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, op, os, lse_p, b, h, hkv, sq,
+                                  d, sl2, c, dt, stream), "gqa_paged_fwd_launch");
+  } else {
+    check_rc(gqa_paged_split_first_launch(qp, qs, kp, ks, vp, vs, tp, ts, lp, qsp, qlp, bsz, ms, wsf, p.n, b, h, hkv,
+                                          sq, d, sl2, c, dt, stream), "gqa_paged_split_first_launch");
+    int rc;
+    if (varlen)
+      rc = gqa_split_reduce_varlen_launch(wsf, p.n, op, os, lse_p, qsp, qlp, b, h, sq, d, dt, stream);
+    else if (return_lse)
+      rc = gqa_split_reduce_lse_launch(wsf, p.n, op, os, lse_p, b, h, sq, d, dt, stream);
+    else
+      rc = gqa_split_reduce_launch(wsf, p.n, op, os, b, h, sq, d, dt, stream);
+    check_rc(rc, "gqa_split_reduce_launch");
+  }
+  if (return_lse) return py::make_tuple(out, lse);
+  return py::cast(out);
+}
+
+// write_kv with its checks; false (nothing launched): Python takes the call.
+bool write_kv(const py::handle& hk, const py::handle& hv, const py::handle& hkc, const py::handle& hvc,
+              const py::handle& hslots) {
+  const at::Tensor *k = plain(hk), *v = plain(hv), *kc = plain(hkc), *vc = plain(hvc), *sl = plain(hslots);
+  if (k == nullptr || v == nullptr || kc == nullptr || vc == nullptr || sl == nullptr || modes_active()) return false;
+  if (k->dim() != 3 || v->sizes() != k->sizes() || !caches_ready(*kc, *vc) || kc->size(2) != k->size(1) ||
+      kc->size(3) != k->size(2) || k->scalar_type() != kc->scalar_type() || v->scalar_type() != k->scalar_type() ||
+      sl->scalar_type() != at::kLong || sl->dim() != 1 || sl->size(0) != k->size(0) || !sl->is_contiguous() ||
+      !rows_ready(*k) || !rows_ready(*v))
+    return false;
+  const int64_t dev = k->get_device();
+  if (v->get_device() != dev || kc->get_device() != dev || sl->get_device() != dev || c10::hip::current_device() != dev)
+    return false;
+  cache_write(*k, *v, *kc, *vc, *sl, dtype_code(*k));
+  return true;
+}
+
+// Host ints to an int32 tensor on `device` in one asynchronous copy from
+// pinned memory (the caching host allocator keeps the pinned block until the
+// copy has run).
+at::Tensor ints_to_device(const std::vector<int32_t>& v, int64_t device) {
+  const int64_t n = static_cast<int64_t>(v.size());
+  at::Tensor host = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  std::copy(v.begin(), v.end(), host.data_ptr<int>());
+  return host.to(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)), at::kInt, /*non_blocking=*/true);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -242,5 +565,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("scale_log2"), py::arg("causal"), py::arg("dtype"));
   m.def("cache_write", &cache_write, "store new tokens' K/V at their paged cache slots", py::arg("key"),
         py::arg("value"), py::arg("k_cache"), py::arg("v_cache"), py::arg("slot_mapping"), py::arg("dtype"));
+  m.def("flash_attn", &flash_attn, "gqa_flash_attn of a planned shape, or None");
+  m.def("paged_attn", &paged_attn, "paged_attention of a planned shape on its default route, or None");
+  m.def("write_kv", &write_kv, "write_kv with its checks, or False");
+  m.def("set_plan", &set_plan, "register the route of a shape");
+  m.def("ints_to_device", &ints_to_device, "host ints to an int32 device tensor, asynchronously");
   m.attr("ABI_VERSION") = gqa_abi_version();
 }

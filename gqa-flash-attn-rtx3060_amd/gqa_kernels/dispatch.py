@@ -16,7 +16,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .gqa_split import (_counter_buffer, _workspace_buffer, decode_forward, flat_forward, stream_handle,
+from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces, decode_forward, flat_forward, stream_handle,
                         workspace_bytes)
 
 __all__ = ["gqa_flash_attn", "Route", "choose_route"]
@@ -143,6 +143,9 @@ COMBINE_BYTES_PER_US = 5.0e6
 # Passes over the fp32 partials charged to the key-chunk route: written by
 # the first pass, read back by the combine (fitted: 1.5).
 CHUNK_PARTIAL_PASSES = 1.5
+
+# Route kinds as the native calls number them (gqa_host.cpp).
+_KIND_IDS = {"split": 0, "single": 1, "chunks": 2, "flat": 3, "short": 4}
 
 _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 
@@ -613,6 +616,12 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
         (batch, num_heads, seq_q, head_dim), same dtype as q; with
         return_lse=True the pair (o, lse).
     """
+    host = _lib._host
+    if host is not None:
+        # A planned shape with every check passed, natively; else None.
+        out = host.flash_attn(q, k, v, bool(causal), bool(return_lse), _workspaces, _counters)
+        if out is not None:
+            return out
     batch, num_heads, seq_q, head_dim = q.shape
     _, num_kv_heads, seq_kv, _ = k.shape
     assert num_heads % num_kv_heads == 0, "num_heads must be divisible by num_kv_heads"
@@ -626,6 +635,11 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
     assert k.get_device() == dev and v.get_device() == dev, "q, k, v must be on one device"
 
     route = _plan_cached(batch, num_heads, num_kv_heads, seq_q, seq_kv, _cu_count(dev), bool(causal), head_dim)
+    host = _decode_host()
+    if host is not None and batch > 0 and seq_q > 0:
+        host.set_plan([0, batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, int(bool(causal)), dev, 0, 0, 0],
+                      _KIND_IDS[route.kind], route.fwd_split if route.kind == "single" else route.splits,
+                      route.reserve, (head_dim ** -0.5) * LOG2E)
     if dev == torch.cuda.current_device():
         return _launch(route, q, k, v, causal, return_lse, dev)
     with torch.cuda.device(dev):  # launch on q's device

@@ -40,10 +40,10 @@ from typing import Dict, Hashable, List, Optional, Sequence
 import torch
 
 from . import _lib
-from .dispatch import (FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
+from .dispatch import (_KIND_IDS, FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
                        fwd_split_makespan, use_short)
-from .gqa_split import (_counter_buffer, _decode_host, _workspace_buffer, flat_workspace_bytes, stream_handle,
-                        workspace_bytes)
+from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces,
+                        flat_workspace_bytes, stream_handle, workspace_bytes)
 
 __all__ = [
     "paged_attention",
@@ -204,7 +204,6 @@ def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     return slots if 0 < rows <= flat_max_rows(head_dim) and 1 <= slots <= _lib.GQA_MAX_SPLITS else 0
 
 
-_ROUTE_IDS = {"split": 0, "single": 1, "chunks": 2, "flat": 3, "short": 4}
 
 
 def _paged_host():
@@ -371,6 +370,17 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
         o (batch, num_heads, seq_q, head_dim), or (o, lse).
     """
     varlen = query_start is not None
+    default_route = route is None and splits is None and (not varlen or query_lens is not None)
+    native = _lib._host if default_route else None
+    if native is not None:
+        # A planned shape with every check passed, natively; else None.
+        res = native.paged_attn(q, k_cache, v_cache, block_table, seq_lens, bool(causal),
+                                -1 if max_seq_len is None or max_seq_len < 0 else max_seq_len,
+                                (q.shape[-1] ** -0.5 if scale is None else scale) * LOG2E, bool(return_lse), out,
+                                query_start, query_lens, -1 if max_query_len is None else int(max_query_len),
+                                _workspaces, _counters) if max_seq_len is None or max_seq_len >= 0 else None
+        if res is not None:
+            return res
     qdev = q.device
     if varlen:
         assert query_lens is not None and max_query_len is not None, "varlen needs query_lens and max_query_len"
@@ -430,6 +440,11 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     lib = _lib.load()
     dtype = _DTYPES[q.dtype]
     stream = stream_handle(qdev)
+    plan_key = None
+    if default_route and batch > 0 and seq_q > 0:
+        interleaved = k_cache.stride(1) != head_dim or v_cache.stride(1) != head_dim
+        plan_key = [1, batch, num_heads, num_kv_heads, seq_q, max_seq_len, head_dim, int(bool(causal)), dev, block_size,
+                    int(interleaved), int(varlen)]
     kv_chunks = fwd_split = 0
     if route is None:
         route = paged_route(num_heads, num_kv_heads, seq_q, block_size, head_dim)
@@ -455,7 +470,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     if route == "split" and flat_slots:
         workspace = _workspace_buffer(qdev, stream, flat_workspace_bytes(batch, num_heads, seq_q, head_dim, flat_slots))
         if host is not None:
-            done = host.paged_forward(_ROUTE_IDS["flat"], q, k_cache, v_cache, block_table, table_stride, seq_lens,
+            done = host.paged_forward(_KIND_IDS["flat"], q, k_cache, v_cache, block_table, table_stride, seq_lens,
                                       query_start if varlen else None, query_lens if varlen else None, max_seq_len,
                                       out, lse, workspace, None, flat_slots, batch, seq_q, scale * LOG2E,
                                       bool(causal), dtype)
@@ -471,6 +486,8 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             if done:
                 _lib.check(rc)
         if done:
+            if host is not None and plan_key is not None:
+                host.set_plan(plan_key, _KIND_IDS["flat"], flat_slots, 0, 0.0)
             return out if lse is None else (out, lse)
     if route == "short":
         n_parts, workspace = 0, None
@@ -486,7 +503,9 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
         n_parts = kv_chunks if route == "chunks" else splits
         workspace = _workspace_buffer(qdev, stream, workspace_bytes(batch, num_heads, seq_q, head_dim, n_parts))
     if host is not None:
-        host.paged_forward(_ROUTE_IDS[route], q, k_cache, v_cache, block_table, table_stride, seq_lens,
+        if plan_key is not None:
+            host.set_plan(plan_key, _KIND_IDS[route], n_parts, 0, 0.0)
+        host.paged_forward(_KIND_IDS[route], q, k_cache, v_cache, block_table, table_stride, seq_lens,
                            query_start if varlen else None, query_lens if varlen else None, max_seq_len, out, lse,
                            workspace, counters, n_parts, batch, seq_q, scale * LOG2E, bool(causal), dtype)
         return out if lse is None else (out, lse)
@@ -551,6 +570,8 @@ def write_kv(key, value, k_cache, v_cache, slot_mapping):
     negative = skip (padding).  Every non-negative slot must lie inside the
     caches.
     """
+    if _lib._host is not None and _lib._host.write_kv(key, value, k_cache, v_cache, slot_mapping):
+        return
     block_size = _check_cache(k_cache, v_cache)
     num_tokens, num_kv_heads, head_dim = key.shape
     assert tuple(value.shape) == tuple(key.shape)
@@ -823,7 +844,11 @@ class GQAPagedAttention(torch.nn.Module):
         host = []
         for _, idx in groups:
             host += idx + [starts[b] for b in idx] + [md.query_lens[b] for b in idx]
-        meta = torch.tensor(host, dtype=torch.int32, pin_memory=True).to(query.device, non_blocking=True)
+        native = _paged_host()
+        if native is not None:
+            meta = native.ints_to_device(host, query.get_device())
+        else:
+            meta = torch.tensor(host, dtype=torch.int32, pin_memory=True).to(query.device, non_blocking=True)
         max_seq_len = md.max_seq_len if md.max_seq_len is not None else md.block_tables.shape[1] * block_size
         off = 0
         for kind, idx in groups:

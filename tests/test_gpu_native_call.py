@@ -1,0 +1,140 @@
+"""The native whole calls (gqa_host.cpp flash_attn, paged_attn, write_kv)
+against the Python path they stand in for: the first call of a shape runs in
+Python and registers its route, later ones run natively and give the same
+bits on every route, also on another stream and under graph capture; calls
+they do not take (unaligned rows, tensor subclasses) fall to Python, and
+wrong arguments raise as before once the shape is planned."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import make_inputs
+from test_gpu_paged import _paged_inputs
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _need_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    from gqa_kernels import _lib
+    _lib.load_host()
+
+
+def _python_only(monkeypatch):
+    """Calls take the Python path (the launches still go through the bindings)."""
+    from gqa_kernels import _lib
+
+    class Bindings:
+        def __init__(self, host):
+            self._host = host
+
+        def flash_attn(self, *a):
+            return None
+
+        paged_attn = flash_attn
+
+        def write_kv(self, *a):
+            return False
+
+        def __getattr__(self, name):
+            return getattr(self._host, name)
+
+    monkeypatch.setattr(_lib, "_host", Bindings(_lib._host))
+
+
+SHAPES = [(1, 32, 8, 1, 3000, 128), (5, 32, 8, 1, 2000, 128), (64, 32, 8, 1, 300, 64), (2, 32, 8, 150, 150, 128),
+          (1, 32, 8, 64, 5000, 128), (2, 8, 2, 3000, 3000, 64)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("lse", [False, True])
+def test_same_bits(shape, lse, monkeypatch):
+    from gqa_kernels import _lib, gqa_flash_attn
+    from gqa_kernels import gqa_split
+    q, k, v = make_inputs(*shape, torch.bfloat16, seed=1, device=DEV)
+    gqa_flash_attn(q, k, v)  # planned from here on
+    native = _lib._host.flash_attn(q, k, v, True, lse, gqa_split._workspaces, gqa_split._counters)
+    assert native is not None
+    with monkeypatch.context() as m:
+        _python_only(m)
+        ref = gqa_flash_attn(q, k, v, return_lse=lse)
+    for a, b in zip(native if lse else (native,), ref if lse else (ref,)):
+        assert torch.equal(a, b) and a.stride() == b.stride() and a.dtype == b.dtype
+
+
+def test_other_stream_and_capture():
+    """A stream without buffers falls to Python, which makes them; a captured
+    call replays to the eager bits."""
+    from gqa_kernels import gqa_flash_attn
+    for shape in SHAPES[:4]:
+        q, k, v = make_inputs(*shape, torch.bfloat16, seed=2, device=DEV)
+        want = gqa_flash_attn(q, k, v)
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            for _ in range(2):
+                assert torch.equal(gqa_flash_attn(q, k, v), want)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = gqa_flash_attn(q, k, v)
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            gqa_flash_attn(q, k, v)
+
+
+def test_refused_and_python_calls():
+    from gqa_kernels import gqa_flash_attn
+    q, k, v = make_inputs(2, 32, 8, 150, 150, 128, torch.bfloat16, seed=3, device=DEV)
+    want = gqa_flash_attn(q, k, v)
+    # rows off 16 bytes: copied
+    odd = torch.empty(k.numel() + 1, dtype=k.dtype, device=DEV)[1:].view_as(k)
+    odd.copy_(k)
+    assert torch.equal(gqa_flash_attn(q, odd, v), want)
+    # a tensor subclass
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert torch.equal(gqa_flash_attn(q.as_subclass(Sub), k, v).as_subclass(torch.Tensor), want)
+    for args in ((q, k, v[:, :4]), (q, k.half(), v), (q.float(), k.float(), v.float()), (q, k.cpu(), v.cpu()),
+                 (q[:, :31], k, v)):
+        with pytest.raises(AssertionError):
+            gqa_flash_attn(*args)
+
+
+@pytest.mark.parametrize("lens,sq", [([300, 40, 1000], 1), ([2000], 1), ([300, 200], 150), ([3000, 3000], 40),
+                                     ([900, 30], 12)])
+def test_paged_same_bits(lens, sq, monkeypatch):
+    from gqa_kernels.paged import paged_attention, write_kv
+    q, kc, vc, table, seq_lens = (t.to(DEV) for t in _paged_inputs(len(lens), 32, 8, sq, lens, 128, 16, torch.bfloat16,
+                                                                   seed=4))
+    new = torch.randn(3, 8, 128, device=DEV).to(torch.bfloat16)
+    slots = torch.tensor([int(table[0, 0]) * 16 + 5, -1, int(table[0, 0]) * 16 + 6], device=DEV)
+    results = []
+    for python in (True, False, False):
+        with monkeypatch.context() as m:
+            if python:
+                _python_only(m)
+            k2, v2 = kc.clone(), vc.clone()
+            write_kv(new, new, k2, v2, slots)
+            o = torch.empty_like(q)
+            res = paged_attention(q, k2, v2, table, seq_lens, max_seq_len=max(lens), return_lse=True, out=o)
+            assert res[0].data_ptr() == o.data_ptr()
+            results.append((k2, v2, *res))
+    for other in results[1:]:
+        for a, b in zip(results[0], other):
+            assert torch.equal(torch.nan_to_num(a.float()), torch.nan_to_num(b.float()))
+    for bad in (dict(max_seq_len=10 ** 6), dict(out=torch.empty(1, device=DEV))):
+        with pytest.raises(AssertionError):
+            paged_attention(q, kc, vc, table, seq_lens, **bad)
+    with pytest.raises(AssertionError):
+        paged_attention(q, kc, vc, table.long(), seq_lens, max_seq_len=max(lens))

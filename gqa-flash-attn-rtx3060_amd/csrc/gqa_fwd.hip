@@ -158,8 +158,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   const uint32_t kssb = (uint32_t)(2 * p.k.ss), vssb = (uint32_t)(2 * p.v.ss);
   auto decode = [&](int w, int i, int block_m) __attribute__((always_inline)) -> Item {
     Item x;
-    x.bh = fast_div(w, p.div_items.mul, p.div_items.shift);
-    int idx = w - x.bh * n_items;
+    int idx;
+    item_of(p, w, n_items, x.bh, idx);
     int chunk = 0;
     if constexpr (chunked) {
       chunk = fast_div(idx, p.div_mblk.mul, p.div_mblk.shift);
@@ -765,7 +765,7 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   const int per_bh = p.kv_splits > 0 ? p.n_mblk * p.kv_splits : p.n_mblk + p.n_split;
   const int total = per_bh * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
-  p.div_items = make_fast_div((uint32_t)per_bh);
+  set_item_order(p, per_bh, PG > 0 || D == 64);
   p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;

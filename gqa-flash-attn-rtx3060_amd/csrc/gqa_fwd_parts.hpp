@@ -5,8 +5,40 @@
 
 #include "gqa_common.hpp"
 #include "gqa_lds.hpp"
+#include "gqa_params.hpp"
 
 namespace gqa {
+
+// Work item w (XCD x takes items [x * total / 8, ...), xcd_remap) as item idx
+// of the (b, kv head) pair bh: pair after pair, or, with several pairs per XCD
+// (FwdParams::xcd_heads), pairs dealt to the XCDs in turn and an XCD's items
+// in the order first of each pair, second of each pair, ...  Dealt, a pair's
+// heavy items no longer start behind the light ones of the pair before it, and
+// the sequences of a batch of unequal lengths spread over all XCDs instead of
+// each filling XCDs of its own.  Measured (us, pair after pair / dealt):
+// * head_dim 64 (items handed out by the hardware as workgroups end): causal
+//   3 x 2999 tokens 131 / 117, 2 x 4096 153 / 138, 8 x 700 35.7 / 30.5;
+//   non-causal 4 x 1025 54.8 / 55.1.
+// * Paged, head_dim 128, 512 query tokens over [1700, 5262] keys: 82 / 71,
+//   short form 80 / 66; [600, 5000, 2000] with 400: 122 / 74; 4 x 17000 with
+//   382: 399 / 384.
+// * Contiguous head_dim 128: the persistent grid of gqa_fwd_kernel spreads its
+//   items itself and keeps the keys of fewer pairs in each L2: 4 x 1024 tokens
+//   42.8 / 44.6, 3 x 1800 58.3 / 60.6, so it stays with pair after pair.  The
+//   short form gains once its workgroups no longer start together: 4 x 300
+//   tokens (320 workgroups) 16.8 / 15.8, 8 x 300 over 16/4 heads 16.3 / 14.9;
+//   2 x 512 (256) 12.4 / 12.8.
+__device__ inline void item_of(const FwdParams& p, int w, int n_items, int& bh, int& idx) {
+  if (p.xcd_heads > 0) {
+    const int x = fast_div(w, p.div_share.mul, p.div_share.shift);
+    const int e = w - x * (p.xcd_heads * n_items);
+    idx = fast_div(e, p.div_heads.mul, p.div_heads.shift);
+    bh = (e - idx * p.xcd_heads) * 8 + x;
+  } else {
+    bh = fast_div(w, p.div_items.mul, p.div_items.shift);
+    idx = w - bh * n_items;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Online softmax of one 64-key S^T tile held as two 32-key blocks (16 values

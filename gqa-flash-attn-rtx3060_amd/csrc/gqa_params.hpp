@@ -45,6 +45,10 @@ struct FwdParams {
   // r < kFwdRows.
   FastDiv div_items, div_mblk, div_hkv;
   uint32_t bm_mul;
+  // Items dealt over the XCDs (item_of in gqa_fwd_parts.hpp): pairs of (b, kv
+  // head) per XCD, B * Hkv / 8 >= 2; 0: pair after pair (set_item_order).
+  int xcd_heads;
+  FastDiv div_heads, div_share;
   float* lse;   // optional (nullptr): natural-log LSE per row, contiguous (B, Hq, Sq)
   // Key-range split of the n_split heaviest query blocks of every (b, kv
   // head) into two work items (lower and upper half of the block's key
@@ -180,6 +184,16 @@ constexpr int kFusedMaxRowSplitsHost = 4096;
 // Block-table entries a split-KV workgroup over pages of fewer than 64 keys
 // copies to LDS (8 KiB): its chunk may span at most this many pages.
 constexpr int kPagedTableMax = 2048;
+
+// Item order of `per_bh` items per (b, kv head); div_items with it.  `deal`:
+// whether the kernel gains from pairs dealt to the XCDs (item_of).
+inline void set_item_order(FwdParams& p, int per_bh, bool deal) {
+  const int n_bh = p.dm.B * p.dm.Hkv;
+  p.div_items = make_fast_div((uint32_t)per_bh);
+  p.xcd_heads = deal && n_bh % 8 == 0 && n_bh > 8 ? n_bh / 8 : 0;
+  p.div_heads = make_fast_div((uint32_t)(p.xcd_heads > 0 ? p.xcd_heads : 1));
+  p.div_share = make_fast_div((uint32_t)(p.xcd_heads > 0 ? p.xcd_heads * per_bh : 1));
+}
 
 // Paged cache write: new tokens (num_tokens, Hkv, D) into
 // (num_blocks, block_size, Hkv, D) caches at slot_mapping[t].

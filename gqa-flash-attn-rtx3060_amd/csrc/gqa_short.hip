@@ -62,8 +62,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // Work item: one query block of one (b, kv head), heavy (late) blocks first
   // under causal; every XCD gets a contiguous range of items.
   const int w = xcd_remap(blockIdx.x, p.n_mblk * dm.Hkv * dm.B);
-  const int bh = fast_div(w, p.div_mblk.mul, p.div_mblk.shift);
-  const int mrank = w - bh * p.n_mblk;
+  int bh, mrank;
+  item_of(p, w, p.n_mblk, bh, mrank);
   const int pid_m = dm.causal ? p.n_mblk - 1 - mrank : mrank;
   const int b = fast_div(bh, p.div_hkv.mul, p.div_hkv.shift), kvh = bh - b * dm.Hkv;
   const int skv = PAGED ? min(max(load_uniform(p.seq_lens + b), 0), dm.Skv) : dm.Skv;
@@ -414,7 +414,7 @@ template <int DT, int D, int PG>
 static hipError_t launch_short_t(FwdParams p, hipStream_t stream) {
   const int64_t total = (int64_t)p.n_mblk * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
-  p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
+  set_item_order(p, p.n_mblk, PG > 0 || D == 64 || total > device_cu_count());
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;
   hipLaunchKernelGGL((gqa_short_kernel<DT, D, PG>), dim3((unsigned)total), dim3(kFwdThreads), 0, stream, p);

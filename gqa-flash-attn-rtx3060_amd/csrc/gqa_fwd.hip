@@ -97,7 +97,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
   // gets a contiguous range of items (same kv head -> same L2).  With a key
   // split, the n_split heaviest blocks of each (b, kv head) come as two
   // items: first the upper halves of their key ranges, then (in the usual
-  // order) the lower halves and the unsplit blocks.
+  // order) the lower halves and the unsplit blocks.  Without a mask all
+  // blocks are as long and the halves fill the last round: the unsplit
+  // blocks, then the upper and the lower halves of the last n_split.
   // Key chunks: kv_splits items per query block, the blocks of one chunk
   // consecutive (they read the same keys).
   constexpr bool chunked = KC;
@@ -165,11 +167,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4
       chunk = fast_div(idx, p.div_mblk.mul, p.div_mblk.shift);
       idx -= chunk * p.n_mblk;
     }
-    if (idx < p.n_split) {
-      x.pid_m = p.n_mblk - 1 - idx;
+    const int up = idx - (dm.causal ? 0 : p.n_mblk - p.n_split);  // place among the upper halves
+    if (up >= 0 && up < p.n_split) {
+      x.pid_m = p.n_mblk - 1 - up;
       x.part = 1;
     } else {
-      const int mrank = idx - p.n_split;
+      const int mrank = up < 0 ? idx : idx - p.n_split;
       x.pid_m = dm.causal ? (p.n_mblk - 1 - mrank) : mrank;
       x.part = (x.pid_m >= p.n_mblk - p.n_split) ? 0 : -1;
     }
@@ -765,7 +768,7 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   const int per_bh = p.kv_splits > 0 ? p.n_mblk * p.kv_splits : p.n_mblk + p.n_split;
   const int total = per_bh * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
-  set_item_order(p, per_bh, PG > 0 || D == 64);
+  set_item_order(p, per_bh, PG > 0 || D == 64 || (!p.dm.causal && p.n_split > 0));
   p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;

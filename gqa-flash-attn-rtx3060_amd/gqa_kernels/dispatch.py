@@ -123,6 +123,23 @@ FWD_ITEM_OVERHEAD = 8
 # at 512-3072 tokens, B = 1-5; the one-workgroup-per-item form at head_dim
 # 64 measured best without it).
 FWD_MERGE_OVERHEAD = 1
+# Without a mask every block is as long, and a last round of few blocks costs
+# as much as a full one (1025 keys, B = 4: 544 blocks on 256 CUs ran three
+# rounds).  With at most three eighths of it used, the blocks left over run as
+# two halves, dealt to the XCDs side by side after the whole blocks; up to
+# four times as many where the model sees no difference (a block's halves then
+# run in different rounds and do not wait for each other's state).  Measured,
+# us, whole / split blocks, head_dim 128: B = 4 x 1025 98.5 / 84.9, 2 x 1300
+# 70.3 / 61.7, 1 x 2304 110.4 / 91.8, 3 x 1500 124.0 / 112.7, 2 x 2100 163.1 /
+# 147.7, 2800 134.7 / 125.6, 6200 629 / 581 (3 rounds), 4 x 2049 288 / 273 (4
+# rounds).  With about half of it used, 3000 145.5 / 140.2, 8 x 1100 165.6 /
+# 172.3 (a part-filled chip steps faster, and halves on every CU bring many
+# merges); with more, 5 x 1100 104.1 / 116.  head_dim 64, two workgroups per
+# CU: 4352 196.4 / 169.9, 5000 231.7 / 211.7, 2 x 2304 108.8 / 97.9, 8 x 1025
+# 93.1 / 87.9, 6 x 700 40.2 / 37.2; 9 x 513 35.6 / 37.4, hence
+# FWD_FILL_MERGE_OVERHEAD (tile steps of a half's merge there).
+FWD_SPLIT_MAX_ROUNDS = 5
+FWD_FILL_MERGE_OVERHEAD = 4
 FWD_TILE = 64
 # The persistent single pass claims work dynamically only with at least this
 # many items per workgroup (kFwdDynMinItemsPerWg, gqa_params.hpp); below it
@@ -185,11 +202,23 @@ def fwd_split_makespan(tiles, n_split: int, n_bh: int, cu_count: int, causal: bo
     """Modelled run time (tile steps) of the single pass with the n_split
     heaviest blocks split: work items in the kernel's order (per (b, kv
     head): upper halves of the split blocks, then every block heavy-first
-    with split blocks as their lower halves), scheduled as _list_makespan
+    with split blocks as their lower halves; not causal: unsplit blocks,
+    then both halves of the last n_split), scheduled as _list_makespan
     describes (`persistent`: the head_dim-128 kernel over contiguous K/V)."""
     n = len(tiles)
     order = list(range(n - 1, -1, -1)) if causal else list(range(n))
     mo = FWD_MERGE_OVERHEAD if persistent else 0
+    if not causal and n_split > 0:
+        # (Pairs dealt to the XCDs: every XCD takes its pairs' items side by side.)
+        per_xcd = n_bh // 8 if n_bh % 8 == 0 else 1
+        mo = FWD_MERGE_OVERHEAD if persistent else FWD_FILL_MERGE_OVERHEAD
+        runs = []
+        for pid in range(n - n_split):
+            _push_run(runs, tiles[pid] + FWD_ITEM_OVERHEAD, per_xcd)
+        for half in (1, 0):
+            for pid in range(n - 1, n - n_split - 1, -1):
+                _push_run(runs, (tiles[pid] + half) // 2 + mo + FWD_ITEM_OVERHEAD, per_xcd)
+        return _list_makespan(runs, n_bh // per_xcd, cu_count, persistent)
     items = [tiles[n - 1 - i] - tiles[n - 1 - i] // 2 + mo for i in range(n_split)]
     for pid in order:
         items.append(tiles[pid] // 2 + mo if pid >= n - n_split else tiles[pid])
@@ -353,23 +382,43 @@ def choose_kv_chunks(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     return best_s if best <= (1.0 - FWD_SPLIT_GAIN) * base else 0
 
 
+def _fill_last_round(n_mblk: int, n_bh: int, seq_kv: int, cu_count: int, head_dim: int) -> int:
+    """Blocks per (b, kv head) whose halves fill the last round of a call
+    without a mask (FWD_SPLIT_MAX_ROUNDS), or 0."""
+    per_xcd, wgs = n_bh // 8, cu_count * (1 if head_dim == 128 else 2)
+    if n_bh % 8 or cu_count < 8 or not wgs < n_mblk * n_bh <= FWD_SPLIT_MAX_ROUNDS * wgs:
+        return 0
+    left = per_xcd * n_mblk % (wgs // 8)  # blocks per XCD in the last round
+    if left == 0 or left > 3 * wgs // 64:
+        return 0
+    tiles = [_cdiv(seq_kv, FWD_TILE)] * n_mblk
+    base, *times = (fwd_split_makespan(tiles, s * _cdiv(left, per_xcd), n_bh, wgs, False, persistent=head_dim == 128)
+                    for s in range(5) if s * _cdiv(left, per_xcd) <= n_mblk)
+    best = min(times)
+    last = max(i for i, t in enumerate(times) if t == best)
+    return (last + 1) * _cdiv(left, per_xcd) if best <= (1.0 - FWD_SPLIT_GAIN) * base else 0
+
+
 def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int,
                      cu_count: int, causal: bool, head_dim: int = 128, persistent: bool = None) -> int:
     """Query blocks per (b, kv head) to run as two key halves (0: none).
 
-    Only causal blocks differ in length; when there are few workgroups per
-    CU the longest block sets the run time, and splitting the heaviest ones
-    shortens it (fwd_split_makespan picks the count).  `persistent`
-    (default: head_dim 128) as fwd_split_makespan; False for paged caches."""
+    Under causal, when there are few workgroups per CU, the longest block
+    sets the run time, and splitting the heaviest ones shortens it
+    (fwd_split_makespan picks the count).  Not causal: FWD_SPLIT_MAX_ROUNDS.
+    `persistent` (default: head_dim 128) as fwd_split_makespan; False for
+    paged caches."""
     group = num_heads // num_kv_heads
     block_m = max(1, FWD_ROWS // group)
     n_mblk = _cdiv(seq_q, block_m)
     n_bh = batch * num_kv_heads
-    if not causal or n_mblk < 2 or n_mblk * n_bh >= FWD_SPLIT_MAX_WG_PER_CU * cu_count:
-        return 0
-    tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
+    if not causal:
+        return _fill_last_round(n_mblk, n_bh, seq_kv, cu_count, head_dim) if persistent is None else 0
     if persistent is None:
         persistent = head_dim == 128
+    if n_mblk < 2 or n_mblk * n_bh >= FWD_SPLIT_MAX_WG_PER_CU * cu_count:
+        return 0
+    tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
     base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent)
     best, best_ns = base, 0
     for f in (0.25, 0.375, 0.5, 0.625, 0.75, 1.0):

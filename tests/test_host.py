@@ -530,3 +530,20 @@ def test_kernel_ready_layouts():
         assert not _is_kernel_ready(t)
         c = _kernel_ready(t)
         assert c is not t and _is_kernel_ready(c) and torch.equal(c, t)
+
+
+def test_fill_last_round_choice():
+    """Calls without a mask split blocks only where few of them are left for
+    the last round, and never over a paged cache (persistent given)."""
+    from gqa_kernels.dispatch import choose_fwd_split, choose_plan, fwd_split_makespan
+    for B, S, D, some in [(4, 1025, 128, True), (1, 2304, 128, True), (1, 6200, 128, True), (4, 2049, 128, True),
+                          (1, 2048, 128, False), (1, 4096, 128, False), (8, 1100, 128, False), (9, 513, 128, False),
+                          (16, 1000, 128, False), (4, 1025, 64, True), (6, 700, 64, True), (9, 513, 64, False)]:
+        plan = choose_plan(B, 32, 8, S, S, 256, False, D)
+        assert plan.kind == "single" and (plan.fwd_split > 0) == some, (B, S, D, plan)
+        assert plan.fwd_split <= -(-S // 64)
+        assert choose_fwd_split(B, 32, 8, S, S, 256, False, D, persistent=False) == 0
+    # Three blocks on two CUs per XCD: a whole block and a half on each,
+    # instead of two whole ones on one of them.
+    assert fwd_split_makespan([40] * 3, 0, 8, 16, False) == 2 * 48
+    assert fwd_split_makespan([40] * 3, 1, 8, 16, False) == 48 + 20 + 1 + 8

@@ -768,13 +768,14 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   const int per_bh = p.kv_splits > 0 ? p.n_mblk * p.kv_splits : p.n_mblk + p.n_split;
   const int total = per_bh * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
-  set_item_order(p, per_bh, PG > 0 || D == 64 || (!p.dm.causal && p.n_split > 0));
+  const int cus = device_cu_count();
+  const bool fixed_lists = p.kv_splits == 0 && total < kFwdDynMinItemsPerWg * std::max(cus, 1);
+  set_item_order(p, per_bh, PG > 0 || D == 64 || (p.dm.causal ? fixed_lists : p.n_split > 0));
   p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;
   int grid = total;
   if (PG == 0 && D == 128) {
-    const int cus = device_cu_count();
     grid = cus > 0 ? std::min(total, cus) : total;
     p.n_wg = grid;
     // The dynamic schedule pays for its claims (atomic round trips of ~2 us,

@@ -22,10 +22,16 @@ namespace gqa {
 // * Paged, head_dim 128, 512 query tokens over [1700, 5262] keys: 82 / 71,
 //   short form 80 / 66; [600, 5000, 2000] with 400: 122 / 74; 4 x 17000 with
 //   382: 399 / 384.
-// * Contiguous head_dim 128: the persistent grid of gqa_fwd_kernel spreads its
-//   items itself and keeps the keys of fewer pairs in each L2: 4 x 1024 tokens
-//   42.8 / 44.6, 3 x 1800 58.3 / 60.6, so it stays with pair after pair.  The
-//   short form gains once its workgroups no longer start together: 4 x 300
+// * Contiguous head_dim 128, causal, fixed lists: sorted heavy first over all
+//   the XCD's pairs, the snake order hands every workgroup the same work;
+//   pair after pair, what met what was chance.  2 x 1300 tokens 42.3 / 35.9, 2
+//   x 3700 236 / 190, 3 x 900 39.7 / 29.6, 3 x 1800 109 / 84, 4 x 1300 91 / 66,
+//   6 x 1300 124 / 93, 2 x 4096 231 / 227.  With many items per workgroup
+//   (claimed as it goes), and key chunks: pair after pair, fewer pairs' keys
+//   in each L2.
+// * Without a mask only the split blocks need it (dispatch.py
+//   FWD_SPLIT_MAX_ROUNDS).
+// * The short form gains once its workgroups no longer start together: 4 x 300
 //   tokens (320 workgroups) 16.8 / 15.8, 8 x 300 over 16/4 heads 16.3 / 14.9;
 //   2 x 512 (256) 12.4 / 12.8.
 __device__ inline void item_of(const FwdParams& p, int w, int n_items, int& bh, int& idx) {

@@ -198,13 +198,15 @@ def _fwd_block_tiles(n_mblk: int, block_m: int, seq_q: int, seq_kv: int, causal:
 
 
 def fwd_split_makespan(tiles, n_split: int, n_bh: int, cu_count: int, causal: bool = True,
-                       persistent: bool = True) -> float:
+                       persistent: bool = True, dealt: bool = False) -> float:
     """Modelled run time (tile steps) of the single pass with the n_split
     heaviest blocks split: work items in the kernel's order (per (b, kv
     head): upper halves of the split blocks, then every block heavy-first
     with split blocks as their lower halves; not causal: unsplit blocks,
     then both halves of the last n_split), scheduled as _list_makespan
-    describes (`persistent`: the head_dim-128 kernel over contiguous K/V)."""
+    describes (`persistent`: the head_dim-128 kernel over contiguous K/V;
+    `dealt`: its pairs are dealt to the XCDs, which take theirs side by
+    side)."""
     n = len(tiles)
     order = list(range(n - 1, -1, -1)) if causal else list(range(n))
     mo = FWD_MERGE_OVERHEAD if persistent else 0
@@ -222,10 +224,11 @@ def fwd_split_makespan(tiles, n_split: int, n_bh: int, cu_count: int, causal: bo
     items = [tiles[n - 1 - i] - tiles[n - 1 - i] // 2 + mo for i in range(n_split)]
     for pid in order:
         items.append(tiles[pid] // 2 + mo if pid >= n - n_split else tiles[pid])
+    per_xcd = n_bh // 8 if dealt and n_bh % 8 == 0 else 1
     runs = []
     for c in items:
-        _push_run(runs, c + FWD_ITEM_OVERHEAD, 1)
-    return _list_makespan(runs, n_bh, cu_count, persistent)
+        _push_run(runs, c + FWD_ITEM_OVERHEAD, per_xcd)
+    return _list_makespan(runs, n_bh // per_xcd, cu_count, persistent)
 
 
 def _push_run(runs, cost, count: int) -> None:
@@ -400,14 +403,15 @@ def _fill_last_round(n_mblk: int, n_bh: int, seq_kv: int, cu_count: int, head_di
 
 
 def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int,
-                     cu_count: int, causal: bool, head_dim: int = 128, persistent: bool = None) -> int:
+                     cu_count: int, causal: bool, head_dim: int = 128, persistent: bool = None,
+                     dealt: bool = False) -> int:
     """Query blocks per (b, kv head) to run as two key halves (0: none).
 
     Under causal, when there are few workgroups per CU, the longest block
     sets the run time, and splitting the heaviest ones shortens it
     (fwd_split_makespan picks the count).  Not causal: FWD_SPLIT_MAX_ROUNDS.
-    `persistent` (default: head_dim 128) as fwd_split_makespan; False for
-    paged caches."""
+    `persistent` (default: head_dim 128) and `dealt` as fwd_split_makespan;
+    persistent False for paged caches."""
     group = num_heads // num_kv_heads
     block_m = max(1, FWD_ROWS // group)
     n_mblk = _cdiv(seq_q, block_m)
@@ -419,11 +423,11 @@ def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     if n_mblk < 2 or n_mblk * n_bh >= FWD_SPLIT_MAX_WG_PER_CU * cu_count:
         return 0
     tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
-    base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent)
+    base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent, dealt=dealt)
     best, best_ns = base, 0
-    for f in (0.25, 0.375, 0.5, 0.625, 0.75, 1.0):
+    for f in (0.1, 0.15, 0.2, 0.25, 0.375, 0.5, 0.625, 0.75, 1.0):
         ns = max(1, min(n_mblk, round(n_mblk * f)))
-        t = fwd_split_makespan(tiles, ns, n_bh, cu_count, persistent=persistent)
+        t = fwd_split_makespan(tiles, ns, n_bh, cu_count, persistent=persistent, dealt=dealt)
         if t < best:
             best, best_ns = t, ns
     return best_ns if best <= (1.0 - FWD_SPLIT_GAIN) * base else 0
@@ -564,7 +568,7 @@ def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv:
         longest = max(max(tiles[:n_mblk - fwd_split], default=0), _cdiv(max(tiles[n_mblk - fwd_split:], default=0), 2))
         lo, hi = OTHER_STEP_US["single"][head_dim]
         other = _step_us(lo, hi, sum(tiles) * n_bh, longest, cu_count) * fwd_split_makespan(
-            tiles, fwd_split, n_bh, cu_count, causal, persistent)
+            tiles, fwd_split, n_bh, cu_count, causal, persistent, dealt=persistent and causal and n_bh > 8)
     return short_us(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim) < other
 
 
@@ -584,12 +588,19 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
     * With one split per sequence the first pass writes the output itself
       (the flat split with one slot per sequence): B = 32 x 700 keys 19.5 ->
       17.6, B = 64 x 700 32.6 -> 30.5.
+    * The single pass at head_dim 128 deals several (b, kv head) pairs per XCD
+      side by side, which leaves less to split than choose_route's model of
+      pair after pair: 2 x 1536 tokens 54.3 -> 45.4 us, 4 x 768 36.3 -> 28.9.
     * Batches that no power-of-two split count spreads evenly over the
       compute units take the flat split (FLAT_MIN_USED)."""
     route = choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
     rows = num_heads // num_kv_heads * seq_q
     if rows <= 0 or seq_kv <= 0 or batch <= 0:
         return route
+    n_bh = batch * num_kv_heads
+    if route.kind == "single" and causal and head_dim == 128 and n_bh > 8 and n_bh % 8 == 0:
+        ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, True, dealt=True)
+        route = Route("single", 1, route.workgroups + (ns - route.fwd_split) * n_bh, ns)
     if rows > flat_max_rows(head_dim) and use_short(
             batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
             route.splits if route.kind == "chunks" else 0, route.fwd_split, head_dim == 128):

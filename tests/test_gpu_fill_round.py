@@ -55,3 +55,19 @@ def test_default_route_fills_the_last_round(B, S, D):
     assert_close(outs[0][:, :, rows], ref, BASELINE_TOL[torch.float16], f"{plan}")
     for o in outs[1:]:
         assert torch.equal(o, outs[0])
+
+
+@pytest.mark.parametrize("B,Hkv", [(2, 8), (3, 8), (8, 2), (3, 4)])
+@pytest.mark.parametrize("sq,skv", [(64, 64), (129, 200), (333, 333), (900, 900)])
+def test_dealt_fixed_lists(B, Hkv, sq, skv):
+    """Causal, head_dim 128: pairs dealt to the XCDs in the persistent
+    kernel's fixed lists (16 and 24 pairs; 12 not), with split blocks."""
+    from gqa_kernels.dispatch import single_pass_forward
+    q, k, v = make_inputs(B, 4 * Hkv, Hkv, sq, skv, 128, torch.bfloat16, seed=B * 5 + sq, device=DEV)
+    ref = oracle(q, k, v)
+    n = -(-sq // 64)
+    for ns in sorted({0, 1, n // 2, n}):
+        print(f"dealt B={B} Hkv={Hkv} {sq}x{skv} split={ns}", flush=True)
+        o, _ = single_pass_forward(q, k, v, torch.empty_like(q), True, ns, True)
+        torch.cuda.synchronize()
+        assert_close(o, ref, BASELINE_TOL[torch.bfloat16], f"split={ns}")

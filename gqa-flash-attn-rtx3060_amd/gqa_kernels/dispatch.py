@@ -112,6 +112,15 @@ SHORT_SPLIT_KEYS = {128: 160.0, 64: 220.0}
 # taken when the modelled run time drops by at least FWD_SPLIT_GAIN.
 FWD_SPLIT_MAX_WG_PER_CU = 2
 FWD_SPLIT_GAIN = 0.05
+# head_dim 64 under causal, contiguous, more blocks than CUs and at most this
+# many per CU: the heaviest of each (b, kv head), eight an XCD in all, are
+# split.  Two workgroups share a CU there, so nearly all start together and
+# the heaviest, which the model above deals one to a CU, ends last, alone on
+# its CU.  Measured, us, whole / split: 2500 tokens 44.1 / 37.8, 3000 55.7 /
+# 47.6, 4096 86.3 / 78.0, 4700 107.5 / 97.0, 2 x 1700 37.8 / 33.5, 2 x 2500 63.9
+# / 60.0, 4 x 900 26.7 / 23.1, 1300 of 64 heads 28.2 / 23.8; past the line, 4 x
+# 1300 38.0 / 39.0, 3 x 2200 68.2 / 67.3, 4096 of 64 heads 136.0 / 138.3.
+FWD_HEAD_MAX_WG_PER_CU = 2.5
 # Per-work-item overhead of the single-pass kernel (first loads in flight,
 # output, and for split blocks the exchange of the fp32 partial state), in
 # 64-key tile steps, for the run-time model.  Calibrated on MI355X against
@@ -420,6 +429,8 @@ def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
         return _fill_last_round(n_mblk, n_bh, seq_kv, cu_count, head_dim) if persistent is None else 0
     if persistent is None:
         persistent = head_dim == 128
+        if not persistent and cu_count < n_mblk * n_bh <= FWD_HEAD_MAX_WG_PER_CU * cu_count:
+            return min(n_mblk, max(1, round(cu_count / 4 / n_bh)))
     if n_mblk < 2 or n_mblk * n_bh >= FWD_SPLIT_MAX_WG_PER_CU * cu_count:
         return 0
     tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)

@@ -71,3 +71,16 @@ def test_dealt_fixed_lists(B, Hkv, sq, skv):
         o, _ = single_pass_forward(q, k, v, torch.empty_like(q), True, ns, True)
         torch.cuda.synchronize()
         assert_close(o, ref, BASELINE_TOL[torch.bfloat16], f"split={ns}")
+
+
+@pytest.mark.parametrize("B,S", [(1, 2500), (2, 1700)])
+def test_head_dim_64_heaviest_blocks_split(B, S):
+    from gqa_kernels import gqa_flash_attn
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    plan = choose_plan(B, 32, 8, S, S, _cu_count(0), True, 64)
+    assert plan.kind == "single" and (plan.fwd_split > 0 or _cu_count(0) != 256)
+    q, k, v = make_inputs(B, 32, 8, S, S, 64, torch.float16, seed=S, device=DEV)
+    print(f"B={B} S={S} {plan}", flush=True)
+    o = gqa_flash_attn(q, k, v)
+    torch.cuda.synchronize()
+    assert_close(o, oracle(q, k, v), BASELINE_TOL[torch.float16], f"{plan}")

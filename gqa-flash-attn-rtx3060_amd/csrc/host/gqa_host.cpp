@@ -346,9 +346,9 @@ py::object flash_attn(const py::handle& hq, const py::handle& hk, const py::hand
     need = gqa_split_flat_workspace_bytes(B, Hq, Sq, D, p.n);
   else if (p.kind == kSingle)
     need = gqa_fwd_split_workspace_bytes(B, Hkv, D, p.n);
-  if (need > 0 && (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr) return py::none();
+  // (A captured call gets partials and counters of its own, in Python.)
+  if (need > 0 && (capturing() || (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr)) return py::none();
   if (p.kind == kSingle || p.kind == kChunks) {
-    // (A captured call gets counters of its own.)
     const size_t n = gqa_fwd_split_counters_count(B, Hkv, p.kind == kSingle ? p.n : 0);
     if (capturing() || (cnt = stream_buffer(counters, dev, stream, n * sizeof(int))) == nullptr) return py::none();
   }
@@ -446,7 +446,8 @@ py::object paged_attn(const py::handle& hq, const py::handle& hkc, const py::han
     need = gqa_split_flat_workspace_bytes(B, H, Sq, D, p.n);
   else if (p.kind == kSingle)
     need = gqa_fwd_split_workspace_bytes(B, Hkv, D, p.n);
-  if (need > 0 && (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr) return py::none();
+  // (A captured call gets partials and counters of its own, in Python.)
+  if (need > 0 && (capturing() || (ws = stream_buffer(workspaces, dev, stream, need)) == nullptr)) return py::none();
   if (p.kind == kSingle && p.n > 0) {
     const size_t n = gqa_fwd_split_counters_count(B, Hkv, p.n);
     if (capturing() || (cnt = stream_buffer(counters, dev, stream, n * sizeof(int))) == nullptr) return py::none();

@@ -759,8 +759,8 @@ def single_pass_forward(q, k, v, o, causal, fwd_split=0, return_lse=False):
     """Launch the single-pass kernel on kernel-ready q, k, v and output o
     through gqa_fwd_split_launch: with fwd_split > 0 the heaviest query
     blocks run as two key halves, and the work items are scheduled across
-    the XCDs dynamically (workspace and counters are the stream's cached
-    buffers)."""
+    the XCDs dynamically (workspace and counters: _workspace_buffer,
+    _counter_buffer)."""
     lib = _lib.load()
     batch, num_heads, seq_q, head_dim = q.shape
     _, num_kv_heads, seq_kv, _ = k.shape
@@ -801,8 +801,8 @@ def chunks_forward(q, k, v, o, causal, kv_splits, return_lse=False):
     """Launch the single pass over key chunks on kernel-ready q, k, v and
     output o through gqa_fwd_chunks_launch: every query block runs as
     kv_splits work items over consecutive key ranges, each writing fp32
-    partials into the stream's cached split workspace, which the split-KV
-    combine reduces into o (and lse)."""
+    partials into the split workspace, which the split-KV combine reduces
+    into o (and lse)."""
     lib = _lib.load()
     batch, num_heads, seq_q, head_dim = q.shape
     _, num_kv_heads, seq_kv, _ = k.shape

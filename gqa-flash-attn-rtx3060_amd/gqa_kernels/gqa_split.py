@@ -32,8 +32,8 @@ _counters_lock = threading.Lock()
 # allocator would hand out the same memory anyway; keeping it saves the
 # allocation on every decode step.)
 _workspaces: dict = {}
-# Buffers replaced by a larger one.  A CUDA/HIP graph captured while a buffer
-# was current keeps its raw address and writes to it on every replay, so a
+# Buffers replaced by a larger one.  Another thread that uses the same stream
+# may have taken a buffer's address for a call it has yet to launch, so a
 # superseded buffer is never released: it stays here for the life of the
 # process.  Each replacement at least doubles the size, so everything kept is
 # less than the current buffer again.
@@ -52,14 +52,27 @@ def stream_handle(device: torch.device) -> int:
     return _raw_stream(torch.cuda.current_device() if device.index is None else device.index)
 
 
+def _capturing(device: torch.device) -> bool:
+    return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 def _workspace_buffer(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
+    """fp32 buffer of at least `nbytes` bytes for the partials of one call.
+
+    Eager calls share the stream's: they run one after another.  A call being
+    captured gets a tensor of its own, from the graph's memory pool (which
+    holds it as long as the graph): graphs captured on one stream may be
+    replayed at the same time on several, and two calls in one buffer would
+    merge each other's partials."""
+    if _capturing(device):
+        return torch.empty(max(-(-nbytes // 4), 1), dtype=torch.float32, device=device)
     key = (device.index, stream)
     with _counters_lock:
         buf = _workspaces.get(key)
         if buf is None or buf.numel() * 4 < nbytes:
             n = max(-(-nbytes // 4), 1 << 16)
             if buf is not None:
-                _retired.append(buf)  # a captured graph may still write to it
+                _retired.append(buf)
                 n = max(n, 2 * buf.numel())
             buf = torch.empty(n, dtype=torch.float32, device=device)
             _workspaces[key] = buf
@@ -74,7 +87,7 @@ _captured: list = []
 
 
 def _counter_buffer(device: torch.device, stream: int, n: int) -> torch.Tensor:
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing(device):
         # Zeroed by a fill kernel recorded in the graph (not a memset node),
         # so every replay also starts from zero counters.
         buf = torch.zeros(max(n, 1), dtype=torch.int32, device=device)
@@ -87,7 +100,7 @@ def _counter_buffer(device: torch.device, stream: int, n: int) -> torch.Tensor:
         if buf is None or buf.numel() < n:
             m = max(n, 1024)
             if buf is not None:
-                _retired.append(buf)  # a captured graph may still count in it
+                _retired.append(buf)
                 m = max(m, 2 * buf.numel())
             buf = torch.zeros(m, dtype=torch.int32, device=device)
             _counters[key] = buf
@@ -158,16 +171,13 @@ def _split_launch_ctypes(q, k, v, ws, splits, causal, scale_log2, return_lse, st
 
 def decode_forward(q, k, v, causal, splits, return_lse, dev):
     """The two-launch split-KV forward as gqa_flash_attn takes it: kernel-ready
-    q, k, v on device index `dev` (the current device), the stream's cached
-    workspace.  Computes exactly what split_kv_forward(q, k, v, causal,
+    q, k, v on device index `dev` (the current device), the workspace of
+    _workspace_buffer.  Computes exactly what split_kv_forward(q, k, v, causal,
     splits, return_lse=return_lse) does, with the host work of a decode step
     kept to one pass over the arguments (every value read once)."""
     batch, num_heads, seq_q, head_dim = q.shape
     stream = _raw_stream(dev) if _raw_stream is not None else torch.cuda.current_stream(dev).cuda_stream
-    need = batch * num_heads * seq_q * splits * (head_dim + 2) * 4
-    ws = _workspaces.get((dev, stream))
-    if ws is None or ws.numel() * 4 < need:
-        ws = _workspace_buffer(q.device, stream, need)
+    ws = _workspace_buffer(q.device, stream, workspace_bytes(batch, num_heads, seq_q, head_dim, splits))
     # gqa_split_launch through the torch-tensor binding (_gqa_host.so): the
     # argument marshalling of a decode step in C++ rather than ctypes.
     host = _lib._host if _lib._host is not None else _decode_host()
@@ -183,10 +193,7 @@ def flat_forward(q, k, v, causal, slots, return_lse, dev):
     (GQA_E_FLAT: more packed rows, or strides past its 32-bit offsets)."""
     batch, num_heads, seq_q, head_dim = q.shape
     stream = stream_handle(q.device)
-    need = flat_workspace_bytes(batch, num_heads, seq_q, head_dim, slots)
-    ws = _workspaces.get((dev, stream))
-    if ws is None or ws.numel() * 4 < need:
-        ws = _workspace_buffer(q.device, stream, need)
+    ws = _workspace_buffer(q.device, stream, flat_workspace_bytes(batch, num_heads, seq_q, head_dim, slots))
     host = _lib._host if _lib._host is not None else _decode_host()
     if host is not None:
         return host.split_flat(q, k, v, ws, slots, bool(causal), _SCALE_LOG2[head_dim], _DTYPES[q.dtype],
@@ -214,8 +221,8 @@ def split_kv_forward(q, k, v, causal, splits, workspace=None, fused=False, retur
     (B, Hq, Sq), computed by the combine; the result is then ``(o, lse)``.
 
     ``workspace`` may be a caller-provided fp32 CUDA tensor with at least
-    ``workspace_bytes(...) / 4`` elements; otherwise the stream's cached
-    workspace is used (grown when too small).
+    ``workspace_bytes(...) / 4`` elements; otherwise that of
+    _workspace_buffer is used.
     """
     lib = _lib.load()
     batch, num_heads, seq_q, head_dim = q.shape

@@ -171,6 +171,67 @@ def test_two_graphs_replayed_concurrently(shape):
             assert torch.equal(out, e), f"replay {rep} of graph {i} differs from the eager result"
 
 
+# Calls whose routes write partials: split-KV, flat split over five
+# sequences, key chunks, split blocks (with and without a mask, head_dim 64),
+# paged flat split and paged split blocks.
+_WORKSPACE_CALLS = [
+    ("contiguous", (1, 32, 8, 1, 700, 128, True)), ("contiguous", (16, 32, 8, 1, 700, 128, True)),
+    ("contiguous", (5, 32, 8, 1, 8192, 128, True)), ("contiguous", (1, 32, 8, 64, 8192, 128, True)),
+    ("contiguous", (2, 32, 8, 1025, 1025, 128, True)), ("contiguous", (4, 32, 8, 1025, 1025, 128, False)),
+    ("contiguous", (1, 32, 8, 3000, 3000, 64, True)),
+    ("paged", ([3000, 700, 1500], 1, {})), ("paged", ([3000, 1200], 256, dict(route="single", splits=4)))]
+
+
+def _workspace_call(kind, spec, seed):
+    from gqa_kernels import gqa_flash_attn
+    from gqa_kernels.paged import paged_attention
+    if kind == "contiguous":
+        *shape, causal = spec
+        q, k, v = make_inputs(*shape, torch.bfloat16, seed=seed, device=DEV)
+        return lambda: gqa_flash_attn(q, k, v, causal=causal)
+    lens, sq, kw = spec
+    cache, g0 = _paged_cache(lens, 16, seed)
+    q = torch.randn(len(lens), 32, sq, 128, generator=g0).to(torch.bfloat16).to(DEV)
+    table, seq_lens = cache.block_table(range(len(lens))), cache.seq_lens(range(len(lens)))
+    return lambda: paged_attention(q, cache.k_cache, cache.v_cache, table, seq_lens, True, max_seq_len=max(lens), **kw)
+
+
+@pytest.mark.parametrize("kind,spec", _WORKSPACE_CALLS)
+def test_captured_partials_are_the_graphs_own(kind, spec):
+    """A replay leaves the capture stream's workspace alone, and two graphs
+    captured on one stream and replayed at the same time on two do not meet
+    in one buffer."""
+    from gqa_kernels import gqa_split
+    print(f"own partials {kind} {spec}", flush=True)
+    calls = [_workspace_call(kind, spec, seed) for seed in (1, 2)]
+    s = torch.cuda.Stream()
+    graphs = []
+    for fn in calls:
+        with torch.cuda.stream(s):
+            expect = fn().clone()
+            fn()  # a planned shape
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = fn()
+        graphs.append((g, out, expect))
+    shared = gqa_split._workspaces[(torch.cuda.current_device(), s.cuda_stream)]
+    shared.fill_(float("nan"))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for rep in range(4):
+        torch.cuda.synchronize()
+        for (g, out, _), st in zip(graphs, streams):
+            out.zero_()
+        torch.cuda.synchronize()
+        for (g, _, _), st in zip(graphs, streams):
+            with torch.cuda.stream(st):
+                g.replay()
+        torch.cuda.synchronize()
+        for i, (_, out, expect) in enumerate(graphs):
+            assert torch.equal(out, expect), f"replay {rep} of graph {i} differs from the eager result"
+    assert bool(torch.isnan(shared).all()), "a replay wrote into the stream's workspace"
+
+
 def _paged_cache(lens, bs, seed):
     from gqa_kernels.paged import PagedKVCache
     g0 = torch.Generator().manual_seed(seed)

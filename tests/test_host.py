@@ -117,6 +117,22 @@ def test_decode_falls_back_to_ctypes_without_host_binding(monkeypatch):
     assert len(gqa_split._host_failed) == 1
 
 
+def test_captured_calls_get_partials_of_their_own(monkeypatch):
+    """Graphs captured on one stream may be replayed at the same time on
+    several: a call made under capture takes neither the stream's workspace
+    nor another captured call's."""
+    from gqa_kernels import gqa_split
+    monkeypatch.setattr(gqa_split, "_workspaces", {})
+    dev = torch.device("cpu")
+    eager = gqa_split._workspace_buffer(dev, 7, 1 << 20)
+    assert gqa_split._workspace_buffer(dev, 7, 1 << 10) is eager
+    monkeypatch.setattr(gqa_split, "_capturing", lambda device: True, raising=False)
+    captured = [gqa_split._workspace_buffer(dev, 7, 1 << 10) for _ in range(2)]
+    assert len({t.data_ptr() for t in captured + [eager]}) == 3
+    assert all(t.numel() * 4 >= 1 << 10 for t in captured)
+    assert gqa_split._workspaces == {(dev.index, 7): eager}
+
+
 def test_workspace_bytes(lib):
     from gqa_kernels.gqa_split import workspace_bytes
     for args in ((1, 32, 1, 128, 128), (16, 64, 4, 128, 8), (2, 8, 3, 64, 7)):

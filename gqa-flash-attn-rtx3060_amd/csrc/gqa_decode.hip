@@ -42,6 +42,7 @@
 #include <type_traits>
 
 #include "gqa_common.hpp"
+#include "gqa_flat.hpp"
 #include "gqa_lds.hpp"
 #include "gqa_params.hpp"
 
@@ -243,113 +244,40 @@ __device__ inline int wave_scan(int n) {
   return n;
 }
 
-// The pieces of one slot of a flat split (SplitParams::slots): ranges of
-// consecutive tile steps ("units" of TK keys) of one sequence each, in order.
-// The slot's range is [j * T / slots, (j + 1) * T / slots) of the T units of
-// all sequences (with fewer units than slots, unit j alone, so that no slot
-// between two pieces of a sequence is empty); every value is wave-uniform except a lane's own sequence in
-// the scans (each wave works the ranges out for itself: the lengths live on
-// the device).
-template <int TK, bool PAGED> struct FlatWalk {
-  int at, end;      // units of the flat order still to do
-  int b, u0, n;     // current sequence, its first unit in the flat order, its units
-  int base, carry;  // paged: first sequence of the scanned group of 64, units before it
-  int incl, own;    // paged, per lane: scan over the group, this lane's sequence's units
-  int len, skv;     // ... and keys; keys of the current sequence
+// The wave as the flat split's walk sees it (gqa_flat.hpp): units of TK keys.
+template <int TK> struct FlatWave {
+  using Lanes = int;
+  const SplitParams& p;
+  int lane, B, slots, seq_units;
 
-  // Units of sequence `s` (per lane): none without query rows.
-  __device__ static int units(const SplitParams& p, int s, int& len) {
-    len = 0;
-    if (s >= p.dm.B) return 0;
-    len = min(max(p.seq_lens[s], 0), p.dm.Skv);
-    return p.q_len != nullptr && p.q_len[s] <= 0 ? 0 : (len + TK - 1) / TK;
+  __device__ FlatWave(const SplitParams& p, int lane)
+      : p(p), lane(lane), B(p.dm.B), slots(p.slots), seq_units((p.dm.Skv + TK - 1) / TK) {}
+  // (None without query rows.)
+  __device__ int units(int base, int& keys) const {
+    const int s = base + lane;
+    keys = 0;
+    if (s >= B) return 0;
+    keys = min(max(p.seq_lens[s], 0), p.dm.Skv);
+    return p.q_len != nullptr && p.q_len[s] <= 0 ? 0 : (keys + TK - 1) / TK;
   }
-  __device__ static int units(const SplitParams& p, int s) {
-    int l;
-    return units(p, s, l);
+  __device__ static int scan(int n) { return wave_scan(n); }
+  __device__ static int read(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+  __device__ static int first_above(int v, int x) {
+    return __builtin_ffsll((long long)__builtin_amdgcn_ballot_w64(v > x)) - 1;
   }
-  __device__ void scan(const SplitParams& p, int lane) {
-    own = units(p, base + lane, len);
-    incl = wave_scan(own);
-  }
-  __device__ static int last(int v) { return __builtin_amdgcn_readlane(v, 63); }
-
-  __device__ void start(const SplitParams& p, int slot, int lane) {
-    int total = 0;
-    if constexpr (PAGED) {
-      for (int g0 = p.dm.B > 64 ? 64 : p.dm.B; g0 < p.dm.B; g0 += 64) total += last(wave_scan(units(p, g0 + lane)));
-      base = 0;
-      carry = 0;
-      scan(p, lane);
-      total += last(incl);
-    } else {
-      n = (p.dm.Skv + TK - 1) / TK;
-      total = n * p.dm.B;
-    }
-    if (total < p.slots) {
-      at = min(slot, total);
-      end = min(slot + 1, total);
-    } else {
-      at = fast_div(slot * total, p.div_splits.mul, p.div_splits.shift);
-      end = fast_div((slot + 1) * total, p.div_splits.mul, p.div_splits.shift);
-    }
-    if constexpr (PAGED) {
-      b = 0;
-      u0 = 0;
-      n = 0;
-    } else if (at < end) {
-      b = fast_div(at, p.div_units.mul, p.div_units.shift);
-      u0 = b * n;
-    }
-  }
-
-  // Paged: (first partial, number of partials) of every sequence for the
-  // combine, by one wave: unit t lies in slot ((t + 1) * slots - 1) / T.
-  // (Contiguous sequences are equally long: the combine works it out.)
-  __device__ static void plan(const SplitParams& p, int lane) {
-    int total = 0, before = 0;
-    for (int g0 = 0; g0 < p.dm.B; g0 += 64) total += last(wave_scan(units(p, g0 + lane)));
-    const int slots = min(p.slots, total);
-    for (int g0 = 0; g0 < p.dm.B; g0 += 64) {
-      const int s = g0 + lane, mine = units(p, s);
-      const int upto = wave_scan(mine) + before;
-      before = last(upto);
-      if (s < p.dm.B) {
-        int first = 0, count = 0;
-        if (mine > 0) {
-          first = ((upto - mine + 1) * slots - 1) / total;
-          count = (upto * slots - 1) / total - first + 1;
-        }
-        p.plan[2 * s] = first + s;
-        p.plan[2 * s + 1] = count;
-      }
-    }
-  }
-
-  // The next piece: units [from, from + cnt) of sequence b.
-  __device__ bool next(const SplitParams& p, int lane, int& from, int& cnt) {
-    if (at >= end) return false;
-    if constexpr (PAGED) {
-      while (at >= carry + last(incl)) {  // (ends: at < T)
-        carry += last(incl);
-        base += 64;
-        scan(p, lane);
-      }
-      const int l = __builtin_ffsll((long long)__builtin_amdgcn_ballot_w64(carry + incl > at)) - 1;
-      b = base + l;
-      n = __builtin_amdgcn_readlane(own, l);
-      skv = __builtin_amdgcn_readlane(len, l);
-      u0 = carry + __builtin_amdgcn_readlane(incl, l) - n;
-    } else if (at >= u0 + n) {
-      ++b;
-      u0 += n;
-    }
-    from = at - u0;
-    cnt = min(end, u0 + n) - at;
-    at += cnt;
-    return true;
-  }
+  __device__ int share(int n) const { return fast_div(n, p.div_splits.mul, p.div_splits.shift); }
+  __device__ int sequence(int n) const { return fast_div(n, p.div_units.mul, p.div_units.shift); }
+  __device__ static int own(int v, int) { return v; }
+  template <typename F> __device__ void each(F f) const { f(lane); }
 };
+
+// The combine's plan, by one wave.
+template <class W> __device__ inline void write_plan(const SplitParams& p, const W& w) {
+  FlatWalk<W, true>::plan(w, [&](int s, int first, int count) {
+    p.plan[2 * s] = first;
+    p.plan[2 * s + 1] = count;
+  });
+}
 
 }  // namespace
 
@@ -425,16 +353,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int head = kvh * dm.G + g;
   const int pos_lo = fast_div(wr0, p.div_g.mul, p.div_g.shift);
   const int pos_end = fast_div(wr0 + 32 * RW - 1, p.div_g.mul, p.div_g.shift);
-  FlatWalk<64, PAGED> walk;
+  const FlatWave<64> flat_wave(p, lane);
+  FlatWalk<FlatWave<64>, PAGED> walk;
   bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
-  if constexpr (flat) walk.start(p, s, lane);
+  if constexpr (flat) walk.start(flat_wave, s);
   // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
   for (;;) {
   int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
   if constexpr (flat) {
     int from, cnt;
-    if (!walk.next(p, lane, from, cnt)) {
-      if (plan_due) walk.plan(p, lane);  // (no sequence has keys)
+    if (!walk.next(flat_wave, from, cnt)) {
+      if (plan_due) write_plan(p, flat_wave);  // (no sequence has keys)
       return;
     }
     b = walk.b;
@@ -586,7 +515,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   issue(1, lds_c_k1, lds_d_v1);
   // (While the first piece's loads are in flight.)
-  if (plan_due) walk.plan(p, lane);
+  if (plan_due) write_plan(p, flat_wave);
   plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).  Waiting here,
   // explicitly, also settles Q for the compiler: otherwise it waits for
@@ -933,16 +862,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // This lane's query row (position-major packing).
   const int pos = fast_div(i16, p.div_g.mul, p.div_g.shift), g = i16 - pos * dm.G;
   const int head = kvh * dm.G + g;
-  FlatWalk<TK, PAGED> walk;
+  const FlatWave<TK> flat_wave(p, lane);
+  FlatWalk<FlatWave<TK>, PAGED> walk;
   bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
-  if constexpr (flat) walk.start(p, s, lane);
+  if constexpr (flat) walk.start(flat_wave, s);
   // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
   for (;;) {
   int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
   if constexpr (flat) {
     int from, cnt;
-    if (!walk.next(p, lane, from, cnt)) {
-      if (plan_due) walk.plan(p, lane);  // (no sequence has keys)
+    if (!walk.next(flat_wave, from, cnt)) {
+      if (plan_due) write_plan(p, flat_wave);  // (no sequence has keys)
       return;
     }
     b = walk.b;
@@ -1073,7 +1003,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   issue(1, lds_c_k1, lds_d_v1);
   // (While the first piece's loads are in flight.)
-  if (plan_due) walk.plan(p, lane);
+  if (plan_due) write_plan(p, flat_wave);
   plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * NI * NSUB));

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -131,6 +132,21 @@ def test_captured_calls_get_partials_of_their_own(monkeypatch):
     assert len({t.data_ptr() for t in captured + [eager]}) == 3
     assert all(t.numel() * 4 >= 1 << 10 for t in captured)
     assert gqa_split._workspaces == {(dev.index, 7): eager}
+
+
+def test_flat_walk_on_the_cpu(tmp_path):
+    """The flat split's walk and plan (gqa_flat.hpp), compiled for the CPU,
+    against a count of the units; with lengths that change while they are
+    read (another stream rewriting seq_lens under a running kernel) every walk
+    ends and no partial lies outside the workspace."""
+    exe = tmp_path / "flat_walk"
+    tests = REPO / "tests"
+    csrc = REPO / "gqa-flash-attn-rtx3060_amd" / "csrc"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-ftrapv", "-D_GLIBCXX_ASSERTIONS", f"-I{csrc}",
+                    str(tests / "flat_walk_host.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.split() == ["150", "batches"]
 
 
 def test_workspace_bytes(lib):

@@ -112,15 +112,24 @@ SHORT_SPLIT_KEYS = {128: 160.0, 64: 220.0}
 # taken when the modelled run time drops by at least FWD_SPLIT_GAIN.
 FWD_SPLIT_MAX_WG_PER_CU = 2
 FWD_SPLIT_GAIN = 0.05
-# head_dim 64 under causal, contiguous, more blocks than CUs and at most this
-# many per CU: the heaviest of each (b, kv head), eight an XCD in all, are
-# split.  Two workgroups share a CU there, so nearly all start together and
-# the heaviest, which the model above deals one to a CU, ends last, alone on
-# its CU.  Measured, us, whole / split: 2500 tokens 44.1 / 37.8, 3000 55.7 /
-# 47.6, 4096 86.3 / 78.0, 4700 107.5 / 97.0, 2 x 1700 37.8 / 33.5, 2 x 2500 63.9
-# / 60.0, 4 x 900 26.7 / 23.1, 1300 of 64 heads 28.2 / 23.8; past the line, 4 x
-# 1300 38.0 / 39.0, 3 x 2200 68.2 / 67.3, 4096 of 64 heads 136.0 / 138.3.
-FWD_HEAD_MAX_WG_PER_CU = 2.5
+# head_dim 64 under causal, contiguous, more blocks than CUs, where the model
+# splits nothing: two workgroups share a CU there, so nearly all start
+# together and the heaviest block, which the model deals one to a CU, ends
+# last, alone on its CU.  Prompts have the heaviest of each (b, kv head) split,
+# eight an XCD in all, for at most HEAD_PAIRS (b, kv head) pairs per XCD and
+# blocks per CU; the blocks of a chunk over a long cache are nearly as long as
+# each other and only get shorter waits, so the cache is at most HEAD_KV times
+# the chunk (more with few blocks).  Measured, us, whole / split, (b, kv head)
+# pairs x blocks: 8 x 35 2200 tokens 43.0 / 36.2, over 4400 keys 91.7 / 79.7;
+# 8 x 64 4096 tokens 91.0 / 82.7, over 5120 keys 124.5 / 116.1, 8192 222 / 226,
+# 16384 482 / 521; 8 x 79 5000 tokens 123.5 / 114.9; 16 x 18 1100 tokens 26.3 /
+# 23.5; 16 x 40 2500 tokens 67.5 / 64.5; 32 x 15 900 tokens 28.3 / 26.6, over
+# 1350 keys 43.1 / 44.5; 32 x 19 1200 tokens 38.3 / 39.1; 64 x 5 300 tokens 14.3
+# / 16.2; 128 x 4 256 tokens 16.8 / 21.3; 512 x 1 64 tokens 16.2 / 26.2.  Where
+# the model splits, its count: 12 x 29 1800 tokens 51.4 / 37.0 (5 blocks 46.2),
+# 8 x 47 3000 tokens over 12000 keys 305 / 263 (8 blocks 299).
+FWD_HEAD_PAIRS = ((2, 2.5), (4, 2.0))
+FWD_HEAD_KV = ((1.5, 2.0), (2.5, 1.25))
 # Per-work-item overhead of the single-pass kernel (first loads in flight,
 # output, and for split blocks the exchange of the fp32 partial state), in
 # 64-key tile steps, for the run-time model.  Calibrated on MI355X against
@@ -427,21 +436,32 @@ def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     n_bh = batch * num_kv_heads
     if not causal:
         return _fill_last_round(n_mblk, n_bh, seq_kv, cu_count, head_dim) if persistent is None else 0
+    if n_mblk < 2:
+        return 0
+    whole = persistent is None and head_dim == 64  # two workgroups per CU, contiguous
     if persistent is None:
         persistent = head_dim == 128
-        if not persistent and cu_count < n_mblk * n_bh <= FWD_HEAD_MAX_WG_PER_CU * cu_count:
-            return min(n_mblk, max(1, round(cu_count / 4 / n_bh)))
-    if n_mblk < 2 or n_mblk * n_bh >= FWD_SPLIT_MAX_WG_PER_CU * cu_count:
-        return 0
-    tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
-    base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent, dealt=dealt)
-    best, best_ns = base, 0
-    for f in (0.1, 0.15, 0.2, 0.25, 0.375, 0.5, 0.625, 0.75, 1.0):
-        ns = max(1, min(n_mblk, round(n_mblk * f)))
-        t = fwd_split_makespan(tiles, ns, n_bh, cu_count, persistent=persistent, dealt=dealt)
-        if t < best:
-            best, best_ns = t, ns
-    return best_ns if best <= (1.0 - FWD_SPLIT_GAIN) * base else 0
+    if n_mblk * n_bh < FWD_SPLIT_MAX_WG_PER_CU * cu_count:
+        tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
+        base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent, dealt=dealt)
+        best, best_ns = base, 0
+        for f in (0.1, 0.15, 0.2, 0.25, 0.375, 0.5, 0.625, 0.75, 1.0):
+            ns = max(1, min(n_mblk, round(n_mblk * f)))
+            t = fwd_split_makespan(tiles, ns, n_bh, cu_count, persistent=persistent, dealt=dealt)
+            if t < best:
+                best, best_ns = t, ns
+        if best <= (1.0 - FWD_SPLIT_GAIN) * base:
+            return best_ns
+    if whole and cu_count >= 8 and _split_head(n_mblk * n_bh / cu_count, n_bh / 8, seq_kv / seq_q):
+        return min(n_mblk, max(1, round(cu_count / 4 / n_bh)))
+    return 0
+
+
+def _split_head(per_cu: float, pairs: float, kv_ratio: float) -> bool:
+    """FWD_HEAD_PAIRS, FWD_HEAD_KV: blocks per CU, (b, kv head) pairs per XCD,
+    keys per query."""
+    return (per_cu > 1 and any(pairs <= p and per_cu <= c for p, c in FWD_HEAD_PAIRS)
+            and any(per_cu <= c and kv_ratio <= k for c, k in FWD_HEAD_KV))
 
 
 def split_rows_per_workgroup(rows: int, head_dim: int = 128) -> int:

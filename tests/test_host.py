@@ -482,6 +482,22 @@ def test_fwd_split_measured_choices():
         assert choose_route(1, 8, 2, 1024, 1024, 256, True, D).kind == "single"
 
 
+@pytest.mark.parametrize("batch,seq_q,seq_kv,split", [
+    (64, 64, 64, 0), (64, 64, 4096, 0),      # one block per (b, kv head)
+    (32, 128, 128, 0), (40, 100, 100, 0),    # two
+    (16, 256, 256, 0), (8, 300, 300, 0),     # many pairs: eight blocks an XCD are most of the call
+    (1, 4096, 16384, 0), (4, 900, 8000, 0),  # a chunk over a long cache: blocks of nearly one length
+    (8, 512, 4096, 0), (4, 1200, 1200, 0),
+    (1, 4096, 4096, 8), (2, 2500, 2500, 4), (4, 900, 900, 2), (1, 2200, 4400, 8),  # measured faster split
+    (1, 3000, 12000, 47),                    # the model's count comes first
+])
+def test_head_split_at_head_dim_64(batch, seq_q, seq_kv, split):
+    from gqa_kernels.dispatch import choose_fwd_split, choose_plan
+    assert choose_fwd_split(batch, 32, 8, seq_q, seq_kv, 256, True, 64) == split
+    plan = choose_plan(batch, 32, 8, seq_q, seq_kv, 256, True, 64)
+    assert plan.kind != "single" or plan.fwd_split == split
+
+
 def test_fwd_split_launch_validation(lib):
     f = lib.gqa_fwd_split_launch
     args = lambda lse, ws, cnt, ns: (_FAKE, _S4, _FAKE, _S4, _FAKE, _S4, _FAKE, _S4, lse, ws, cnt, ns,

@@ -106,7 +106,9 @@ OTHER_STEP_US = {"single": {128: (1.25, 1.65), 64: (1.0, 1.0)}, "chunks": {128: 
 # 12.5 / 13.1, 1000 16.5 / 13.9; B = 16 1500 23.9 / 29.6, 3000 43.0 / 45.9;
 # head_dim 64, 8 tokens, B = 1 600 9.1 / 10.2, 1000 12.1 / 10.3; B = 4 1000
 # 12.1 / 12.5; B = 16 3000 28.1 / 30.6.
-SHORT_SPLIT_KEYS = {128: 160.0, 64: 220.0}
+# Paged at head_dim 64 a step waits for more table reads: 8 x 7 tokens over
+# 1484 keys (50 workgroups) 19.8 / 15.9.
+SHORT_SPLIT_KEYS = {(128, False): 160.0, (128, True): 160.0, (64, False): 220.0, (64, True): 187.0}
 # Single pass with key-range split of the heaviest causal query blocks: only
 # considered while there are fewer than this many workgroups per CU, and
 # taken when the modelled run time drops by at least FWD_SPLIT_GAIN.
@@ -575,11 +577,11 @@ def short_us(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: 
 
 
 def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int, cu_count: int,
-              causal: bool, head_dim: int, kv_chunks: int, fwd_split: int, persistent: bool) -> bool:
+              causal: bool, head_dim: int, kv_chunks: int, fwd_split: int, paged: bool = False) -> bool:
     """Whether the short form beats the route it would replace: the split-KV
     pass for at most split_max_rows(head_dim) packed rows per kv head, else
     the single pass with `fwd_split` split blocks, or over `kv_chunks` key
-    chunks (`persistent` as chunks_makespan)."""
+    chunks."""
     group = num_heads // num_kv_heads
     if group > SHORT_ROWS or seq_q <= 0 or batch <= 0:
         return False
@@ -587,10 +589,11 @@ def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv:
     if wgs > SHORT_MAX_WG_PER_CU * cu_count:
         return False
     if group * seq_q <= split_max_rows(head_dim):
-        return seq_kv <= SHORT_SPLIT_KEYS[head_dim] * math.sqrt(wgs)
+        return seq_kv <= SHORT_SPLIT_KEYS[head_dim, paged] * math.sqrt(wgs)
     block_m = max(1, FWD_ROWS // group)
     n_mblk, n_bh = _cdiv(seq_q, block_m), batch * num_kv_heads
     tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
+    persistent = head_dim == 128 and not paged
     if kv_chunks:
         other = OTHER_STEP_US["chunks"][head_dim] * chunks_makespan(
             tiles, kv_chunks, n_bh, cu_count, batch * num_heads * seq_q, head_dim, causal, persistent)
@@ -600,7 +603,27 @@ def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv:
         lo, hi = OTHER_STEP_US["single"][head_dim]
         other = _step_us(lo, hi, sum(tiles) * n_bh, longest, cu_count) * fwd_split_makespan(
             tiles, fwd_split, n_bh, cu_count, causal, persistent, dealt=persistent and causal and n_bh > 8)
-    return short_us(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim) < other
+    share = _short_share(kv_chunks, paged, wgs / cu_count)
+    return short_us(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim) < share * other
+
+
+def _short_share(kv_chunks: int, paged: bool, wgs_per_cu: float) -> float:
+    """The share of the other route's modelled time below which the short form
+    is taken: what the models cannot tell apart stays with the other route.
+
+    Key chunks are faster than their model says by up to a quarter, most when
+    there are many; and a step of the short form waits for table reads when
+    paged, which few workgroups do not hide.  Measured, share and short /
+    chunks in us: contiguous, up to 4 chunks, 128 or more workgroups 0.95 44.7 /
+    49.9, 0.96 0.83 times, fewer 0.88 37.6 / 41.4, 0.96 1.08 times, 0.98 1.29
+    times; 8 chunks 0.80 22.8 / 24.9, 0.90 19.1 / 16.3, 0.99 27.0 / 21.8; paged,
+    up to 4 0.84 0.86 times, 0.90 1.05 times, 8 0.78 0.87 times, 0.91 23.0 / 16.9;
+    paged with 8-28 workgroups 0.65-0.70 1.0-1.22 times."""
+    if not kv_chunks:
+        return 1.0
+    if paged or kv_chunks >= 8:
+        return 0.0 if wgs_per_cu < 0.125 else 0.9 - 0.05 * paged - 0.05 * (kv_chunks >= 8)
+    return 1.0 if wgs_per_cu >= 0.5 else 0.9
 
 
 def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv: int,
@@ -634,7 +657,7 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
         route = Route("single", 1, route.workgroups + (ns - route.fwd_split) * n_bh, ns)
     if rows > flat_max_rows(head_dim) and use_short(
             batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
-            route.splits if route.kind == "chunks" else 0, route.fwd_split, head_dim == 128):
+            route.splits if route.kind == "chunks" else 0, route.fwd_split):
         wgs = _cdiv(seq_q, SHORT_ROWS // (num_heads // num_kv_heads)) * num_kv_heads * batch
         if route.kind == "single":
             need = _fwd_split_bytes(batch, num_kv_heads, head_dim, route.fwd_split)

@@ -307,7 +307,7 @@ def paged_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_s
     if rows <= flat_max_rows(head_dim) or max_seq_len < 1 or block_size < single_pass_min_block(head_dim):
         return False
     kc, ns = paged_single_plan(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, causal, head_dim)
-    return use_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, causal, head_dim, kc, ns, False)
+    return use_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, causal, head_dim, kc, ns, True)
 
 
 def paged_kv_chunks(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_seq_len: int,

@@ -770,7 +770,15 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   if (total <= 0) return hipSuccess;
   const int cus = device_cu_count();
   const bool fixed_lists = p.kv_splits == 0 && total < kFwdDynMinItemsPerWg * std::max(cus, 1);
-  set_item_order(p, per_bh, PG > 0 || D == 64 || (p.dm.causal ? fixed_lists : p.n_split > 0));
+  // (item_of has the figures.)  Contiguous without a mask: only the split
+  // blocks, whose count is chosen for this order (dispatch.py
+  // FWD_SPLIT_MAX_ROUNDS).
+  if (p.kv_splits > 0)
+    set_item_order(p, per_bh, PG > 0 && D == 128, kDealPairs(D));
+  else if (PG == 0 && !p.dm.causal)
+    set_item_order(p, per_bh, p.n_split > 0, p.dm.B * p.dm.Hkv);
+  else
+    set_item_order(p, per_bh, total > cus && (PG > 0 || D == 64 || fixed_lists), kDealPairs(D));
   p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;

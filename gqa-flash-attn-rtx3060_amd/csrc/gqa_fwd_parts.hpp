@@ -15,13 +15,12 @@ namespace gqa {
 // in the order first of each pair, second of each pair, ...  Dealt, a pair's
 // heavy items no longer start behind the light ones of the pair before it, and
 // the sequences of a batch of unequal lengths spread over all XCDs instead of
-// each filling XCDs of its own.  Measured (us, pair after pair / dealt):
+// each filling XCDs of its own.  Measured (us, pair after pair / dealt), more
+// items than CUs:
 // * head_dim 64 (items handed out by the hardware as workgroups end): causal
-//   3 x 2999 tokens 131 / 117, 2 x 4096 153 / 138, 8 x 700 35.7 / 30.5;
-//   non-causal 4 x 1025 54.8 / 55.1.
-// * Paged, head_dim 128, 512 query tokens over [1700, 5262] keys: 82 / 71,
-//   short form 80 / 66; [600, 5000, 2000] with 400: 122 / 74; 4 x 17000 with
-//   382: 399 / 384.
+//   3 x 2999 tokens 131 / 117, 2 x 4096 153 / 138, 8 x 700 35.7 / 30.5.
+// * Paged, 512 query tokens over [1700, 5262] keys: 82 / 71, short form 80 /
+//   66; [600, 5000, 2000] with 400: 122 / 74; 4 x 17000 with 382: 399 / 384.
 // * Contiguous head_dim 128, causal, fixed lists: sorted heavy first over all
 //   the XCD's pairs, the snake order hands every workgroup the same work;
 //   pair after pair, what met what was chance.  2 x 1300 tokens 42.3 / 35.9, 2
@@ -29,8 +28,20 @@ namespace gqa {
 //   6 x 1300 124 / 93, 2 x 4096 231 / 227.  With many items per workgroup
 //   (claimed as it goes), and key chunks: pair after pair, fewer pairs' keys
 //   in each L2.
-// * Without a mask only the split blocks need it (dispatch.py
-//   FWD_SPLIT_MAX_ROUNDS).
+// * Many pairs per XCD (kDealPairs): nothing is shared in L2 any more.  Paged
+//   head_dim 128, 34 pairs, 197 tokens over 2755 keys 358 / 418, 28 pairs 183
+//   over 8184 662 / 727, 18 pairs 659 over 689 115 / 123; contiguous 28 pairs
+//   376 over 4341 1.20 times; head_dim 64 36 pairs 134 over 7635 448 / 509, 32
+//   pairs 295 over 10192 777 / 916.  Up to 12 (24 at head_dim 64) 90 shapes
+//   are faster by 6 % in the mean.
+// * At most one item per CU, all start together: paged head_dim 64, 13 pairs
+//   21.8 / 23.5, 14 pairs 20.2 / 21.7; contiguous 10 pairs 13.0 / 14.0.
+// * Key chunks, paged head_dim 128: 97 tokens of [4223, 9688] keys 49.5 / 44.7,
+//   equal lengths alike; head_dim 64 35 tokens over 1981 keys 18.9 / 22.6, 127
+//   over 4834 32.9 / 35.7, so pair after pair there.
+// * Without a mask, contiguous, only the split blocks need it (dispatch.py
+//   FWD_SPLIT_MAX_ROUNDS): head_dim 64 4 x 1025 54.8 / 55.1, 25 pairs 2194
+//   tokens 954 / 1010.
 // * The short form gains once its workgroups no longer start together: 4 x 300
 //   tokens (320 workgroups) 16.8 / 15.8, 8 x 300 over 16/4 heads 16.3 / 14.9;
 //   2 x 512 (256) 12.4 / 12.8.

@@ -186,14 +186,18 @@ constexpr int kFusedMaxRowSplitsHost = 4096;
 constexpr int kPagedTableMax = 2048;
 
 // Item order of `per_bh` items per (b, kv head); div_items with it.  `deal`:
-// whether the kernel gains from pairs dealt to the XCDs (item_of).
-inline void set_item_order(FwdParams& p, int per_bh, bool deal) {
+// whether the kernel gains from pairs dealt to the XCDs (item_of), for at most
+// `max_pairs` pairs per XCD.
+inline void set_item_order(FwdParams& p, int per_bh, bool deal, int max_pairs) {
   const int n_bh = p.dm.B * p.dm.Hkv;
   p.div_items = make_fast_div((uint32_t)per_bh);
-  p.xcd_heads = deal && n_bh % 8 == 0 && n_bh > 8 ? n_bh / 8 : 0;
+  p.xcd_heads = deal && n_bh % 8 == 0 && n_bh > 8 && n_bh <= 8 * max_pairs ? n_bh / 8 : 0;
   p.div_heads = make_fast_div((uint32_t)(p.xcd_heads > 0 ? p.xcd_heads : 1));
   p.div_share = make_fast_div((uint32_t)(p.xcd_heads > 0 ? p.xcd_heads * per_bh : 1));
 }
+// Pairs an XCD takes side by side before their K and V no longer share its L2
+// (measured in gqa_fwd_parts.hpp, item_of).
+constexpr int kDealPairs(int head_dim) { return head_dim == 64 ? 24 : 12; }
 
 // Paged cache write: new tokens (num_tokens, Hkv, D) into
 // (num_blocks, block_size, Hkv, D) caches at slot_mapping[t].

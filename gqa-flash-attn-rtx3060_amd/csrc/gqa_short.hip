@@ -414,7 +414,7 @@ template <int DT, int D, int PG>
 static hipError_t launch_short_t(FwdParams p, hipStream_t stream) {
   const int64_t total = (int64_t)p.n_mblk * p.dm.Hkv * p.dm.B;
   if (total <= 0) return hipSuccess;
-  set_item_order(p, p.n_mblk, PG > 0 || D == 64 || total > device_cu_count());
+  set_item_order(p, p.n_mblk, PG > 0 || D == 64 || total > device_cu_count(), kDealPairs(D));
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;
   hipLaunchKernelGGL((gqa_short_kernel<DT, D, PG>), dim3((unsigned)total), dim3(kFwdThreads), 0, stream, p);

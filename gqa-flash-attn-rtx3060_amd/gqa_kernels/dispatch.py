@@ -161,6 +161,9 @@ FWD_MERGE_OVERHEAD = 1
 FWD_SPLIT_MAX_ROUNDS = 5
 FWD_FILL_MERGE_OVERHEAD = 4
 FWD_TILE = 64
+# Pairs per XCD up to which the head_dim-128 single pass deals them (kDealPairs,
+# gqa_params.hpp).
+FWD_DEAL_PAIRS = 12
 # The persistent single pass claims work dynamically only with at least this
 # many items per workgroup (kFwdDynMinItemsPerWg, gqa_params.hpp); below it
 # every workgroup takes a fixed list (gqa_fwd.hip item_at: XCD x's
@@ -249,6 +252,12 @@ def fwd_split_makespan(tiles, n_split: int, n_bh: int, cu_count: int, causal: bo
     for c in items:
         _push_run(runs, c + FWD_ITEM_OVERHEAD, per_xcd)
     return _list_makespan(runs, n_bh // per_xcd, cu_count, persistent)
+
+
+def _dealt(n_bh: int) -> bool:
+    """Whether the head_dim-128 kernel deals n_bh (b, kv head) pairs to the
+    XCDs (set_item_order, kDealPairs)."""
+    return n_bh % 8 == 0 and 8 < n_bh <= 8 * FWD_DEAL_PAIRS
 
 
 def _push_run(runs, cost, count: int) -> None:
@@ -602,7 +611,7 @@ def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv:
         longest = max(max(tiles[:n_mblk - fwd_split], default=0), _cdiv(max(tiles[n_mblk - fwd_split:], default=0), 2))
         lo, hi = OTHER_STEP_US["single"][head_dim]
         other = _step_us(lo, hi, sum(tiles) * n_bh, longest, cu_count) * fwd_split_makespan(
-            tiles, fwd_split, n_bh, cu_count, causal, persistent, dealt=persistent and causal and n_bh > 8)
+            tiles, fwd_split, n_bh, cu_count, causal, persistent, dealt=persistent and causal and _dealt(n_bh))
     share = _short_share(kv_chunks, paged, wgs / cu_count)
     return short_us(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim) < share * other
 
@@ -652,7 +661,7 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
     if rows <= 0 or seq_kv <= 0 or batch <= 0:
         return route
     n_bh = batch * num_kv_heads
-    if route.kind == "single" and causal and head_dim == 128 and n_bh > 8 and n_bh % 8 == 0:
+    if route.kind == "single" and causal and head_dim == 128 and _dealt(n_bh):
         ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, True, dealt=True)
         route = Route("single", 1, route.workgroups + (ns - route.fwd_split) * n_bh, ns)
     if rows > flat_max_rows(head_dim) and use_short(

@@ -2,7 +2,8 @@
 dealt over the XCDs (item_of in gqa_fwd_parts.hpp) against the CPU oracle:
 batch * kv heads 16, 24 and 32 (two to four pairs per XCD), beside 8 and 12
 (pair after pair), one to several query blocks, split blocks, LSE, and ragged
-paged batches."""
+paged batches; and at sizes on both sides of the lines of set_item_order,
+against the same sequences alone."""
 from __future__ import annotations
 
 import pytest
@@ -46,3 +47,21 @@ def test_ragged_paged_order(lens, D, route, splits):
     o, lse = paged_attention(*args, True, max_seq_len=max(lens), return_lse=True, route=route, splits=splits)
     torch.cuda.synchronize()
     _check(o, lse, q, kc, vc, table, seq_lens, True, torch.bfloat16)
+
+
+@pytest.mark.parametrize("B,D,sq", [(3, 64, 800), (2, 64, 2100), (24, 64, 200), (25, 64, 200), (3, 128, 900),
+                                    (12, 128, 333), (13, 128, 333)])
+@pytest.mark.parametrize("causal,n_split", [(True, 0), (True, 2), (False, 0), (False, 2)])
+def test_order_does_not_change_results(B, D, sq, causal, n_split):
+    """More items than CUs, on both sides of the line where pairs are dealt: each
+    sequence of the batch has the bits that it has alone (eight pairs, pair after
+    pair)."""
+    from gqa_kernels.dispatch import single_pass_forward
+    print(f"order B={B} D={D} sq={sq} causal={causal} n_split={n_split}", flush=True)
+    q, k, v = make_inputs(B, 32, 8, sq, sq + 70, D, torch.bfloat16, seed=B + sq, device=DEV)
+    o, lse = single_pass_forward(q, k, v, torch.empty_like(q), causal, n_split, True)
+    for b in range(0, B, 1 if B < 4 else 5):
+        one = [t[b:b + 1] for t in (q, k, v)]
+        ob, lb = single_pass_forward(*one, torch.empty_like(one[0]), causal, n_split, True)
+        torch.cuda.synchronize()
+        assert torch.equal(o[b:b + 1], ob) and torch.equal(lse[b:b + 1], lb), b

@@ -603,6 +603,15 @@ def use_short(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_kv:
     n_mblk, n_bh = _cdiv(seq_q, block_m), batch * num_kv_heads
     tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
     persistent = head_dim == 128 and not paged
+    # A second round of workgroups against one round of whole blocks of few
+    # tiles, us, short / single: 15 x 74 tokens 15.6 / 13.9, 11 x 78 paged 16.1 /
+    # 12.4, 15 x 54 over 64/16 heads 16.8 / 14.7; longer or split blocks gain (4 x
+    # 400 19.4 / 20.7).  One tile gives the second key group nothing to do: 52 x
+    # 21 paged at head_dim 64 12.2 / 10.7.
+    if not kv_chunks and wgs > cu_count and (
+            (head_dim == 128 and not fwd_split and n_mblk * n_bh <= cu_count and max(tiles) <= 4)
+            or (head_dim == 64 and paged and max(tiles) <= 1)):
+        return False
     if kv_chunks:
         other = OTHER_STEP_US["chunks"][head_dim] * chunks_makespan(
             tiles, kv_chunks, n_bh, cu_count, batch * num_heads * seq_q, head_dim, causal, persistent)

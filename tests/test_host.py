@@ -486,9 +486,11 @@ def test_fwd_split_measured_choices():
     ((2, 32, 8, 39, 2075), True, 128, "chunks"), ((3, 8, 4, 90, 2084), True, 128, "chunks"),  # 8 key chunks
     ((4, 4, 4, 86, 2028), False, 64, "chunks"), ((1, 64, 8, 16, 2016), False, 64, "chunks"),
     ((2, 8, 2, 33, 1624), True, 64, "chunks"),                                                # few workgroups
+    ((15, 32, 8, 74, 74), True, 128, "single"), ((15, 64, 16, 54, 54), False, 128, "single"),  # a second round
+    ((4, 32, 8, 400, 400), True, 128, "short"), ((6, 32, 8, 200, 200), True, 128, "short"),
     ((1, 32, 8, 512, 4096), True, 128, "short"), ((3, 32, 8, 303, 2923), False, 128, "short"),  # measured faster
     ((3, 32, 8, 81, 2798), True, 64, "short"), ((4, 32, 8, 53, 1966), True, 64, "short")])
-def test_short_form_against_key_chunks(shape, causal, head_dim, kind):
+def test_short_form_of_contiguous_calls(shape, causal, head_dim, kind):
     from gqa_kernels.dispatch import choose_plan
     assert choose_plan(*shape, 256, causal, head_dim).kind == kind
 
@@ -496,6 +498,7 @@ def test_short_form_against_key_chunks(shape, causal, head_dim, kind):
 @pytest.mark.parametrize("batch,seq_q,keys,head_dim,short", [
     (4, 20, 2048, 64, False), (2, 30, 1675, 64, False), (3, 80, 3970, 64, False), (2, 163, 4791, 64, False),
     (9, 36, 10097, 128, False), (6, 7, 1490, 64, False),  # chunks, and the split-KV pass, measured faster
+    (11, 78, 78, 128, False), (52, 21, 21, 64, False),    # a second round of short workgroups
     (16, 20, 2048, 64, True), (5, 48, 1738, 64, True), (12, 5, 1224, 64, True), (2, 512, 5262, 128, True)])
 def test_short_form_of_paged_calls(batch, seq_q, keys, head_dim, short):
     from gqa_kernels.paged import paged_short

@@ -261,6 +261,7 @@ template <int TK> struct FlatWave {
     return p.q_len != nullptr && p.q_len[s] <= 0 ? 0 : (keys + TK - 1) / TK;
   }
   __device__ static int scan(int n) { return wave_scan(n); }
+  __device__ static void add(int& a, int b) { a += b; }
   __device__ static int read(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
   __device__ static int first_above(int v, int x) {
     return __builtin_ffsll((long long)__builtin_amdgcn_ballot_w64(v > x)) - 1;
@@ -355,17 +356,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int pos_end = fast_div(wr0 + 32 * RW - 1, p.div_g.mul, p.div_g.shift);
   const FlatWave<64> flat_wave(p, lane);
   FlatWalk<FlatWave<64>, PAGED> walk;
-  bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
+  if constexpr (FLAT && PAGED) {
+    // One workgroup past the slots writes the combine's plan: its two passes
+    // over the lengths held up the launch in the first slot's workgroup (8
+    // sequences of 128 keys 8.9 -> 8.5 us).
+    if (blockIdx.x == (unsigned)total) {
+      if (wave == 0) write_plan(p, flat_wave);
+      return;
+    }
+  }
   if constexpr (flat) walk.start(flat_wave, s);
   // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
   for (;;) {
   int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
   if constexpr (flat) {
     int from, cnt;
-    if (!walk.next(flat_wave, from, cnt)) {
-      if (plan_due) write_plan(p, flat_wave);  // (no sequence has keys)
-      return;
-    }
+    if (!walk.next(flat_wave, from, cnt)) return;
     b = walk.b;
     c0 = from * 64;
     len = cnt * 64;
@@ -514,9 +520,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       qreg[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 32u * ks, 0, 0));
   }
   issue(1, lds_c_k1, lds_d_v1);
-  // (While the first piece's loads are in flight.)
-  if (plan_due) write_plan(p, flat_wave);
-  plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).  Waiting here,
   // explicitly, also settles Q for the compiler: otherwise it waits for
   // every load in flight before entering the tile loop.
@@ -864,17 +867,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int head = kvh * dm.G + g;
   const FlatWave<TK> flat_wave(p, lane);
   FlatWalk<FlatWave<TK>, PAGED> walk;
-  bool plan_due = FLAT && PAGED && w == 0 && wave == 0;  // one wave of the launch writes the plan
+  if constexpr (FLAT && PAGED) {
+    // One workgroup past the slots writes the combine's plan: its two passes
+    // over the lengths held up the launch in the first slot's workgroup (8
+    // sequences of 128 keys 8.9 -> 8.5 us).
+    if (blockIdx.x == (unsigned)total) {
+      if (wave == 0) write_plan(p, flat_wave);
+      return;
+    }
+  }
   if constexpr (flat) walk.start(flat_wave, s);
   // The pieces of this workgroup: its chunk, or (flat split) those of its slot.
   for (;;) {
   int c0 = s * p.chunk, len = p.chunk;  // keys [c0, c0 + len)
   if constexpr (flat) {
     int from, cnt;
-    if (!walk.next(flat_wave, from, cnt)) {
-      if (plan_due) write_plan(p, flat_wave);  // (no sequence has keys)
-      return;
-    }
+    if (!walk.next(flat_wave, from, cnt)) return;
     b = walk.b;
     c0 = from * TK;
     len = cnt * TK;
@@ -1002,9 +1010,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       qreg[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 64u * ks, 0, 0));
   }
   issue(1, lds_c_k1, lds_d_v1);
-  // (While the first piece's loads are in flight.)
-  if (plan_due) write_plan(p, flat_wave);
-  plan_due = false;
   // Tile 0 and Q have landed (tile 1 may still be in flight).
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * NI * NSUB));
 
@@ -1249,7 +1254,7 @@ static hipError_t launch_decode_t(SplitParams p, hipStream_t stream) {
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.div_g = make_fast_div((uint32_t)p.dm.G);
   p.div_units = make_fast_div((uint32_t)std::max((p.dm.Skv + unit - 1) / unit, 1));
-  const dim3 grid((unsigned)total), block(256);
+  const dim3 grid((unsigned)(total + (FLAT && KV != 0 ? 1 : 0))), block(256);
   if (p.dm.D == 64)  // decode_kernel_fits: at most 16 packed rows
     hipLaunchKernelGGL((gqa_decode16_kernel<DT, KV, FLAT, 64>), grid, block, 0, stream, p);
   else if (p.dm.G * p.dm.Sq <= 16)

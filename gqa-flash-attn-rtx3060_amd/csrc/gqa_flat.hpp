@@ -6,10 +6,10 @@
 //
 // W: B, slots, seq_units (contiguous: units per sequence); Lanes, one int per
 // lane; units(base, keys): per lane, the units and keys of sequence base +
-// lane; scan: inclusive sum over the lanes; read(v, l): lane l's value;
-// first_above(v, x): first lane whose value exceeds x; share(n) = n / slots,
-// sequence(n) = n / seq_units; own(v, lane): the value of `lane`; each(f):
-// f(lane) for every lane of the caller.
+// lane; scan: inclusive sum over the lanes; add: lane by lane; read(v, l):
+// lane l's value; first_above(v, x): first lane whose value exceeds x; share(n)
+// = n / slots, sequence(n) = n / seq_units; own(v, lane): the value of `lane`;
+// each(f): f(lane) for every lane of the caller.
 #pragma once
 
 #if defined(__HIPCC__)
@@ -38,10 +38,9 @@ template <class W, bool PAGED> struct FlatWalk {
     incl = W::scan(mine);
   }
   GQA_WAVE_FN static int total_of(const W& w, int from) {
-    int total = 0;
-    Lanes k;
-    for (int g0 = from; g0 < w.B; g0 += 64) total += W::read(W::scan(w.units(g0, k)), 63);
-    return total;
+    Lanes sum{}, k;
+    for (int g0 = from; g0 < w.B; g0 += 64) W::add(sum, w.units(g0, k));
+    return W::read(W::scan(sum), 63);
   }
 
   GQA_WAVE_FN void start(const W& w, int slot) {
@@ -50,7 +49,8 @@ template <class W, bool PAGED> struct FlatWalk {
       base = 0;
       carry = 0;
       scan(w);
-      total = W::read(incl, 63) + total_of(w, 64);
+      total = W::read(incl, 63);
+      if (w.B > 64) total += total_of(w, 64);
     } else {
       n = w.seq_units;
       total = n * w.B;

@@ -30,6 +30,9 @@ struct HostWave {
     for (int i = 1; i < 64; ++i) n[i] += n[i - 1];
     return n;
   }
+  static void add(Lanes& a, const Lanes& b) {
+    for (int i = 0; i < 64; ++i) a[i] += b[i];
+  }
   static int read(const Lanes& v, int l) { return v[l]; }
   static int first_above(const Lanes& v, int x) {
     for (int i = 0; i < 64; ++i)

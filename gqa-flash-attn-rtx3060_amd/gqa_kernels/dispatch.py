@@ -80,6 +80,11 @@ DEC16_ROWS = 16
 # 14.3 / 16.5, powers of two 0.2-1.5 us the other way (a workgroup that
 # crosses into the next sequence drains and refills its pipeline).
 FLAT_MIN_USED = 0.7
+# ... and whose pieces keep this many tile steps (flat_piece_steps) for the
+# start of each: 260 such batches, steps a piece and flat / fixed in the mean
+# 2-4 1.07, 4-6 1.05, 6-8 0.99, 8-10 0.94, 10-16 0.92, more 0.87 (4 tokens, 5 x
+# 1527 keys at head_dim 64 12.2 / 11.1, 20 x 1910 of 4 kv heads 21.7 / 20.6).
+FLAT_MIN_PIECE = 8
 # The short form of the single pass (gqa_fwd_short_launch: workgroups of
 # SHORT_ROWS packed rows, two key tiles a step), considered for at most
 # SHORT_MAX_WG_PER_CU workgroups per CU.  Its run time in us, fitted within
@@ -560,6 +565,12 @@ def _fwd_split_bytes(batch: int, num_kv_heads: int, head_dim: int, n_split: int)
     return batch * num_kv_heads * n_split * 2 * 512 * (head_dim // 2 + 2) * 4
 
 
+def flat_piece_steps(batch: int, seq_kv: int, slots: int, head_dim: int = 128) -> float:
+    """Tile steps of a piece of a flat split over `slots` ranges: every range
+    is one piece, and one more for each sequence that it crosses into."""
+    return batch * _cdiv(seq_kv, 128 if head_dim == 64 else 64) / (slots + batch)
+
+
 def flat_max_rows(head_dim: int = 128) -> int:
     """Packed rows per kv head up to which the flat split is built."""
     return DEC16_ROWS if head_dim == 64 else SPLIT_ROWS
@@ -664,7 +675,7 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
       side by side, which leaves less to split than choose_route's model of
       pair after pair: 2 x 1536 tokens 54.3 -> 45.4 us, 4 x 768 36.3 -> 28.9.
     * Batches that no power-of-two split count spreads evenly over the
-      compute units take the flat split (FLAT_MIN_USED)."""
+      compute units take the flat split (FLAT_MIN_USED, FLAT_MIN_PIECE)."""
     route = choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
     rows = num_heads // num_kv_heads * seq_q
     if rows <= 0 or seq_kv <= 0 or batch <= 0:
@@ -694,7 +705,8 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
         return wgs / (cu_count * _cdiv(wgs, cu_count))
 
     slots = max(1, cu_count // num_kv_heads)
-    if batch > 1 and slots <= _lib.GQA_MAX_SPLITS and used(base * splits) < FLAT_MIN_USED and base * splits > cu_count:
+    if (batch > 1 and slots <= _lib.GQA_MAX_SPLITS and used(base * splits) < FLAT_MIN_USED and base * splits > cu_count
+            and flat_piece_steps(batch, seq_kv, slots, head_dim) >= FLAT_MIN_PIECE):
         return Route("flat", slots, slots * num_kv_heads)
     if splits == 1 and batch <= _lib.GQA_MAX_SPLITS:
         return Route("flat", batch, base)

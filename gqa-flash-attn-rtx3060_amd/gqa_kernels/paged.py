@@ -41,7 +41,7 @@ import torch
 
 from . import _lib
 from .dispatch import (_KIND_IDS, FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
-                       fwd_split_makespan, use_short)
+                       flat_piece_steps, fwd_split_makespan, use_short)
 from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces,
                         flat_workspace_bytes, stream_handle, workspace_bytes)
 
@@ -102,6 +102,9 @@ _SPLIT_WG_PER_CU = 2
 _LDS_WG_PER_CU = 1
 _LDS_WG_PER_CU_INTERLEAVED = 4
 _MIN_CHUNK = 256
+# Tile steps a piece of the flat split keeps (paged_flat_slots).
+_FLAT_MIN_PIECE = 16
+_FLAT_MIN_PIECE_WIDE = 10
 _SPLIT_MAX_ROWS = 64  # packed rows per kv head up to which the split-KV pass is used
 _SPLIT_MAX_ROWS_WIDE = 128  # ... at head_dim 128 with pages of >= 4 keys (128-row workgroups)
 _DEC16_ROWS = 16  # packed rows up to which head_dim 64 runs the LDS-DMA first pass
@@ -182,28 +185,42 @@ def paged_splits(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_
 
 @functools.lru_cache(maxsize=4096)
 def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, max_seq_len: int, cu_count: int,
-                     block_size: int = 64, head_dim: int = 128) -> int:
+                     block_size: int = 64, head_dim: int = 128, heads_interleaved: bool = False) -> int:
     """Slots of the flat split (gqa_paged_split_flat_launch) for a paged call,
     0 for the fixed split count of ``paged_splits``.
 
     Cutting every sequence alike leaves a batch of unequal lengths waiting
     for its longest sequences; the flat split gives every workgroup the same
     number of keys, read from the lengths on the device.  One workgroup per
-    compute unit (two or four measured the same or slower).  Measured on
-    MI355X (bf16, one token, G = 4, 8 kv heads, us, fixed -> flat): 16-key
-    token-major pages, B = 32 of 100-8000 keys 111.7 -> 94.2, B = 16 of
-    500-16000 112.0 -> 93.5, B = 64 of 100-4000 114.4 -> 97.8, B = 14 of
-    600-6000 45.2 -> 37.5, 4 tokens B = 8 of 100-8000 37.2 -> 28.9; head-major
-    64-key pages, B = 8 of 1000-30000 114.7 -> 80.9; equal lengths B = 16 x 8192
-    84.4 -> 83.7, B = 4 x 32768 85.1 -> 88.3.  One sequence (10.3 against 12.4
-    at 8192 keys) keeps the fixed count."""
+    compute unit (two or four measured the same or slower).  Each piece of a
+    range costs its own start, so pieces have to keep _FLAT_MIN_PIECE tile
+    steps, more with many sequences to a range, whose fixed split hands out
+    more workgroups than the device holds.  Measured on MI355X (bf16, us, fixed
+    -> flat): 16-key token-major pages, one token, B = 32 of 100-8000 keys
+    111.7 -> 94.2, B = 16 of 500-16000 112.0 -> 93.5, B = 64 of 100-4000 114.4 ->
+    97.8, B = 14 of 600-6000 45.2 -> 37.5, 4 tokens B = 8 of 100-8000 37.2 ->
+    28.9; head-major 64-key pages, B = 8 of 1000-30000 114.7 -> 80.9.  900 batches,
+    flat / fixed in the mean, equal lengths and lengths drawn from a tenth to
+    the whole of max_seq_len, by steps a piece: at head_dim 128 up to one
+    sequence a range 4-7 1.08 and 1.09, 7-10 1.03 and 1.08, 10-16 0.99 and 0.94,
+    16-32 0.96 and 0.88, more 0.96 and 0.79 (fewer than 5 sequences 10-16 1.02
+    and 0.96, more 1.00 and 0.89); two 10-16 1.03 and 0.98, 16-32 1.00 and 0.94,
+    more 0.98 and 0.86; four 16-32 1.04 and 0.98, more 1.00 and 0.89; more than
+    four 1.0-1.4.  At head_dim 64 up to one 10-16 1.02 and 0.93, 16-32 1.02 and
+    0.90, more 0.93 and 0.87; one token over interleaved heads, which the
+    fixed count gives four workgroups per CU, 16-32 up to 1.09."""
     rows = num_heads // num_kv_heads * seq_q
     if batch < 2 or max_seq_len < 1 or block_size < single_pass_min_block(head_dim):
         return 0
     slots = cu_count // num_kv_heads
-    return slots if 0 < rows <= flat_max_rows(head_dim) and 1 <= slots <= _lib.GQA_MAX_SPLITS else 0
-
-
+    if not 0 < rows <= flat_max_rows(head_dim) or not 1 <= slots <= _lib.GQA_MAX_SPLITS or batch > 4 * slots:
+        return 0
+    least = _FLAT_MIN_PIECE
+    if batch > 2 * slots or (head_dim == 64 and heads_interleaved and seq_q == 1):
+        least *= 2
+    elif head_dim == 128 and 5 <= batch <= slots:
+        least = _FLAT_MIN_PIECE_WIDE
+    return slots if flat_piece_steps(batch, max_seq_len, slots, head_dim) >= least else 0
 
 
 def _paged_host():
@@ -420,11 +437,11 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     dev = qdev.index if qdev.index is not None else torch.cuda.current_device()
     splits_given = splits is not None
     flat_slots = 0
+    interleaved = k_cache.stride(1) != head_dim or v_cache.stride(1) != head_dim
     if splits is None and route in (None, "split"):
         flat_slots = paged_flat_slots(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
-                                      head_dim)
+                                      head_dim, interleaved)
     if splits is None:
-        interleaved = k_cache.stride(1) != head_dim or v_cache.stride(1) != head_dim
         splits = paged_splits(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
                               head_dim, interleaved)
     if scale is None:
@@ -442,7 +459,6 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     stream = stream_handle(qdev)
     plan_key = None
     if default_route and batch > 0 and seq_q > 0:
-        interleaved = k_cache.stride(1) != head_dim or v_cache.stride(1) != head_dim
         plan_key = [1, batch, num_heads, num_kv_heads, seq_q, max_seq_len, head_dim, int(bool(causal)), dev, block_size,
                     int(interleaved), int(varlen)]
     kv_chunks = fwd_split = 0

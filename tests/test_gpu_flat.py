@@ -69,18 +69,32 @@ def test_flat_matches_fixed_split(layout, dtype, sq):
     from gqa_kernels import gqa_flash_attn
     from gqa_kernels.dispatch import _cu_count, choose_plan
     from gqa_kernels.gqa_split import split_kv_forward
-    assert choose_plan(5, 32, 8, sq, 2500, _cu_count(0)).kind == "flat"
-    q, k, v = make_inputs(5, 32, 8, sq, 2500, 128, dtype, seed=sq, device=DEV)
+    assert choose_plan(5, 32, 8, sq, 4000, _cu_count(0)).kind == "flat"
+    q, k, v = make_inputs(5, 32, 8, sq, 4000, 128, dtype, seed=sq, device=DEV)
     if layout == "bshd":
         q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
     elif layout == "cache":  # views of longer caches
-        k, v = (torch.cat([t, torch.full_like(t, float("nan"))], 2)[:, :, :2500] for t in (k, v))
+        k, v = (torch.cat([t, torch.full_like(t, float("nan"))], 2)[:, :, :4000] for t in (k, v))
     o, lse = gqa_flash_attn(q, k, v, True, return_lse=True)
     fo, flse = split_kv_forward(q, k, v, True, 4, return_lse=True)
     # Both round P and o once: two results differ by at most the parity gate.
     assert_close(o, fo, BASELINE_TOL[dtype], "flat against fixed")
     assert (lse - flse).abs().max().item() <= LSE_TOL
     assert o.stride() == fo.stride()
+
+
+def _force_flat(monkeypatch):
+    """Split-KV calls take the flat split, whatever the rule says of their
+    sizes; returns the slots chosen, in order."""
+    from gqa_kernels import paged
+    chosen = []
+
+    def slots(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, *rest):
+        chosen.append(cu_count // num_kv_heads)
+        return chosen[-1]
+
+    monkeypatch.setattr(paged, "paged_flat_slots", slots)
+    return chosen
 
 
 LENS = {
@@ -96,24 +110,26 @@ LENS = {
 @pytest.mark.parametrize("lens", list(LENS))
 @pytest.mark.parametrize("Hq,Hkv,sq,D,bs", [(32, 8, 1, 128, 16), (64, 8, 4, 128, 64), (24, 8, 1, 64, 8),
                                           (4, 1, 2, 128, 4)])
-def test_flat_paged(lens, Hq, Hkv, sq, D, bs):
-    from gqa_kernels.dispatch import _cu_count
-    from gqa_kernels.paged import paged_attention, paged_flat_slots
+def test_flat_paged(lens, Hq, Hkv, sq, D, bs, monkeypatch):
+    from gqa_kernels.paged import paged_attention
+    chosen = _force_flat(monkeypatch)
     L = LENS[lens]
     q, kc, vc, table, seq_lens = _paged_inputs(len(L), Hq, Hkv, sq, L, D, bs, torch.bfloat16, seed=len(L), hnd=bs == 64)
     mx = max(1, max(L))
-    assert paged_flat_slots(len(L), Hq, Hkv, sq, mx, _cu_count(0), bs, D) > 0
-    o, lse = paged_attention(*(t.to(DEV) for t in (q, kc, vc, table, seq_lens)), True, max_seq_len=mx, return_lse=True)
+    o, lse = paged_attention(*(t.to(DEV) for t in (q, kc, vc, table, seq_lens)), True, max_seq_len=mx, return_lse=True,
+                             route="split")
+    assert chosen and chosen[0] > 0
     if not any(L):  # (the check below takes a maximum over the finite LSEs)
         assert torch.isneginf(lse).all()
         lse = None
     _check(o, lse, q, kc, vc, table, seq_lens, True, torch.bfloat16)
 
 
-def test_flat_paged_varlen():
+def test_flat_paged_varlen(monkeypatch):
     """Variable query lengths through the flat split: sequences without query
     rows take no part, each has its own causal alignment."""
     from gqa_kernels.paged import paged_attention
+    chosen = _force_flat(monkeypatch)
     L, ql = [500, 40, 0, 333, 1000, 3], [1, 4, 2, 0, 3, 3]
     B, H, Hkv, D = len(L), 32, 8, 128
     q, kc, vc, table, seq_lens = _paged_inputs(B, H, Hkv, 4, L, D, 16, torch.bfloat16, seed=3)
@@ -123,6 +139,7 @@ def test_flat_paged_varlen():
                              max_seq_len=max(L), return_lse=True, route="split",
                              query_start=torch.tensor(start, dtype=torch.int32, device=DEV),
                              query_lens=torch.tensor(ql, dtype=torch.int32, device=DEV), max_query_len=4)
+    assert chosen and chosen[0] > 0
     for b, n in enumerate(ql):
         if n:
             one = slice(b, b + 1)

@@ -179,7 +179,7 @@ _WORKSPACE_CALLS = [
     ("contiguous", (5, 32, 8, 1, 8192, 128, True)), ("contiguous", (1, 32, 8, 64, 8192, 128, True)),
     ("contiguous", (2, 32, 8, 1025, 1025, 128, True)), ("contiguous", (4, 32, 8, 1025, 1025, 128, False)),
     ("contiguous", (1, 32, 8, 3000, 3000, 64, True)),
-    ("paged", ([3000, 700, 1500], 1, {})), ("paged", ([3000, 1200], 256, dict(route="single", splits=4)))]
+    ("paged", ([6000, 700, 1500, 3000, 4000, 100], 1, {})), ("paged", ([3000, 1200], 256, dict(route="single", splits=4)))]
 
 
 def _workspace_call(kind, spec, seed):

@@ -482,6 +482,26 @@ def test_fwd_split_measured_choices():
         assert choose_route(1, 8, 2, 1024, 1024, 256, True, D).kind == "single"
 
 
+@pytest.mark.parametrize("batch,keys,head_dim,interleaved,flat", [
+    (2, 2048, 128, True, False), (4, 32768, 128, True, True), (4, 8192, 128, True, False),  # pieces of few steps
+    (12, 600, 128, True, False), (12, 8192, 128, True, True), (8, 2048, 128, True, False),
+    (32, 128, 128, True, False), (32, 2048, 128, True, True), (64, 600, 128, True, False),
+    (64, 4096, 128, True, True), (128, 600, 128, True, False), (128, 4096, 128, True, True),
+    (256, 4096, 128, True, False),                                                          # many workgroups as it is
+    (8, 16000, 64, True, False), (8, 16000, 64, False, True), (12, 32768, 64, True, True)])
+def test_paged_flat_rule(batch, keys, head_dim, interleaved, flat):
+    from gqa_kernels.paged import paged_flat_slots
+    assert paged_flat_slots(batch, 32, 8, 1, keys, 256, 16, head_dim, interleaved) == (32 if flat else 0)
+
+
+@pytest.mark.parametrize("shape,head_dim,kind", [
+    ((5, 32, 8, 4, 1527), 64, "split"), ((20, 16, 4, 4, 1910), 128, "split"), ((11, 8, 8, 4, 1039), 128, "split"),
+    ((5, 32, 8, 1, 8192), 128, "flat"), ((20, 32, 8, 1, 3000), 128, "flat"), ((33, 32, 8, 1, 3000), 128, "flat")])
+def test_contiguous_flat_rule(shape, head_dim, kind):
+    from gqa_kernels.dispatch import choose_plan
+    assert choose_plan(*shape, 256, True, head_dim).kind == kind
+
+
 @pytest.mark.parametrize("shape,causal,head_dim,kind", [
     ((2, 32, 8, 39, 2075), True, 128, "chunks"), ((3, 8, 4, 90, 2084), True, 128, "chunks"),  # 8 key chunks
     ((4, 4, 4, 86, 2028), False, 64, "chunks"), ((1, 64, 8, 16, 2016), False, 64, "chunks"),

@@ -239,9 +239,9 @@ void cache_write(const at::Tensor& key, const at::Tensor& value, const at::Tenso
 // of a short call take on the GPU (333 tokens: 16 us of host time beside 9.9
 // us).  These entries do the usual case natively: every check passes, the
 // route of these shapes is known (set_plan, from Python's rules) and the
-// stream's buffers are large enough.  Anything else returns None before
-// allocating or launching, and Python takes the call: it raises, copies,
-// chooses the route (and registers it here) or grows the buffer.
+// stream's buffers are large enough.  Anything else returns None with
+// nothing launched, and Python takes the call: it raises, copies, chooses the
+// route (and registers it here) or grows the buffer.
 // ---------------------------------------------------------------------------
 enum Kind : int { kSplit = 0, kSingle = 1, kChunks = 2, kFlat = 3, kShort = 4 };
 

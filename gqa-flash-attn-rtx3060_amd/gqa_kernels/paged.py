@@ -464,10 +464,13 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     kv_chunks = fwd_split = 0
     if route is None:
         route = paged_route(num_heads, num_kv_heads, seq_q, block_size, head_dim)
-        # (The short form spans a tile's 64 rows with 32-bit byte offsets.)
-        if (not splits_given and max(k_cache.stride(1), v_cache.stride(1)) < 1 << 24
-                and paged_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), bool(causal),
-                                block_size, head_dim)):
+        short = not splits_given and paged_short(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev),
+                                                 bool(causal), block_size, head_dim)
+        # (The short form spans a tile's 64 rows with 32-bit byte offsets.)  A
+        # route that this call's strides refuse is not the shape's.
+        if short and max(k_cache.stride(1), v_cache.stride(1)) >= 1 << 24:
+            short, plan_key = False, None
+        if short:
             route = "short"
         elif route == "single":
             kv_chunks, fwd_split = paged_single_plan(batch, num_heads, num_kv_heads, seq_q, max_seq_len,
@@ -505,6 +508,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             if host is not None and plan_key is not None:
                 host.set_plan(plan_key, _KIND_IDS["flat"], flat_slots, 0, 0.0)
             return out if lse is None else (out, lse)
+        plan_key = None  # refused for this call's strides
     if route == "short":
         n_parts, workspace = 0, None
     elif route == "single":

@@ -138,3 +138,27 @@ def test_paged_same_bits(lens, sq, monkeypatch):
             paged_attention(q, kc, vc, table, seq_lens, **bad)
     with pytest.raises(AssertionError):
         paged_attention(q, kc, vc, table.long(), seq_lens, max_seq_len=max(lens))
+
+
+def test_strides_of_one_call_do_not_plan_the_shape():
+    """A cache whose slots lie too far apart for the short form: the shape is
+    planned by the next ordinary cache, not by the route that this one takes."""
+    from gqa_kernels.dispatch import _cu_count
+    from gqa_kernels.paged import paged_attention, paged_short
+    lens, sq, bs = [301, 250, 90], 45, 4
+    q, kc, vc, table, seq_lens = (t.to(DEV) for t in _paged_inputs(3, 32, 8, sq, lens, 128, bs, torch.bfloat16, seed=8))
+    assert paged_short(3, 32, 8, sq, 301, _cu_count(0), True, bs)
+    n, far = kc.shape[0], 1 << 24
+
+    def spread(c):
+        buf = torch.empty(far * (bs - 1) + n * 8 * 128, dtype=c.dtype, device=DEV)
+        v = buf.as_strided(c.shape, (8 * 128, far, 128, 1))
+        return v.copy_(c)
+
+    call = lambda k, v, **kw: paged_attention(q, k, v, table, seq_lens, max_seq_len=301, **kw)
+    apart = call(spread(kc), spread(vc))
+    near = [call(kc, vc) for _ in range(2)]
+    short = call(kc, vc, route="short")
+    assert not torch.equal(apart, short), "the far cache took the short form too"
+    for o in near:
+        assert torch.equal(o, short)

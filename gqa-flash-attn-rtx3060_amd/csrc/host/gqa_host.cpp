@@ -259,7 +259,7 @@ struct KeyHash {
     return (size_t)(h ^ (h >> 32));
   }
 };
-// Calls hold the GIL throughout, which guards the table; bounded as Python's
+// Guarded by the GIL, which every use of the table holds; bounded as Python's
 // own route caches are.
 std::unordered_map<Key, Plan, KeyHash> g_plans;
 
@@ -368,24 +368,32 @@ py::object flash_attn(const py::handle& hq, const py::handle& hk, const py::hand
   int* cnti = static_cast<int*>(cnt);
   const void *qp = q.data_ptr(), *kp = k.data_ptr(), *vp = v.data_ptr();
   void* op = o.data_ptr();
+  int rc;
+  const char* what;
   if (p.kind == kSplit) {
-    check_rc(gqa_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2, c, dt,
-                              stream), "gqa_split_launch");
+    what = "gqa_split_launch";
+    rc = gqa_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2, c, dt, stream);
   } else if (p.kind == kFlat) {
-    const int rc = gqa_split_flat_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2,
-                                         c, dt, stream);
+    what = "gqa_split_flat_launch";
+    rc = gqa_split_flat_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, p.n, b, hq_, hkv, sq, skv, d, sl2, c, dt,
+                               stream);
     if (rc == GQA_E_FLAT) return py::none();
-    check_rc(rc, "gqa_split_flat_launch");
-  } else if (p.kind == kShort) {
-    check_rc(gqa_fwd_short_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, b, hq_, hkv, sq, skv, d, sl2, c, dt, stream),
-             "gqa_fwd_short_launch");
   } else if (p.kind == kChunks) {
-    check_rc(gqa_fwd_chunks_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2,
-                                   c, dt, stream), "gqa_fwd_chunks_launch");
+    what = "gqa_fwd_chunks_launch";
+    rc = gqa_fwd_chunks_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2, c,
+                               dt, stream);
   } else {
-    check_rc(gqa_fwd_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2,
-                                  c, dt, stream), "gqa_fwd_split_launch");
+    // One launch: other threads run while it waits for room in a full queue.
+    // (The two launches of the calls above share the stream's workspace, which
+    // a call of another thread must not enter in between.)
+    py::gil_scoped_release others;
+    what = p.kind == kShort ? "gqa_fwd_short_launch" : "gqa_fwd_split_launch";
+    rc = p.kind == kShort
+             ? gqa_fwd_short_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, b, hq_, hkv, sq, skv, d, sl2, c, dt, stream)
+             : gqa_fwd_split_launch(qp, qs, kp, ks, vp, vs, op, os, lse_p, wsf, cnti, p.n, b, hq_, hkv, sq, skv, d, sl2,
+                                    c, dt, stream);
   }
+  check_rc(rc, what);
   if (return_lse) return py::make_tuple(o, lse);
   return py::cast(o);
 }

@@ -162,3 +162,31 @@ def test_strides_of_one_call_do_not_plan_the_shape():
     assert not torch.equal(apart, short), "the far cache took the short form too"
     for o in near:
         assert torch.equal(o, short)
+
+
+def test_threads_on_their_own_streams():
+    """Native calls of every kind from three threads, each on a stream of its own
+    (the single launches let the other threads run): every result has the bits
+    of the call alone."""
+    import threading
+    from gqa_kernels import gqa_flash_attn
+    cases = []
+    for i, shape in enumerate(SHAPES):
+        q, k, v = make_inputs(*shape, torch.bfloat16, seed=20 + i, device=DEV)
+        cases.append((q, k, v, gqa_flash_attn(q, k, v)))
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(seed):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for n in range(30):
+                q, k, v, want = cases[(n * (seed + 1) + seed) % len(cases)]
+                if not torch.equal(gqa_flash_attn(q, k, v), want):
+                    bad.append((seed, n))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

@@ -247,7 +247,6 @@ enum Kind : int { kSplit = 0, kSingle = 1, kChunks = 2, kFlat = 3, kShort = 4 };
 
 struct Plan {
   int kind, n;         // n: splits, split blocks, key chunks or slots
-  int64_t reserve;     // bytes of stream workspace the call keeps
   float scale_log2;    // gqa_flash_attn: head_dim^-0.5 * log2(e)
 };
 
@@ -263,12 +262,12 @@ struct KeyHash {
 // own route caches are.
 std::unordered_map<Key, Plan, KeyHash> g_plans;
 
-void set_plan(const std::vector<int64_t>& key, int64_t kind, int64_t n, int64_t reserve, double scale_log2) {
+void set_plan(const std::vector<int64_t>& key, int64_t kind, int64_t n, double scale_log2) {
   Key k{};
   if (key.size() != k.size()) throw std::invalid_argument("set_plan: key length");
   std::copy(key.begin(), key.end(), k.begin());
   if (g_plans.size() >= 8192) g_plans.clear();
-  g_plans[k] = Plan{static_cast<int>(kind), static_cast<int>(n), reserve, static_cast<float>(scale_log2)};
+  g_plans[k] = Plan{static_cast<int>(kind), static_cast<int>(n), static_cast<float>(scale_log2)};
 }
 
 // A plain tensor (no subclass, wrapper or active mode that would have to see
@@ -339,7 +338,7 @@ py::object flash_attn(const py::handle& hq, const py::handle& hk, const py::hand
   hipStream_t stream = c10::hip::getCurrentHIPStream(dev).stream();
 
   void *ws = nullptr, *cnt = nullptr;
-  size_t need = static_cast<size_t>(p.reserve);
+  size_t need = 0;
   if (p.kind == kSplit || p.kind == kChunks)
     need = gqa_split_workspace_bytes(B, Hq, Sq, D, p.n);
   else if (p.kind == kFlat)

@@ -16,8 +16,8 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces, decode_forward, flat_forward, stream_handle,
-                        workspace_bytes)
+from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces, decode_forward,
+                        flat_forward, stream_handle)
 
 __all__ = ["gqa_flash_attn", "Route", "choose_route"]
 
@@ -203,10 +203,6 @@ class Route:
     splits: int = 1
     workgroups: int = 0
     fwd_split: int = 0  # single pass: query blocks per (b, kv head) run as two key halves
-    # short: bytes of stream workspace choose_route's route takes.  The short
-    # form uses none, but a call whose rows lie too far apart for it falls
-    # back to that route, so the stream's buffer is as large either way.
-    reserve: int = 0
 
 
 def _cdiv(a: int, b: int) -> int:
@@ -560,11 +556,6 @@ def choose_route(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_
     return Route("single", 1, single_wgs + ns * num_kv_heads * batch, ns)
 
 
-def _fwd_split_bytes(batch: int, num_kv_heads: int, head_dim: int, n_split: int) -> int:
-    """gqa_fwd_split_workspace_bytes: two fp32 states of 512 lanes x (D / 2 + 2) per split block."""
-    return batch * num_kv_heads * n_split * 2 * 512 * (head_dim // 2 + 2) * 4
-
-
 def flat_piece_steps(batch: int, seq_kv: int, slots: int, head_dim: int = 128) -> float:
     """Tile steps of a piece of a flat split over `slots` ranges: every range
     is one piece, and one more for each sequence that it crosses into."""
@@ -688,11 +679,7 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
             batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
             route.splits if route.kind == "chunks" else 0, route.fwd_split):
         wgs = _cdiv(seq_q, SHORT_ROWS // (num_heads // num_kv_heads)) * num_kv_heads * batch
-        if route.kind == "single":
-            need = _fwd_split_bytes(batch, num_kv_heads, head_dim, route.fwd_split)
-        else:
-            need = workspace_bytes(batch, num_heads, seq_q, head_dim, route.splits)
-        return Route("short", 1, wgs, reserve=need)
+        return Route("short", 1, wgs)
     if rows > split_max_rows(head_dim):
         return route
     rpw = split_rows_per_workgroup(rows, head_dim)
@@ -783,7 +770,7 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
     if host is not None and batch > 0 and seq_q > 0:
         host.set_plan([0, batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, int(bool(causal)), dev, 0, 0, 0],
                       _KIND_IDS[route.kind], route.fwd_split if route.kind == "single" else route.splits,
-                      route.reserve, (head_dim ** -0.5) * LOG2E)
+                      (head_dim ** -0.5) * LOG2E)
     if dev == torch.cuda.current_device():
         return _launch(route, q, k, v, causal, return_lse, dev)
     with torch.cuda.device(dev):  # launch on q's device
@@ -822,8 +809,6 @@ def _launch(route, q_in, k, v, causal, return_lse, dev):
     if route.kind == "chunks":
         return chunks_forward(q, k, v, o, causal, route.splits, return_lse)
     if route.kind == "short":
-        if route.reserve:
-            _workspace_buffer(q.device, stream_handle(q.device), route.reserve)
         return short_forward(q, k, v, o, causal, return_lse)
     return single_pass_forward(q, k, v, o, causal, route.fwd_split, return_lse)
 

@@ -506,7 +506,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
                 _lib.check(rc)
         if done:
             if host is not None and plan_key is not None:
-                host.set_plan(plan_key, _KIND_IDS["flat"], flat_slots, 0, 0.0)
+                host.set_plan(plan_key, _KIND_IDS["flat"], flat_slots, 0.0)
             return out if lse is None else (out, lse)
         plan_key = None  # refused for this call's strides
     if route == "short":
@@ -524,7 +524,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
         workspace = _workspace_buffer(qdev, stream, workspace_bytes(batch, num_heads, seq_q, head_dim, n_parts))
     if host is not None:
         if plan_key is not None:
-            host.set_plan(plan_key, _KIND_IDS[route], n_parts, 0, 0.0)
+            host.set_plan(plan_key, _KIND_IDS[route], n_parts, 0.0)
         host.paged_forward(_KIND_IDS[route], q, k_cache, v_cache, block_table, table_stride, seq_lens,
                            query_start if varlen else None, query_lens if varlen else None, max_seq_len, out, lse,
                            workspace, counters, n_parts, batch, seq_q, scale * LOG2E, bool(causal), dtype)

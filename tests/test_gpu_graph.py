@@ -72,20 +72,18 @@ def test_public_path_in_graph(case):
 
 
 def test_graph_workspace_outlives_growth():
-    """A decode graph keeps the raw address of the split workspace it was
-    captured with.  A later, larger call on the same stream (a 1024-token
-    prefill with the key split) replaces the stream's cached workspace; the
-    replaced buffer must stay allocated, or the decode replays would write
-    their partials into memory handed to other tensors.  Both calls warm up
-    eagerly on the capture stream (so the first workspace comes from the
-    general pool), the captures share one memory pool (vLLM's pattern), and
-    tensors allocated afterwards at the first workspace's size must keep
-    their contents across replays."""
+    """A decode graph has its partials in its own memory; a later, larger call
+    on the same stream (64 tokens over 16384 keys, in key chunks) replaces the
+    stream's cached workspace, and neither the replays nor the eager call see
+    the other's.  Both calls warm up eagerly on the capture stream, the
+    captures share one memory pool (vLLM's pattern), and tensors allocated
+    afterwards at the first workspace's size must keep their contents across
+    replays."""
     from gqa_kernels import gqa_flash_attn, gqa_split
-    from gqa_kernels.dispatch import _cu_count, choose_route
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     qd, kd, vd = make_inputs(1, 32, 8, 1, 16384, 128, torch.bfloat16, seed=31, device=DEV)
-    qp, kp, vp = make_inputs(1, 32, 8, 1024, 1024, 128, torch.bfloat16, seed=32, device=DEV)
-    assert choose_route(1, 32, 8, 1024, 1024, _cu_count(0)).fwd_split > 0
+    qp, kp, vp = make_inputs(1, 32, 8, 64, 16384, 128, torch.bfloat16, seed=32, device=DEV)
+    assert choose_plan(1, 32, 8, 64, 16384, _cu_count(0)).kind == "chunks"
     dec = lambda: gqa_flash_attn(qd, kd, vd, causal=True)
     pre = lambda: gqa_flash_attn(qp, kp, vp, causal=True)
     s = torch.cuda.Stream()

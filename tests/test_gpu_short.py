@@ -132,3 +132,17 @@ def test_short_rows_far_apart():
     far = big.as_strided((16, 8, 1100, 128), (8 * 128, 128, 900_000, 1))
     far.copy_(k)
     assert_close(gqa_flash_attn(q, far, v), gqa_flash_attn(q, k, v), BASELINE_TOL[torch.bfloat16], "far rows")
+
+
+def test_short_calls_hold_no_workspace():
+    from gqa_kernels import gqa_flash_attn, gqa_split
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    assert choose_plan(1, 32, 8, 1024, 1024, _cu_count(0)).kind == "short"
+    q, k, v = make_inputs(1, 32, 8, 1024, 1024, 128, torch.bfloat16, device=DEV)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        first, again = gqa_flash_attn(q, k, v), gqa_flash_attn(q, k, v)
+    torch.cuda.synchronize()
+    assert torch.equal(first, again)
+    assert (torch.cuda.current_device(), s.cuda_stream) not in gqa_split._workspaces

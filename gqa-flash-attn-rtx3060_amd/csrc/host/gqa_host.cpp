@@ -545,6 +545,81 @@ bool write_kv(const py::handle& hk, const py::handle& hv, const py::handle& hkc,
   return true;
 }
 
+// gqa_kernels.dispatch._list_makespan, step for step (its docstring describes
+// the schedules): runs of count[i] items of cost[i], repeated n_rep times.
+double list_makespan(const std::vector<double>& cost, const std::vector<int64_t>& count, int64_t n_rep, int64_t cu,
+                     bool persistent, int64_t dyn_min) {
+  if (cost.size() != count.size()) throw std::invalid_argument("list_makespan: one count per cost");
+  int64_t period = 0;
+  for (int64_t k : count) {
+    if (k < 0) throw std::invalid_argument("list_makespan: negative count");
+    period += k;
+  }
+  const int64_t total = period * n_rep;
+  if (total <= 0) return 0.0;
+  const int64_t n_wg = std::min(total, cu), q = total / 8, r = total % 8;
+  const bool fixed = persistent && total < dyn_min * n_wg;
+  const size_t n = static_cast<size_t>(std::max<int64_t>(1, cu / 8));
+  std::vector<double> flat, loads;
+  if (fixed)
+    for (size_t i = 0; i < cost.size(); ++i) flat.insert(flat.end(), static_cast<size_t>(count[i]), cost[i]);
+  std::vector<std::array<int64_t, 3>> seen;
+  double worst = 0.0;
+  for (int64_t x = 0; x < 8; ++x) {
+    const int64_t lo = (x * q + std::min(x, r)) % period, cnt = q + (x < r ? 1 : 0), slots = (n_wg - x + 7) >> 3;
+    const std::array<int64_t, 3> key{lo, cnt, fixed ? slots : 0};
+    if (cnt == 0 || std::find(seen.begin(), seen.end(), key) != seen.end()) continue;
+    seen.push_back(key);
+    if (fixed) {
+      // Rows of `slots` items dealt left to right, the odd ones right to left.
+      loads.assign(static_cast<size_t>(slots), 0.0);
+      for (int64_t e = 0; e < cnt; ++e) {
+        const int64_t row = e / slots, at = e % slots;
+        loads[static_cast<size_t>(row & 1 ? slots - 1 - at : at)] += flat[static_cast<size_t>((lo + e) % period)];
+      }
+      worst = std::max(worst, *std::max_element(loads.begin(), loads.end()));
+      continue;
+    }
+    // Each item to the least loaded CU; `loads` ascending.  A run on loads
+    // within its cost of each other goes round by round.
+    loads.assign(n, 0.0);
+    size_t i = 0;
+    int64_t off = lo;
+    while (off >= count[i]) off -= count[i++];
+    for (int64_t left = cnt; left > 0;) {
+      const double c = cost[i];
+      int64_t k = std::min(count[i] - off, left);
+      left -= k;
+      // (A run goes on over the end of the period, as _slice_runs joins them.)
+      for (;;) {
+        i = (i + 1) % cost.size();
+        off = 0;
+        if (left <= 0 || cost[i] != c) break;
+        const int64_t more = std::min(count[i], left);
+        k += more;
+        left -= more;
+      }
+      while (k > 0) {
+        if (loads.back() - loads.front() <= c) {
+          const int64_t full = k / static_cast<int64_t>(n), rem = k % static_cast<int64_t>(n);
+          if (full > 0)
+            for (double& l : loads) l += static_cast<double>(full) * c;
+          for (int64_t j = 0; j < rem; ++j) loads[static_cast<size_t>(j)] += c;
+          std::rotate(loads.begin(), loads.begin() + rem, loads.end());
+          break;
+        }
+        const double l = loads.front() + c;
+        const auto to = std::upper_bound(loads.begin() + 1, loads.end(), l);
+        std::move(loads.begin() + 1, to, loads.begin());
+        *(to - 1) = l;
+        --k;
+      }
+    }
+    worst = std::max(worst, loads.back());
+  }
+  return worst;
+}
+
 // Host ints to an int32 tensor on `device` in one asynchronous copy from
 // pinned memory (the caching host allocator keeps the pinned block until the
 // copy has run).
@@ -577,6 +652,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attn", &paged_attn, "paged_attention of a planned shape on its default route, or None");
   m.def("write_kv", &write_kv, "write_kv with its checks, or False");
   m.def("set_plan", &set_plan, "register the route of a shape");
+  m.def("list_makespan", &list_makespan, "run time of a list of items over the CUs (the routing models)");
   m.def("ints_to_device", &ints_to_device, "host ints to an int32 device tensor, asynchronously");
   m.attr("ABI_VERSION") = gqa_abi_version();
 }

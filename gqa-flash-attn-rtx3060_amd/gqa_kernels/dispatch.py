@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import bisect
 import functools
+import itertools
 import math
 from dataclasses import dataclass
 
@@ -211,13 +212,12 @@ def _cdiv(a: int, b: int) -> int:
 
 def _fwd_block_tiles(n_mblk: int, block_m: int, seq_q: int, seq_kv: int, causal: bool):
     """Key tiles of each single-pass query block (gqa_fwd.hip's key range)."""
-    out = []
-    for pid in range(n_mblk):
-        kv_end = seq_kv
-        if causal:
-            pos_hi = min((pid + 1) * block_m, seq_q) - 1
-            kv_end = min(seq_kv, pos_hi + (seq_kv - seq_q) + 1)
-        out.append(_cdiv(max(kv_end, 0), FWD_TILE))
+    if not causal:
+        return [max(0, _cdiv(seq_kv, FWD_TILE))] * n_mblk
+    off = seq_kv - seq_q + FWD_TILE - 1  # a block's last position + 1 sees that many keys more, rounded up to tiles
+    out = [max(0, (pid * block_m + off) // FWD_TILE) for pid in range(1, n_mblk)]
+    if n_mblk > 0:
+        out.append(max(0, (min(n_mblk * block_m, seq_q) + off) // FWD_TILE))
     return out
 
 
@@ -232,26 +232,27 @@ def fwd_split_makespan(tiles, n_split: int, n_bh: int, cu_count: int, causal: bo
     `dealt`: its pairs are dealt to the XCDs, which take theirs side by
     side)."""
     n = len(tiles)
-    order = list(range(n - 1, -1, -1)) if causal else list(range(n))
     mo = FWD_MERGE_OVERHEAD if persistent else 0
     if not causal and n_split > 0:
         # (Pairs dealt to the XCDs: every XCD takes its pairs' items side by side.)
         per_xcd = n_bh // 8 if n_bh % 8 == 0 else 1
-        mo = FWD_MERGE_OVERHEAD if persistent else FWD_FILL_MERGE_OVERHEAD
-        runs = []
-        for pid in range(n - n_split):
-            _push_run(runs, tiles[pid] + FWD_ITEM_OVERHEAD, per_xcd)
+        mo = (FWD_MERGE_OVERHEAD if persistent else FWD_FILL_MERGE_OVERHEAD) + FWD_ITEM_OVERHEAD
+        items = [t + FWD_ITEM_OVERHEAD for t in tiles[:n - n_split]]
         for half in (1, 0):
-            for pid in range(n - 1, n - n_split - 1, -1):
-                _push_run(runs, (tiles[pid] + half) // 2 + mo + FWD_ITEM_OVERHEAD, per_xcd)
-        return _list_makespan(runs, n_bh // per_xcd, cu_count, persistent)
-    items = [tiles[n - 1 - i] - tiles[n - 1 - i] // 2 + mo for i in range(n_split)]
-    for pid in order:
-        items.append(tiles[pid] // 2 + mo if pid >= n - n_split else tiles[pid])
-    per_xcd = n_bh // 8 if dealt and n_bh % 8 == 0 else 1
-    runs = []
-    for c in items:
-        _push_run(runs, c + FWD_ITEM_OVERHEAD, per_xcd)
+            items += [(t + half) // 2 + mo for t in reversed(tiles[n - n_split:])]
+    else:
+        per_xcd = n_bh // 8 if dealt and n_bh % 8 == 0 else 1
+        lo = FWD_ITEM_OVERHEAD
+        whole = [t + lo for t in tiles[:n - n_split]]
+        mo += lo
+        halves = [t // 2 + mo for t in tiles[n - n_split:]]
+        items = [t - t // 2 + mo for t in reversed(tiles[n - n_split:])] if n_split else []
+        items += (whole + halves)[::-1] if causal else whole + halves
+    host = _lib._host
+    if host is not None:
+        return host.list_makespan(items, [per_xcd] * len(items), n_bh // per_xcd, cu_count, persistent,
+                                  FWD_DYN_MIN_ITEMS_PER_WG)
+    runs = [[c, per_xcd * len(list(k))] for c, k in itertools.groupby(items)]
     return _list_makespan(runs, n_bh // per_xcd, cu_count, persistent)
 
 
@@ -316,7 +317,13 @@ def _list_makespan(runs, n_rep: int, cu_count: int, persistent: bool = False) ->
     Otherwise (the dynamic schedule, or one workgroup per item) each CU
     takes the next item when free.  XCD shares with the same start within
     the period and the same length are scheduled once (with 8 kv heads
-    every XCD's share is the same list)."""
+    every XCD's share is the same list).  Natively once the bindings are
+    loaded (gqa_host.cpp, the same steps: a plan of a new shape asks for about
+    twenty of these, 0.4 ms in Python)."""
+    host = _lib._host
+    if host is not None:
+        return host.list_makespan([c for c, _ in runs], [k for _, k in runs], n_rep, cu_count, persistent,
+                                  FWD_DYN_MIN_ITEMS_PER_WG)
     period = sum(k for _, k in runs)
     total = period * n_rep
     if total == 0:
@@ -456,9 +463,13 @@ def choose_fwd_split(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     if n_mblk * n_bh < FWD_SPLIT_MAX_WG_PER_CU * cu_count:
         tiles = _fwd_block_tiles(n_mblk, block_m, seq_q, seq_kv, causal)
         base = fwd_split_makespan(tiles, 0, n_bh, cu_count, persistent=persistent, dealt=dealt)
-        best, best_ns = base, 0
+        best, best_ns, last = base, 0, 0
         for f in (0.1, 0.15, 0.2, 0.25, 0.375, 0.5, 0.625, 0.75, 1.0):
             ns = max(1, min(n_mblk, round(n_mblk * f)))
+            # (No shorter than its longest item: the heaviest whole block.)
+            if ns == last or (ns < n_mblk and tiles[n_mblk - 1 - ns] + FWD_ITEM_OVERHEAD >= best):
+                continue
+            last = ns
             t = fwd_split_makespan(tiles, ns, n_bh, cu_count, persistent=persistent, dealt=dealt)
             if t < best:
                 best, best_ns = t, ns
@@ -534,6 +545,12 @@ def choose_route(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_
     split-KV combine (choose_kv_chunks, route kind "chunks") when the model
     says that is faster.
     """
+    return _choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim, False)
+
+
+def _choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim, dealt) -> Route:
+    """choose_route; `dealt`: a single pass's split blocks by the model of
+    dealt pairs (choose_plan)."""
     group = num_heads // num_kv_heads
     rows = group * seq_q
     single_wgs = _cdiv(seq_q, max(1, FWD_ROWS // group)) * num_kv_heads * batch
@@ -542,17 +559,22 @@ def choose_route(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_
         base = _cdiv(rows, rpw) * num_kv_heads * batch
         splits = split_count(base, seq_kv, cu_count, rpw, head_dim, rows16=rows <= DEC16_ROWS)
         return Route("split", splits, base * splits)
-    ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
     # Key chunks, against the better of the plain and the block-split single pass.
     # (Only from SPLIT_MIN_KV keys on, the length from which the reference
     # splits the key axis at all.)
     n_mblk = _cdiv(seq_q, max(1, FWD_ROWS // group))
-    if n_mblk * num_kv_heads * batch < cu_count and seq_q > 0 and seq_kv >= SPLIT_MIN_KV:
+    chunked = n_mblk * num_kv_heads * batch < cu_count and seq_q > 0 and seq_kv >= SPLIT_MIN_KV
+    ns = 0
+    if chunked or not dealt:
+        ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
+    if chunked:
         tiles = _fwd_block_tiles(n_mblk, max(1, FWD_ROWS // group), seq_q, seq_kv, causal)
         base = fwd_split_makespan(tiles, ns, num_kv_heads * batch, cu_count, causal, persistent=head_dim == 128)
         kc = choose_kv_chunks(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim, base)
         if kc:
             return Route("chunks", kc, single_wgs * kc)
+    if dealt:
+        ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim, dealt=True)
     return Route("single", 1, single_wgs + ns * num_kv_heads * batch, ns)
 
 
@@ -667,21 +689,18 @@ def choose_plan(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, seq_k
       pair after pair: 2 x 1536 tokens 54.3 -> 45.4 us, 4 x 768 36.3 -> 28.9.
     * Batches that no power-of-two split count spreads evenly over the
       compute units take the flat split (FLAT_MIN_USED, FLAT_MIN_PIECE)."""
-    route = choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim)
     rows = num_heads // num_kv_heads * seq_q
-    if rows <= 0 or seq_kv <= 0 or batch <= 0:
-        return route
-    n_bh = batch * num_kv_heads
-    if route.kind == "single" and causal and head_dim == 128 and _dealt(n_bh):
-        ns = choose_fwd_split(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, True, dealt=True)
-        route = Route("single", 1, route.workgroups + (ns - route.fwd_split) * n_bh, ns)
-    if rows > flat_max_rows(head_dim) and use_short(
-            batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
-            route.splits if route.kind == "chunks" else 0, route.fwd_split):
-        wgs = _cdiv(seq_q, SHORT_ROWS // (num_heads // num_kv_heads)) * num_kv_heads * batch
-        return Route("short", 1, wgs)
-    if rows > split_max_rows(head_dim):
-        return route
+    if not 0 < rows <= flat_max_rows(head_dim) or seq_kv <= 0 or batch <= 0:
+        route = _choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
+                              causal and head_dim == 128 and _dealt(batch * num_kv_heads))
+        if rows <= 0 or seq_kv <= 0 or batch <= 0:
+            return route
+        if use_short(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causal, head_dim,
+                     route.splits if route.kind == "chunks" else 0, route.fwd_split):
+            wgs = _cdiv(seq_q, SHORT_ROWS // (num_heads // num_kv_heads)) * num_kv_heads * batch
+            return Route("short", 1, wgs)
+        if rows > split_max_rows(head_dim):
+            return route
     rpw = split_rows_per_workgroup(rows, head_dim)
     base = _cdiv(rows, rpw) * num_kv_heads * batch
     splits = split_count(base, seq_kv, cu_count, rpw, head_dim, rows16=rows <= DEC16_ROWS)
@@ -765,12 +784,15 @@ def gqa_flash_attn(q, k, v, causal=True, *, return_lse=False):
     dev = q.get_device()  # device index (an int: no torch.device objects on this path)
     assert k.get_device() == dev and v.get_device() == dev, "q, k, v must be on one device"
 
-    route = _plan_cached(batch, num_heads, num_kv_heads, seq_q, seq_kv, _cu_count(dev), bool(causal), head_dim)
     host = _decode_host()
+    route = _plan_cached(batch, num_heads, num_kv_heads, seq_q, seq_kv, _cu_count(dev), bool(causal), head_dim)
     if host is not None and batch > 0 and seq_q > 0:
         host.set_plan([0, batch, num_heads, num_kv_heads, seq_q, seq_kv, head_dim, int(bool(causal)), dev, 0, 0, 0],
                       _KIND_IDS[route.kind], route.fwd_split if route.kind == "single" else route.splits,
                       (head_dim ** -0.5) * LOG2E)
+        out = host.flash_attn(q, k, v, bool(causal), bool(return_lse), _workspaces, _counters)
+        if out is not None:
+            return out
     if dev == torch.cuda.current_device():
         return _launch(route, q, k, v, causal, return_lse, dev)
     with torch.cuda.device(dev):  # launch on q's device

@@ -441,7 +441,7 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
     if splits is None and route in (None, "split"):
         flat_slots = paged_flat_slots(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
                                       head_dim, interleaved)
-    if splits is None:
+    if splits is None and (not flat_slots or max_seq_len > 1 << 20):  # (only there can it refuse the call)
         splits = paged_splits(batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size,
                               head_dim, interleaved)
     if scale is None:
@@ -483,10 +483,19 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), causal, head_dim))
     assert route in ("split", "single", "chunks", "short")
     assert route == "split" or block_size >= single_pass_min_block(head_dim)
+    flat = route == "split" and flat_slots > 0
+    n_parts = {"short": 0, "single": fwd_split, "chunks": kv_chunks, "split": splits}[route]
+    host = _paged_host()
+    if host is not None and plan_key is not None:
+        host.set_plan(plan_key, _KIND_IDS["flat" if flat else route], flat_slots if flat else n_parts, 0.0)
+        res = host.paged_attn(q, k_cache, v_cache, block_table, seq_lens, bool(causal), max_seq_len, scale * LOG2E,
+                              bool(return_lse), out, query_start, query_lens if varlen else None,
+                              seq_q if varlen else -1, _workspaces, _counters)
+        if res is not None:
+            return res
     lse = torch.empty(lse_shape, dtype=torch.float32, device=qdev) if return_lse else None
     counters = None
-    host = _paged_host()
-    if route == "split" and flat_slots:
+    if flat:
         workspace = _workspace_buffer(qdev, stream, flat_workspace_bytes(batch, num_heads, seq_q, head_dim, flat_slots))
         if host is not None:
             done = host.paged_forward(_KIND_IDS["flat"], q, k_cache, v_cache, block_table, table_stride, seq_lens,
@@ -505,26 +514,21 @@ def paged_attention(q, k_cache, v_cache, block_table, seq_lens, causal=True, *,
             if done:
                 _lib.check(rc)
         if done:
-            if host is not None and plan_key is not None:
-                host.set_plan(plan_key, _KIND_IDS["flat"], flat_slots, 0.0)
             return out if lse is None else (out, lse)
-        plan_key = None  # refused for this call's strides
+        n_parts = splits if splits is not None else paged_splits(
+            batch, num_heads, num_kv_heads, seq_q, max_seq_len, _cu_count(dev), block_size, head_dim, interleaved)
     if route == "short":
-        n_parts, workspace = 0, None
+        workspace = None
     elif route == "single":
         # Split query blocks: their halves' fp32 state and the stream's
         # zeroed merge counters (left zero by the kernel).
-        n_parts = fwd_split
         workspace = None if not fwd_split else _workspace_buffer(
             qdev, stream, lib.gqa_fwd_split_workspace_bytes(batch, num_kv_heads, head_dim, fwd_split))
         if fwd_split:
             counters = _counter_buffer(qdev, stream, lib.gqa_fwd_split_counters_count(batch, num_kv_heads, fwd_split))
     else:
-        n_parts = kv_chunks if route == "chunks" else splits
         workspace = _workspace_buffer(qdev, stream, workspace_bytes(batch, num_heads, seq_q, head_dim, n_parts))
     if host is not None:
-        if plan_key is not None:
-            host.set_plan(plan_key, _KIND_IDS[route], n_parts, 0.0)
         host.paged_forward(_KIND_IDS[route], q, k_cache, v_cache, block_table, table_stride, seq_lens,
                            query_start if varlen else None, query_lens if varlen else None, max_seq_len, out, lse,
                            workspace, counters, n_parts, batch, seq_q, scale * LOG2E, bool(causal), dtype)

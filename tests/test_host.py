@@ -541,6 +541,27 @@ def test_head_split_at_head_dim_64(batch, seq_q, seq_kv, split):
     assert plan.kind != "single" or plan.fwd_split == split
 
 
+def test_native_makespan_equals_python(monkeypatch):
+    """The routing models' schedules in C++ against the Python that states them,
+    and whole plans with and without the bindings."""
+    import random
+    from gqa_kernels import _lib, dispatch
+    host = _lib.load_host()
+    rng = random.Random(7)
+    shapes = [(b, 32, 8, s, s + e, 256, c, d) for b in (1, 2, 5, 16) for s in (40, 333, 1100, 2500)
+              for e in (0, 3000) for c in (True, False) for d in (64, 128)]
+    for _ in range(400):
+        runs = [[float(rng.choice((8, 9, 12, 40.5, 64))), rng.randint(1, 40)] for _ in range(rng.randint(1, 30))]
+        args = (rng.choice((1, 2, 8, 12, 64)), rng.choice((64, 256, 304)), rng.random() < 0.5)
+        monkeypatch.setattr(_lib, "_host", None)
+        want = dispatch._list_makespan(runs, *args)
+        monkeypatch.setattr(_lib, "_host", host)
+        assert dispatch._list_makespan(runs, *args) == want, (runs, args)
+    native = [dispatch.choose_plan(*s) for s in shapes]
+    monkeypatch.setattr(_lib, "_host", None)
+    assert [dispatch.choose_plan(*s) for s in shapes] == native
+
+
 def test_fwd_split_launch_validation(lib):
     f = lib.gqa_fwd_split_launch
     args = lambda lse, ws, cnt, ns: (_FAKE, _S4, _FAKE, _S4, _FAKE, _S4, _FAKE, _S4, lse, ws, cnt, ns,

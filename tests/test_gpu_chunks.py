@@ -88,8 +88,8 @@ def test_chunks_route_long_cache():
     # A 128-token chunk of Llama-3.1-8B attention against 131072 keys: the
     # route takes key chunks; checked against fp32 torch attention on the GPU.
     from gqa_kernels import gqa_flash_attn
-    from gqa_kernels.dispatch import _cu_count, choose_route
-    route = choose_route(1, 32, 8, 128, 131072, _cu_count(0))
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    route = choose_plan(1, 32, 8, 128, 131072, _cu_count(0))
     assert route.kind == "chunks", route
     q, k, v = make_inputs(1, 32, 8, 128, 131072, 128, torch.bfloat16, seed=9, device=DEV)
     print(f"chunks route {route}", flush=True)

@@ -92,8 +92,8 @@ def test_decode_wide_row_blocks_route_and_repeatability():
     # route, 64-row workgroups): oracle parity, and the same bits on every
     # call (fixed combine order).
     from gqa_kernels import gqa_flash_attn
-    from gqa_kernels.dispatch import _cu_count, choose_route
-    assert choose_route(2, 32, 8, 16, 20000, _cu_count(0)).kind == "split"
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    assert choose_plan(2, 32, 8, 16, 20000, _cu_count(0)).kind == "split"
     q, k, v = make_inputs(2, 32, 8, 16, 20000, 128, torch.bfloat16, seed=16, device=DEV)
     o = gqa_flash_attn(q, k, v, causal=True)
     for _ in range(3):

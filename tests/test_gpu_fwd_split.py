@@ -36,14 +36,14 @@ def _rows(sq, n=96):
                                      np.arange(max(0, sq - 16), sq)]))
 
 
-@pytest.mark.parametrize("S", [512, 1024, 2048])
-def test_auto_split_prefill_matches_oracle(S):
+@pytest.mark.parametrize("B,S", [(1, 2300), (1, 2500), (2, 1025)])
+def test_auto_split_prefill_matches_oracle(B, S):
     from gqa_kernels import gqa_flash_attn
-    from gqa_kernels.dispatch import _cu_count, choose_route
-    route = choose_route(1, 32, 8, S, S, _cu_count(0), True)
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    route = choose_plan(B, 32, 8, S, S, _cu_count(0), True)
     assert route.kind == "single" and route.fwd_split > 0, route
-    q, k, v = make_inputs(1, 32, 8, S, S, 128, torch.bfloat16, seed=S, device=DEV)
-    print(f"auto split S={S} n_split={route.fwd_split}", flush=True)
+    q, k, v = make_inputs(B, 32, 8, S, S, 128, torch.bfloat16, seed=S, device=DEV)
+    print(f"auto split B={B} S={S} n_split={route.fwd_split}", flush=True)
     o, lse = gqa_flash_attn(q, k, v, causal=True, return_lse=True)
     torch.cuda.synchronize()
     rows = _rows(S)

@@ -57,12 +57,15 @@ def _replays(g, out, expect, n=4):
 def test_public_path_in_graph(case):
     from gqa_kernels import gqa_flash_attn
     shapes = {"decode": (1, 32, 8, 1, 16384), "decode_lse": (2, 32, 8, 1, 5000),
-              "prefill": (1, 32, 8, 4096, 4096), "prefill_split": (1, 32, 8, 1024, 1024),
+              "prefill": (1, 32, 8, 4096, 4096), "prefill_split": (1, 32, 8, 2300, 2300),
               "chunked": (2, 32, 8, 256, 3000)}
     B, Hq, Hkv, Sq, Skv = shapes[case]
     q, k, v = make_inputs(B, Hq, Hkv, Sq, Skv, 128, torch.bfloat16, seed=len(case), device=DEV)
     lse = case == "decode_lse"
     print(f"graph {case}", flush=True)
+    if case == "prefill_split":
+        from gqa_kernels.dispatch import _cu_count, choose_plan
+        assert choose_plan(*shapes[case], _cu_count(0)).fwd_split > 0
     fn = lambda: gqa_flash_attn(q, k, v, causal=True, return_lse=lse)
     expect = fn()
     torch.cuda.synchronize()
@@ -145,14 +148,17 @@ def test_paged_decode_in_graph():
 
 
 @pytest.mark.parametrize("shape", [(4, 32, 8, 4096, 4096),   # 2048 items: the dynamic schedule's queues
-                                   (1, 32, 8, 1024, 1024)])  # key-split blocks: the merge counters
+                                   (1, 32, 8, 2300, 2300)])  # key-split blocks: the merge counters
 def test_two_graphs_replayed_concurrently(shape):
     # Two prefills captured into two graphs (on torch's one capture stream),
     # then replayed at the same time on two streams: each captured call has
     # its own counters (queue and merge counters that the kernel leaves
     # zero), so neither replay sees the other's claims.
     from gqa_kernels import gqa_flash_attn
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     b, hq, hkv, sq, skv = shape
+    plan = choose_plan(*shape, _cu_count(0))
+    assert plan.kind == "single" and (plan.fwd_split > 0) == (b == 1)
     print(f"two graphs concurrently {shape}", flush=True)
     ins = [make_inputs(b, hq, hkv, sq, skv, 128, torch.bfloat16, seed=s, device=DEV) for s in (1, 2)]
     expect = [gqa_flash_attn(*x, causal=True) for x in ins]

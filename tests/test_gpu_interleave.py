@@ -45,10 +45,16 @@ def _kinds():
     from gqa_kernels.paged import paged_attention
     from test_gpu_paged import _check, _paged_inputs
 
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     kinds = {}
 
     def contiguous(name, B, Hq, Hkv, Sq, Skv, D, causal, lse=False, rows=None):
         q, k, v = make_inputs(B, Hq, Hkv, Sq, Skv, D, seed=Sq + Skv + D, device=DEV)
+        plan = choose_plan(B, Hq, Hkv, Sq, Skv, _cu_count(0), causal, D)
+        for word, holds in (("key-split", plan.fwd_split > 0), ("chunks", plan.kind == "chunks"),
+                            ("dynamic", plan.kind == "single"), ("short", plan.kind == "short"),
+                            ("decode", plan.kind == "split")):
+            assert word not in name or holds, (name, plan)
 
         def call():
             r = gqa_flash_attn(q, k, v, causal=causal, return_lse=lse)
@@ -67,10 +73,13 @@ def _kinds():
 
     # Single pass with key-split blocks (merge counters), persistent kernel
     # with the dynamic schedule (queue counters), key chunks + combine, LSE.
-    contiguous("prefill 2048 key-split", 1, 32, 8, 2048, 2048, 128, True, rows=np.arange(1800, 2048))
+    contiguous("prefill 2300 key-split", 1, 32, 8, 2300, 2300, 128, True, rows=np.arange(2050, 2300))
     contiguous("prefill B=8 4096 dynamic", 8, 32, 8, 4096, 4096, 128, True, rows=np.arange(4000, 4096))
     contiguous("chunks 128 x 16384", 1, 32, 8, 128, 16384, 128, True)
-    contiguous("prefill 1024 head_dim 64 lse", 1, 32, 8, 1024, 1024, 64, True, lse=True)
+    contiguous("prefill 2200 head_dim 64 key-split lse", 1, 32, 8, 2200, 2200, 64, True, lse=True,
+               rows=np.arange(1950, 2200))
+    # The short form, which keeps nothing between calls.
+    contiguous("prefill 1024 short lse", 1, 32, 8, 1024, 1024, 128, True, lse=True)
     contiguous("non-causal chunks 300 x 5000", 1, 32, 8, 300, 5000, 128, False)
     # Split-KV decode (cached workspace), verify step, head_dim 64.
     contiguous("decode 8192", 1, 32, 8, 1, 8192, 128, True)

@@ -33,9 +33,9 @@ def _lse_err(lse, q, k, v, causal=True):
 
 
 def _route(q, k):
-    from gqa_kernels.dispatch import _cu_count, choose_route
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     B, Hq, Sq, _ = q.shape
-    return choose_route(B, Hq, k.shape[1], Sq, k.shape[2], _cu_count(0))
+    return choose_plan(B, Hq, k.shape[1], Sq, k.shape[2], _cu_count(0))
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,dtype,causal", [

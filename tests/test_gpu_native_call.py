@@ -47,8 +47,18 @@ def _python_only(monkeypatch):
     monkeypatch.setattr(_lib, "_host", Bindings(_lib._host))
 
 
-SHAPES = [(1, 32, 8, 1, 3000, 128), (5, 32, 8, 1, 2000, 128), (64, 32, 8, 1, 300, 64), (2, 32, 8, 150, 150, 128),
-          (1, 32, 8, 64, 5000, 128), (2, 8, 2, 3000, 3000, 64)]
+# split, flat, flat with one slot per sequence, short, chunks, single with and
+# without split blocks
+SHAPES = [(1, 32, 8, 1, 3000, 128), (5, 32, 8, 1, 4000, 128), (64, 32, 8, 1, 300, 64), (2, 32, 8, 150, 150, 128),
+          (1, 32, 8, 64, 5000, 128), (2, 8, 2, 3000, 3000, 64), (2, 32, 8, 1100, 1100, 128)]
+
+
+def test_shapes_cover_the_kinds():
+    from gqa_kernels.dispatch import _KIND_IDS, _cu_count, choose_plan
+    plans = [choose_plan(*s[:5], _cu_count(0), True, s[5]) for s in SHAPES]
+    assert {p.kind for p in plans} == set(_KIND_IDS)
+    assert {p.fwd_split > 0 for p in plans if p.kind == "single"} == {True, False}
+    assert {p.splits == s[0] for p, s in zip(plans, SHAPES) if p.kind == "flat"} == {True, False}
 
 
 @pytest.mark.parametrize("shape", SHAPES)
@@ -71,7 +81,7 @@ def test_other_stream_and_capture():
     """A stream without buffers falls to Python, which makes them; a captured
     call replays to the eager bits."""
     from gqa_kernels import gqa_flash_attn
-    for shape in SHAPES[:4]:
+    for shape in SHAPES:
         q, k, v = make_inputs(*shape, torch.bfloat16, seed=2, device=DEV)
         want = gqa_flash_attn(q, k, v)
         s = torch.cuda.Stream()
@@ -111,33 +121,83 @@ def test_refused_and_python_calls():
             gqa_flash_attn(*args)
 
 
-@pytest.mark.parametrize("lens,sq", [([300, 40, 1000], 1), ([2000], 1), ([300, 200], 150), ([3000, 3000], 40),
-                                     ([900, 30], 12)])
-def test_paged_same_bits(lens, sq, monkeypatch):
-    from gqa_kernels.paged import paged_attention, write_kv
+# (lengths, query tokens, keyword arguments, kind): the flat split, the fixed
+# count, the short form, key chunks, the single pass without and with split
+# blocks.
+PAGED = [([6000, 40, 2000, 1000, 700, 2500], 1, "flat"), ([2000], 1, "split"), ([300, 200], 150, "short"),
+         ([3000, 3000], 40, "chunks"), ([700, 650, 600, 500], 400, "single"), ([2000, 1500, 1999, 30] * 2, 300, "halves")]
+
+
+def _paged_kind(lens, sq):
+    from gqa_kernels.dispatch import _cu_count
+    from gqa_kernels.paged import paged_flat_slots, paged_route, paged_short, paged_single_plan
+    args = (len(lens), 32, 8, sq, max(lens), _cu_count(0))
+    if paged_short(*args, True, 16):
+        return "short"
+    if paged_route(32, 8, sq, 16) == "split":
+        return "flat" if paged_flat_slots(*args, 16, 128, True) else "split"
+    chunks, halves = paged_single_plan(*args)
+    return "chunks" if chunks else "halves" if halves else "single"
+
+
+def _native_paged(q, kc, vc, table, seq_lens, max_seq_len, lse, out=None, qs=None, ql=None, max_query_len=-1):
+    from gqa_kernels import _lib, gqa_split
+    return _lib._host.paged_attn(q, kc, vc, table, seq_lens, True, max_seq_len, 128 ** -0.5 * gqa_split.LOG2E, lse, out,
+                                 qs, ql, max_query_len, gqa_split._workspaces, gqa_split._counters)
+
+
+@pytest.mark.parametrize("lse", [False, True])
+@pytest.mark.parametrize("varlen", [False, True])
+@pytest.mark.parametrize("lens,sq,kind", PAGED)
+def test_paged_same_bits(lens, sq, kind, varlen, lse, monkeypatch):
+    """The native call of a planned shape, asked for directly, gives the bits and
+    the layout of the Python path; token-major queries of unequal counts too."""
+    from gqa_kernels.paged import paged_attention
+    assert _paged_kind(lens, sq) == kind
     q, kc, vc, table, seq_lens = (t.to(DEV) for t in _paged_inputs(len(lens), 32, 8, sq, lens, 128, 16, torch.bfloat16,
                                                                    seed=4))
+    kw, native_kw = {}, {}
+    if varlen:
+        n = [max(0, sq - 3 * b) if b != 1 else sq for b in range(len(lens))]
+        ql = torch.tensor(n, dtype=torch.int32, device=DEV)
+        qs = torch.tensor([sum(n[:b]) for b in range(len(n))], dtype=torch.int32, device=DEV)
+        q = torch.cat([q[b, :, :m].transpose(0, 1) for b, m in enumerate(n)]).contiguous()
+        kw = dict(query_start=qs, query_lens=ql, max_query_len=sq)
+        native_kw = dict(qs=qs, ql=ql, max_query_len=sq)
+    mx = max(lens)
+    with monkeypatch.context() as m:
+        _python_only(m)
+        ref = paged_attention(q, kc, vc, table, seq_lens, max_seq_len=mx, return_lse=lse, **kw)
+    out = torch.empty_like(q)
+    for o in (None, out):
+        native = _native_paged(q, kc, vc, table, seq_lens, mx, lse, o, **native_kw)
+        assert native is not None, "the native call did not take a planned shape"
+        for a, b in zip(native if lse else (native,), ref if lse else (ref,)):
+            assert torch.equal(torch.nan_to_num(a.float()), torch.nan_to_num(b.float()))
+            assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype
+    assert (native[0] if lse else native).data_ptr() == out.data_ptr()
+
+
+def test_write_kv_same_bytes_and_refused_paged_calls(monkeypatch):
+    from gqa_kernels import _lib
+    from gqa_kernels.paged import paged_attention, write_kv
+    lens = [300, 40, 1000]
+    q, kc, vc, table, seq_lens = (t.to(DEV) for t in _paged_inputs(3, 32, 8, 1, lens, 128, 16, torch.bfloat16, seed=4))
     new = torch.randn(3, 8, 128, device=DEV).to(torch.bfloat16)
     slots = torch.tensor([int(table[0, 0]) * 16 + 5, -1, int(table[0, 0]) * 16 + 6], device=DEV)
-    results = []
-    for python in (True, False, False):
-        with monkeypatch.context() as m:
-            if python:
-                _python_only(m)
-            k2, v2 = kc.clone(), vc.clone()
-            write_kv(new, new, k2, v2, slots)
-            o = torch.empty_like(q)
-            res = paged_attention(q, k2, v2, table, seq_lens, max_seq_len=max(lens), return_lse=True, out=o)
-            assert res[0].data_ptr() == o.data_ptr()
-            results.append((k2, v2, *res))
-    for other in results[1:]:
-        for a, b in zip(results[0], other):
-            assert torch.equal(torch.nan_to_num(a.float()), torch.nan_to_num(b.float()))
+    k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    with monkeypatch.context() as m:
+        _python_only(m)
+        write_kv(new, new, k1, v1, slots)
+    assert _lib._host.write_kv(new, new, k2, v2, slots) is True
+    for a, b in ((k1, k2), (v1, v2)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    paged_attention(q, kc, vc, table, seq_lens, max_seq_len=1000)
     for bad in (dict(max_seq_len=10 ** 6), dict(out=torch.empty(1, device=DEV))):
         with pytest.raises(AssertionError):
             paged_attention(q, kc, vc, table, seq_lens, **bad)
     with pytest.raises(AssertionError):
-        paged_attention(q, kc, vc, table.long(), seq_lens, max_seq_len=max(lens))
+        paged_attention(q, kc, vc, table.long(), seq_lens, max_seq_len=1000)
 
 
 def test_strides_of_one_call_do_not_plan_the_shape():

@@ -32,10 +32,11 @@ def _attn():
     return gqa_flash_attn
 
 
-def _route(q, k):
-    from gqa_kernels.dispatch import _cu_count, choose_route
-    B, Hq, Sq, _ = q.shape
-    return choose_route(B, Hq, k.shape[1], Sq, k.shape[2], _cu_count(0))
+def _route(q, k, causal=True):
+    """What gqa_flash_attn launches for these tensors."""
+    from gqa_kernels.dispatch import _cu_count, choose_plan
+    B, Hq, Sq, D = q.shape
+    return choose_plan(B, Hq, k.shape[1], Sq, k.shape[2], _cu_count(0), causal, D)
 
 
 def _run(q, k, v, causal=True):
@@ -74,10 +75,10 @@ def test_chunked_prefill(seq_q, seq_kv):
 # --------------------------------------------------------------------------
 # BASELINE configs, N(0,1) inputs.
 # --------------------------------------------------------------------------
-@pytest.mark.parametrize("seq", [2048, 4096])
-def test_baseline_prefill_full(seq):
+@pytest.mark.parametrize("seq,kind", [(2048, "short"), (4096, "single")])
+def test_baseline_prefill_full(seq, kind):
     q, k, v = make_inputs(1, 32, 8, seq, seq, 128, device=DEV)
-    assert _route(q, k).kind == "single"
+    assert _route(q, k).kind == kind
     out = _run(q, k, v)
     assert_close(out, oracle(q, k, v), BASELINE_TOL[torch.bfloat16], f"prefill {seq}")
 
@@ -324,6 +325,17 @@ def test_fully_masked_rows_are_nan():
 # tiles exceed the running reference, so it is raised mid-row) and scores
 # large enough that exponentials against a stale reference overflow.
 # --------------------------------------------------------------------------
+def _every_single_pass(q, k, v, causal=True):
+    """(name, output) of the routed call, the single pass with none, some and
+    all of its blocks as key halves, and the short form."""
+    from gqa_kernels.dispatch import short_forward, single_pass_forward
+    yield "routed", _run(q, k, v, causal)
+    blocks = -(-q.shape[2] // (256 // (q.shape[1] // k.shape[1])))
+    for n_split in (0, blocks // 2, blocks):
+        yield f"single, {n_split} split", single_pass_forward(q, k, v, torch.empty_like(q), causal, n_split)
+    yield "short", short_forward(q, k, v, torch.empty_like(q), causal)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [True, False])
@@ -331,9 +343,9 @@ def test_growing_scores(D, causal, dtype):
     q, k, v = make_inputs(1, 8, 2, 1024, 1024, D, torch.float32)
     ramp = 0.1 + 4.0 * torch.arange(1024, dtype=torch.float32) / 1024
     q, k, v = (t.to(dtype).to(DEV) for t in (q, k * ramp[None, None, :, None], v))
-    assert _route(q, k).kind == "single"
-    out = _run(q, k, v, causal)
-    assert_close(out, oracle(q, k, v, causal, dtype=np.float64), BASELINE_TOL[dtype], "growing scores")
+    ref = oracle(q, k, v, causal, dtype=np.float64)
+    for name, out in _every_single_pass(q, k, v, causal):
+        assert_close(out, ref, BASELINE_TOL[dtype], f"growing scores, {name}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -342,8 +354,9 @@ def test_large_scores(D, dtype):
     q, k, _ = make_inputs(1, 8, 2, 512, 512, D, torch.float32, scale=4.0)
     _, _, v = make_inputs(1, 8, 2, 512, 512, D, torch.float32, seed=1)
     q, k, v = (t.to(dtype).to(DEV) for t in (q, k, v))
-    out = _run(q, k, v)
-    assert_close(out, oracle(q, k, v, dtype=np.float64), BASELINE_TOL[dtype], "large scores")
+    ref = oracle(q, k, v, dtype=np.float64)
+    for name, out in _every_single_pass(q, k, v):
+        assert_close(out, ref, BASELINE_TOL[dtype], f"large scores, {name}")
 
 
 def test_empty_query():

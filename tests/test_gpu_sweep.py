@@ -9,8 +9,8 @@ single-token decode, multi-token verify, chunked prefill and prefill at
 ragged lengths, contiguous and (batch, seq, head, d) strided layouts, and
 causal calls with more queries than keys (their leading rows see no key:
 NaN in both, as the reference's softmax over an all -inf row).  Every case
-goes through choose_route, so the split-KV, single-pass, key-split and
-key-chunk routes all meet odd shapes.  Shapes come from a fixed seed, so a
+goes through choose_plan, so the split-KV, flat, single-pass, key-split,
+key-chunk and short routes all meet odd shapes.  Shapes come from a fixed seed, so a
 failure names a reproducible case; each is sized for the oracle to finish in
 well under a second.
 """
@@ -107,10 +107,10 @@ def _compare(got, ref, tol, what):
 @pytest.mark.parametrize("case", CASES, ids=[_ids(c) for c in CASES])
 def test_sweep(case):
     from gqa_kernels import gqa_flash_attn
-    from gqa_kernels.dispatch import _cu_count, choose_route
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     B, Hq, Hkv, Sq, Skv, D, dtype_s, causal, kind, layout, want_lse = case
     dtype = torch.bfloat16 if dtype_s == "bf16" else torch.float16
-    route = choose_route(B, Hq, Hkv, Sq, Skv, _cu_count(0), causal, D)
+    route = choose_plan(B, Hq, Hkv, Sq, Skv, _cu_count(0), causal, D)
     print(f"sweep {_ids(case)} route={route}", flush=True)
     g = torch.Generator(device="cpu").manual_seed(Sq * 7919 + Skv)
     q = _draw(B, Hq, Sq, D, dtype, layout, g)

@@ -400,8 +400,8 @@ def main() -> int:
                    warm_ms=WARM_MS)
         by = hbm_bytes(B, HQ, HKV, 1, DECODE_S, D)
         gbs = by / (ms * 1e-3) / 1e9
-        from gqa_kernels.dispatch import _cu_count, choose_route
-        route = choose_route(B, HQ, HKV, 1, DECODE_S, _cu_count(0), causal=True, head_dim=D)
+        from gqa_kernels.dispatch import _cu_count, choose_plan
+        route = choose_plan(B, HQ, HKV, 1, DECODE_S, _cu_count(0), causal=True, head_dim=D)
         result["decode"] = {
             "workload": f"causal GQA decode B={B} Hq={HQ} Hkv={HKV} D={D} seq_q=1 seq_kv={DECODE_S}",
             "us": ms * 1e3, "gbs": gbs, "steps": dsteps, "splits": route.splits,
@@ -573,7 +573,7 @@ def sweep(torch, gqa_flash_attn, steps=20, warmup=5, only=None, table=CONFIGS):
     least WARM_MS of untimed calls, with
     TFLOP/s, HBM GB/s and the fraction of the roofline that bounds the
     config.  HBM-bound configs rotate K/V sets (ROTATE_BYTES in total)."""
-    from gqa_kernels.dispatch import _cu_count, choose_route
+    from gqa_kernels.dispatch import _cu_count, choose_plan
     rows = []
     sel = table
     if only is not None:  # the config of that exact name, else those starting with it
@@ -595,10 +595,10 @@ def sweep(torch, gqa_flash_attn, steps=20, warmup=5, only=None, table=CONFIGS):
         tflops, gbs = fl / (ms * 1e-3) / 1e12, by1 / (ms * 1e-3) / 1e9
         achieved, peak, unit = (tflops, PEAK_BF16_TFLOPS, "TFLOP/s") if bound == "mfma" else \
             (gbs, PEAK_HBM_GBS, "GB/s")
-        route = choose_route(b, hq, hkv, sq, skv, _cu_count(0), causal=True, head_dim=d)
+        route = choose_plan(b, hq, hkv, sq, skv, _cu_count(0), causal=True, head_dim=d)
         rows.append({"config": name, "B": b, "Hq": hq, "Hkv": hkv, "seq_q": sq, "seq_kv": skv, "D": d,
                      "dtype": dtype_s, "return_lse": lse, "us": ms * 1e3, "tflops": tflops, "gbs": gbs, "steps": n, "kv_sets": nset,
-                     "route": route.kind + (f" splits={route.splits}" if route.kind in ("split", "chunks") else
+                     "route": route.kind + (f" splits={route.splits}" if route.kind in ("split", "chunks", "flat") else
                                             f" key-split blocks={route.fwd_split}" if route.fwd_split else ""),
                      "roofline": {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit,
                                   "frac": achieved / peak, "flops_per_call": fl, "bytes_per_call": by1}})

@@ -416,9 +416,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // step with the others, concentrating the concurrent reads on a subset of
   // the HBM channels; splits s = 0..3 (mod 4) start a quarter of the chunk
   // apart.  The online softmax does not depend on the order.
-  // Tiles past the chunk (the prologue's tiles of a chunk shorter than two,
-  // the padding of an odd count) are not rotated: they lie beyond the
-  // descriptors, read as zero and are fully masked.
+  // Tiles past the chunk (the prologue's, of a chunk shorter than two) are not
+  // rotated: they lie beyond the descriptors and read as zero.
   const int rot = (p.rotate && ntiles >= 4) ? (s & 3) * (ntiles >> 2) : 0;
   auto tile_rel = [&](int it) {
     const int j = it + rot;

@@ -232,10 +232,11 @@ hipError_t launch_split_first(const SplitParams& p, int dtype, hipStream_t strea
 hipError_t launch_paged_split_first(const SplitParams& p, int dtype, hipStream_t stream);
 hipError_t launch_paged_cache_write(const CacheWriteParams& p, hipStream_t stream);
 hipError_t launch_split_reduce(const ReduceParams& p, int dtype, hipStream_t stream);
-// Decode-shaped first pass (gqa_decode.hip): head_dim 128, contiguous K/V,
-// fixed query lengths, 32-bit chunk and workspace offsets.
-// Keys of one of its tile steps, the unit of a flat split.
+// Keys of one tile step of the decode-shaped first pass, the unit of a flat
+// split.
 constexpr int decode_unit(int head_dim) { return head_dim == 64 ? 128 : 64; }
+// Decode-shaped first pass (gqa_decode.hip): whether it takes these rows,
+// pages, strides and workspace offsets.
 bool decode_kernel_fits(const SplitParams& p);
 hipError_t launch_decode_first(const SplitParams& p, int dtype, hipStream_t stream);  // fused if p.counters
 

@@ -20,7 +20,7 @@ from . import _lib
 from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces, decode_forward,
                         flat_forward, stream_handle)
 
-__all__ = ["gqa_flash_attn", "Route", "choose_route"]
+__all__ = ["gqa_flash_attn", "Route", "choose_plan", "choose_route"]
 
 LOG2E = math.log2(math.e)
 

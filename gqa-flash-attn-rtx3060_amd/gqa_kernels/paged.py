@@ -204,7 +204,8 @@ def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     the whole of max_seq_len, by steps a piece: at head_dim 128 up to one
     sequence a range 4-7 1.08 and 1.09, 7-10 1.03 and 1.08, 10-16 0.99 and 0.94,
     16-32 0.96 and 0.88, more 0.96 and 0.79 (fewer than 5 sequences 10-16 1.02
-    and 0.96, more 1.00 and 0.89); two 10-16 1.03 and 0.98, 16-32 1.00 and 0.94,
+    and 0.96, more 1.00 and 0.89; 17-32 rows 10-16 up to 1.13, 6 x 8 tokens over
+    4160 keys 28.1 -> 31.8); two 10-16 1.03 and 0.98, 16-32 1.00 and 0.94,
     more 0.98 and 0.86; four 16-32 1.04 and 0.98, more 1.00 and 0.89; more than
     four 1.0-1.4.  At head_dim 64 up to one 10-16 1.02 and 0.93, 16-32 1.02 and
     0.90, more 0.93 and 0.87; one token over interleaved heads, which the
@@ -218,7 +219,7 @@ def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     least = _FLAT_MIN_PIECE
     if batch > 2 * slots or (head_dim == 64 and heads_interleaved and seq_q == 1):
         least *= 2
-    elif head_dim == 128 and 5 <= batch <= slots:
+    elif head_dim == 128 and 5 <= batch <= slots and rows <= _DEC16_ROWS:
         least = _FLAT_MIN_PIECE_WIDE
     return slots if flat_piece_steps(batch, max_seq_len, slots, head_dim) >= least else 0
 

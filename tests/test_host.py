@@ -494,6 +494,12 @@ def test_paged_flat_rule(batch, keys, head_dim, interleaved, flat):
     assert paged_flat_slots(batch, 32, 8, 1, keys, 256, 16, head_dim, interleaved) == (32 if flat else 0)
 
 
+@pytest.mark.parametrize("seq_q,keys,flat", [(4, 4160, True), (8, 4160, False), (8, 8192, True), (9, 8192, False)])
+def test_paged_flat_rule_by_rows(seq_q, keys, flat):
+    from gqa_kernels.paged import paged_flat_slots
+    assert paged_flat_slots(6, 32, 8, seq_q, keys, 256) == (32 if flat else 0)
+
+
 @pytest.mark.parametrize("shape,head_dim,kind", [
     ((5, 32, 8, 4, 1527), 64, "split"), ((20, 16, 4, 4, 1910), 128, "split"), ((11, 8, 8, 4, 1039), 128, "split"),
     ((5, 32, 8, 1, 8192), 128, "flat"), ((20, 32, 8, 1, 3000), 128, "flat"), ((33, 32, 8, 1, 3000), 128, "flat")])

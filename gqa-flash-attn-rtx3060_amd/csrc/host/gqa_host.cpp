@@ -571,6 +571,7 @@ double list_makespan(const std::vector<double>& cost, const std::vector<int64_t>
     if (cnt == 0 || std::find(seen.begin(), seen.end(), key) != seen.end()) continue;
     seen.push_back(key);
     if (fixed) {
+      if (slots < 1) throw std::invalid_argument("list_makespan: fewer than eight CUs");
       // Rows of `slots` items dealt left to right, the odd ones right to left.
       loads.assign(static_cast<size_t>(slots), 0.0);
       for (int64_t e = 0; e < cnt; ++e) {

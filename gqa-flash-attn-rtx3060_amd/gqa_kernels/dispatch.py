@@ -124,10 +124,9 @@ FWD_SPLIT_GAIN = 0.05
 # splits nothing: two workgroups share a CU there, so nearly all start
 # together and the heaviest block, which the model deals one to a CU, ends
 # last, alone on its CU.  Prompts have the heaviest of each (b, kv head) split,
-# eight an XCD in all, for at most HEAD_PAIRS (b, kv head) pairs per XCD and
-# blocks per CU; the blocks of a chunk over a long cache are nearly as long as
-# each other and only get shorter waits, so the cache is at most HEAD_KV times
-# the chunk (more with few blocks).  Measured, us, whole / split, (b, kv head)
+# eight an XCD in all, up to so many ((b, kv head) pairs per XCD, blocks per
+# CU); the blocks of a chunk over a long cache are nearly as long as each
+# other, so up to (blocks per CU, keys per query).  Measured, us, whole / split,
 # pairs x blocks: 8 x 35 2200 tokens 43.0 / 36.2, over 4400 keys 91.7 / 79.7;
 # 8 x 64 4096 tokens 91.0 / 82.7, over 5120 keys 124.5 / 116.1, 8192 222 / 226,
 # 16384 482 / 521; 8 x 79 5000 tokens 123.5 / 114.9; 16 x 18 1100 tokens 26.3 /

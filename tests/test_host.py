@@ -547,6 +547,13 @@ def test_head_split_at_head_dim_64(batch, seq_q, seq_kv, split):
     assert plan.kind != "single" or plan.fwd_split == split
 
 
+def test_dealt_pairs_as_the_kernel_counts_them():
+    from gqa_kernels import dispatch
+    text = (REPO / "gqa-flash-attn-rtx3060_amd" / "csrc" / "gqa_params.hpp").read_text()
+    m = re.search(r"kDealPairs\(int head_dim\) \{ return head_dim == 64 \? \d+ : (\d+); \}", text)
+    assert m and int(m.group(1)) == dispatch.FWD_DEAL_PAIRS
+
+
 def test_native_makespan_equals_python(monkeypatch):
     """The routing models' schedules in C++ against the Python that states them,
     and whole plans with and without the bindings."""

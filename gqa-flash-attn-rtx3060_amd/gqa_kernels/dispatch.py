@@ -577,10 +577,15 @@ def _choose_route(batch, num_heads, num_kv_heads, seq_q, seq_kv, cu_count, causa
     return Route("single", 1, single_wgs + ns * num_kv_heads * batch, ns)
 
 
+def flat_steps(seq_kv: int, head_dim: int = 128) -> int:
+    """Tile steps of a sequence's keys under the flat split."""
+    return _cdiv(seq_kv, 128 if head_dim == 64 else 64)
+
+
 def flat_piece_steps(batch: int, seq_kv: int, slots: int, head_dim: int = 128) -> float:
     """Tile steps of a piece of a flat split over `slots` ranges: every range
     is one piece, and one more for each sequence that it crosses into."""
-    return batch * _cdiv(seq_kv, 128 if head_dim == 64 else 64) / (slots + batch)
+    return batch * flat_steps(seq_kv, head_dim) / (slots + batch)
 
 
 def flat_max_rows(head_dim: int = 128) -> int:

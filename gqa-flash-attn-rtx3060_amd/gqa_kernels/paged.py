@@ -41,7 +41,7 @@ import torch
 
 from . import _lib
 from .dispatch import (_KIND_IDS, FWD_ROWS, SPLIT_MIN_KV, _fwd_block_tiles, choose_fwd_split, choose_kv_chunks, flat_max_rows,
-                       flat_piece_steps, fwd_split_makespan, use_short)
+                       flat_piece_steps, flat_steps, fwd_split_makespan, use_short)
 from .gqa_split import (_counter_buffer, _counters, _decode_host, _workspace_buffer, _workspaces,
                         flat_workspace_bytes, stream_handle, workspace_bytes)
 
@@ -102,9 +102,13 @@ _SPLIT_WG_PER_CU = 2
 _LDS_WG_PER_CU = 1
 _LDS_WG_PER_CU_INTERLEAVED = 4
 _MIN_CHUNK = 256
-# Tile steps a piece of the flat split keeps (paged_flat_slots).
-_FLAT_MIN_PIECE = 16
-_FLAT_MIN_PIECE_WIDE = 10
+# Tile steps a piece of the flat split keeps, and steps that its ranges are
+# shorter than the fixed count's chunks (paged_flat_slots): head_dim 64,
+# head_dim 128 up to 16 packed rows, 17-32 rows.
+_FLAT_MIN_PIECE = {64: 8, 128: 10}
+_FLAT_MIN_PIECE_WIDE = 12
+_FLAT_MIN_SAVED = {64: 2, 128: 3}
+_FLAT_MIN_SAVED_WIDE = 6
 _SPLIT_MAX_ROWS = 64  # packed rows per kv head up to which the split-KV pass is used
 _SPLIT_MAX_ROWS_WIDE = 128  # ... at head_dim 128 with pages of >= 4 keys (128-row workgroups)
 _DEC16_ROWS = 16  # packed rows up to which head_dim 64 runs the LDS-DMA first pass
@@ -192,36 +196,51 @@ def paged_flat_slots(batch: int, num_heads: int, num_kv_heads: int, seq_q: int, 
     Cutting every sequence alike leaves a batch of unequal lengths waiting
     for its longest sequences; the flat split gives every workgroup the same
     number of keys, read from the lengths on the device.  One workgroup per
-    compute unit (two or four measured the same or slower).  Each piece of a
-    range costs its own start, so pieces have to keep _FLAT_MIN_PIECE tile
-    steps, more with many sequences to a range, whose fixed split hands out
-    more workgroups than the device holds.  Measured on MI355X (bf16, us, fixed
-    -> flat): 16-key token-major pages, one token, B = 32 of 100-8000 keys
-    111.7 -> 94.2, B = 16 of 500-16000 112.0 -> 93.5, B = 64 of 100-4000 114.4 ->
-    97.8, B = 14 of 600-6000 45.2 -> 37.5, 4 tokens B = 8 of 100-8000 37.2 ->
-    28.9; head-major 64-key pages, B = 8 of 1000-30000 114.7 -> 80.9.  900 batches,
+    compute unit (two or four measured the same or slower).  A piece of a
+    range costs its own start and merge, so the flat split is taken where
+    pieces keep _FLAT_MIN_PIECE tile steps (twice that, three times with 17-32
+    rows, from two sequences a range on, whose fixed split hands out more
+    workgroups than the device holds; four sequences a range are its end), and
+    where the fixed count leaves the device idle: chunks of at least
+    _FLAT_MIN_SAVED steps more than a range has (one more if the fixed count is
+    one chunk a sequence, whose workgroups write no partials).
+    Measured on MI355X (bf16, us, fixed -> flat): 16-key token-major pages, one
+    token, B = 32 of 100-8000 keys 111.7 -> 94.2, B = 16 of 500-16000 112.0 ->
+    93.5, B = 64 of 100-4000 114.4 -> 97.8, B = 14 of 600-6000 45.2 -> 37.5, 4
+    tokens B = 8 of 100-8000 37.2 -> 28.9, B = 2 of 1213 and 1956 14.3 -> 10.0;
+    head-major 64-key pages, B = 8 of 1000-30000 114.7 -> 80.9.  2400 batches,
     flat / fixed in the mean, equal lengths and lengths drawn from a tenth to
-    the whole of max_seq_len, by steps a piece: at head_dim 128 up to one
-    sequence a range 4-7 1.08 and 1.09, 7-10 1.03 and 1.08, 10-16 0.99 and 0.94,
-    16-32 0.96 and 0.88, more 0.96 and 0.79 (fewer than 5 sequences 10-16 1.02
-    and 0.96, more 1.00 and 0.89; 17-32 rows 10-16 up to 1.13, 6 x 8 tokens over
-    4160 keys 28.1 -> 31.8); two 10-16 1.03 and 0.98, 16-32 1.00 and 0.94,
-    more 0.98 and 0.86; four 16-32 1.04 and 0.98, more 1.00 and 0.89; more than
-    four 1.0-1.4.  At head_dim 64 up to one 10-16 1.02 and 0.93, 16-32 1.02 and
-    0.90, more 0.93 and 0.87; one token over interleaved heads, which the
-    fixed count gives four workgroups per CU, 16-32 up to 1.09."""
+    the whole of max_seq_len, by steps a piece up to two sequences a range:
+    head_dim 128 up to 16 rows 6-8 1.06 and 1.00, 8-10 1.03 and 0.95, 10-12
+    1.02 and 0.93, 12-16 0.99 and 0.90, 32 on 0.95 and 0.82; 17-32 rows 8-10
+    1.09 and 1.10, 12-16 0.99 and 0.93; head_dim 64 6-8 1.03 and 0.96, 8-10 0.99
+    and 0.91, 20-32 0.96 and 0.82.  Two to four sequences a range: head_dim 128
+    12-16 1.06 and 0.98, 18-24 1.03 and 0.93, 17-32 rows 24-32 1.08 and 1.02;
+    head_dim 64 12-16 1.05 and 0.97, 16-18 0.94 and 0.91.  By steps saved, under
+    8 a piece: head_dim 128 2-2.5 1.11 and 1.04, 3-4 0.99 and 0.91, 4-6 0.88 and
+    0.85 (one chunk a sequence 3-4 0.95 and 0.95, yet 1.12 with all lengths far
+    under max_seq_len, 4-5 0.91, 0.86 and 1.03); 17-32 rows 4-6 1.01 and 0.99,
+    more 0.84 and 0.84; head_dim 64 1.5-2 1.07 and 0.99, 2-2.5 0.96 and 0.95."""
     rows = num_heads // num_kv_heads * seq_q
     if batch < 2 or max_seq_len < 1 or block_size < single_pass_min_block(head_dim):
         return 0
     slots = cu_count // num_kv_heads
     if not 0 < rows <= flat_max_rows(head_dim) or not 1 <= slots <= _lib.GQA_MAX_SPLITS or batch > 4 * slots:
         return 0
-    least = _FLAT_MIN_PIECE
-    if batch > 2 * slots or (head_dim == 64 and heads_interleaved and seq_q == 1):
-        least *= 2
-    elif head_dim == 128 and 5 <= batch <= slots and rows <= _DEC16_ROWS:
-        least = _FLAT_MIN_PIECE_WIDE
-    return slots if flat_piece_steps(batch, max_seq_len, slots, head_dim) >= least else 0
+    wide = rows > _DEC16_ROWS
+    least = _FLAT_MIN_PIECE_WIDE if wide else _FLAT_MIN_PIECE[head_dim]
+    if batch > 2 * slots:
+        least *= 3 if wide else 2
+    if flat_piece_steps(batch, max_seq_len, slots, head_dim) >= least:
+        return slots
+    if batch > 2 * slots:
+        return 0
+    splits = paged_splits(batch, num_heads, num_kv_heads, seq_q, max_seq_len, cu_count, block_size, head_dim,
+                          heads_interleaved)
+    steps = flat_steps(max_seq_len, head_dim)
+    saved = -(-steps // splits) - batch * steps / slots
+    least = (_FLAT_MIN_SAVED_WIDE if wide else _FLAT_MIN_SAVED[head_dim]) + (splits == 1)
+    return slots if saved >= least else 0
 
 
 def _paged_host():

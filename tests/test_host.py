@@ -483,21 +483,26 @@ def test_fwd_split_measured_choices():
 
 
 @pytest.mark.parametrize("batch,keys,head_dim,interleaved,flat", [
-    (2, 2048, 128, True, False), (4, 32768, 128, True, True), (4, 8192, 128, True, False),  # pieces of few steps
+    (2, 2048, 128, True, False), (4, 32768, 128, True, True), (3, 3807, 128, True, False),  # pieces of few steps
     (12, 600, 128, True, False), (12, 8192, 128, True, True), (8, 2048, 128, True, False),
     (32, 128, 128, True, False), (32, 2048, 128, True, True), (64, 600, 128, True, False),
     (64, 4096, 128, True, True), (128, 600, 128, True, False), (128, 4096, 128, True, True),
     (256, 4096, 128, True, False),                                                          # many workgroups as it is
-    (8, 16000, 64, True, False), (8, 16000, 64, False, True), (12, 32768, 64, True, True)])
+    (8, 16000, 64, True, True), (8, 4000, 64, False, False), (12, 32768, 64, True, True),
+    (65, 1600, 128, True, False), (64, 1600, 128, True, True),                              # twice the steps from 65 on
+    (2, 700, 128, True, True), (3, 1200, 128, True, True), (24, 900, 128, True, False),     # few long chunks
+    (6, 256, 128, True, False), (6, 257, 128, True, True), (3, 512, 64, False, False), (3, 513, 64, False, True)])
 def test_paged_flat_rule(batch, keys, head_dim, interleaved, flat):
     from gqa_kernels.paged import paged_flat_slots
     assert paged_flat_slots(batch, 32, 8, 1, keys, 256, 16, head_dim, interleaved) == (32 if flat else 0)
 
 
-@pytest.mark.parametrize("seq_q,keys,flat", [(4, 4160, True), (8, 4160, False), (8, 8192, True), (9, 8192, False)])
-def test_paged_flat_rule_by_rows(seq_q, keys, flat):
+@pytest.mark.parametrize("batch,seq_q,keys,flat", [
+    (6, 4, 4160, True), (6, 8, 4160, False), (6, 8, 8192, True), (6, 9, 8192, False),
+    (65, 4, 2000, True), (65, 5, 2000, False), (2, 4, 448, True), (2, 5, 448, False), (2, 5, 449, True)])
+def test_paged_flat_rule_by_rows(batch, seq_q, keys, flat):
     from gqa_kernels.paged import paged_flat_slots
-    assert paged_flat_slots(6, 32, 8, seq_q, keys, 256) == (32 if flat else 0)
+    assert paged_flat_slots(batch, 32, 8, seq_q, keys, 256) == (32 if flat else 0)
 
 
 @pytest.mark.parametrize("shape,head_dim,kind", [

@@ -30,10 +30,13 @@ namespace gqa {
 //   in each L2.
 // * Many pairs per XCD (kDealPairs): nothing is shared in L2 any more.  Paged
 //   head_dim 128, 34 pairs, 197 tokens over 2755 keys 358 / 418, 28 pairs 183
-//   over 8184 662 / 727, 18 pairs 659 over 689 115 / 123; contiguous 28 pairs
-//   376 over 4341 1.20 times; head_dim 64 36 pairs 134 over 7635 448 / 509, 32
-//   pairs 295 over 10192 777 / 916.  Up to 12 (24 at head_dim 64) 90 shapes
-//   are faster by 6 % in the mean.
+//   over 8184 662 / 727; contiguous 28 pairs 376 over 4341 1.20 times; head_dim
+//   64 36 pairs 134 over 7635 448 / 509.  Means of dealt / pair after pair,
+//   head_dim 128 with 13-24 pairs: paged, equal lengths 1.00 (22 pairs 659 over
+//   689 keys 1.07), unequal 0.93 (568 tokens over 590-4076 484 / 399), contiguous
+//   0.98 (14 pairs 168 tokens 26.4 / 21.7); with 25-32: 1.04, 0.96 and 1.06.
+//   head_dim 64 with 25-32: 0.97, 0.94 and 0.98 (worst 295 over 10192 1.17);
+//   with more, equal lengths 1.06.
 // * At most one item per CU, all start together: paged head_dim 64, 13 pairs
 //   21.8 / 23.5, 14 pairs 20.2 / 21.7; contiguous 10 pairs 13.0 / 14.0.
 // * Key chunks, paged head_dim 128: 97 tokens of [4223, 9688] keys 49.5 / 44.7,

@@ -197,7 +197,7 @@ inline void set_item_order(FwdParams& p, int per_bh, bool deal, int max_pairs) {
 }
 // Pairs an XCD takes side by side before their K and V no longer share its L2
 // (measured in gqa_fwd_parts.hpp, item_of).
-constexpr int kDealPairs(int head_dim) { return head_dim == 64 ? 24 : 12; }
+constexpr int kDealPairs(int head_dim) { return head_dim == 64 ? 32 : 24; }
 
 // Paged cache write: new tokens (num_tokens, Hkv, D) into
 // (num_blocks, block_size, Hkv, D) caches at slot_mapping[t].

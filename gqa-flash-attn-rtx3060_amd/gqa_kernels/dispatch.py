@@ -168,7 +168,7 @@ FWD_FILL_MERGE_OVERHEAD = 4
 FWD_TILE = 64
 # Pairs per XCD up to which the head_dim-128 single pass deals them (kDealPairs,
 # gqa_params.hpp).
-FWD_DEAL_PAIRS = 12
+FWD_DEAL_PAIRS = 24
 # The persistent single pass claims work dynamically only with at least this
 # many items per workgroup (kFwdDynMinItemsPerWg, gqa_params.hpp); below it
 # every workgroup takes a fixed list (gqa_fwd.hip item_at: XCD x's

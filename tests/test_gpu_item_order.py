@@ -49,8 +49,9 @@ def test_ragged_paged_order(lens, D, route, splits):
     _check(o, lse, q, kc, vc, table, seq_lens, True, torch.bfloat16)
 
 
-@pytest.mark.parametrize("B,D,sq", [(3, 64, 800), (2, 64, 2100), (24, 64, 200), (25, 64, 200), (3, 128, 900),
-                                    (12, 128, 333), (13, 128, 333)])
+@pytest.mark.parametrize("B,D,sq", [(3, 64, 800), (2, 64, 2100), (24, 64, 200), (25, 64, 200), (32, 64, 200),
+                                    (33, 64, 200), (3, 128, 900), (12, 128, 333), (13, 128, 333),
+                                    (24, 128, 333), (25, 128, 333)])
 @pytest.mark.parametrize("causal,n_split", [(True, 0), (True, 2), (False, 0), (False, 2)])
 def test_order_does_not_change_results(B, D, sq, causal, n_split):
     """More items than CUs, on both sides of the line where pairs are dealt: each

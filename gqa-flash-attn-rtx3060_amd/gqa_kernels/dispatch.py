@@ -663,10 +663,15 @@ def _short_share(kv_chunks: int, paged: bool, wgs_per_cu: float) -> float:
     chunks in us: contiguous, up to 4 chunks, 128 or more workgroups 0.95 44.7 /
     49.9, 0.96 0.83 times, fewer 0.88 37.6 / 41.4, 0.96 1.08 times, 0.98 1.29
     times; 8 chunks 0.80 22.8 / 24.9, 0.90 19.1 / 16.3, 0.99 27.0 / 21.8; paged,
-    up to 4 0.84 0.86 times, 0.90 1.05 times, 8 0.78 0.87 times, 0.91 23.0 / 16.9;
-    paged with 8-28 workgroups 0.65-0.70 1.0-1.22 times."""
+    4 0.84 0.86 times, 0.90 1.05 times, 8 0.78 0.87 times, 0.91 23.0 / 16.9;
+    paged with 8-28 workgroups 0.65-0.70 1.0-1.22 times.  Two paged chunks, 128
+    or more workgroups, equal / unequal lengths: 0.86 146.6 / 155.7 and 114.7 /
+    140.1, 0.87 132.0 / 133.8 and 111.0 / 117.5, 0.94 119.7 / 119.6 and 95.2 /
+    102.5, 0.98 184.9 / 179.5 and 138.6 / 149.4."""
     if not kv_chunks:
         return 1.0
+    if paged and kv_chunks == 2 and wgs_per_cu >= 0.5:
+        return 0.95
     if paged or kv_chunks >= 8:
         return 0.0 if wgs_per_cu < 0.125 else 0.9 - 0.05 * paged - 0.05 * (kv_chunks >= 8)
     return 1.0 if wgs_per_cu >= 0.5 else 0.9

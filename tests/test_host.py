@@ -528,8 +528,9 @@ def test_short_form_of_contiguous_calls(shape, causal, head_dim, kind):
 
 @pytest.mark.parametrize("batch,seq_q,keys,head_dim,short", [
     (4, 20, 2048, 64, False), (2, 30, 1675, 64, False), (3, 80, 3970, 64, False), (2, 163, 4791, 64, False),
-    (9, 36, 10097, 128, False), (6, 7, 1490, 64, False),  # chunks, and the split-KV pass, measured faster
+    (11, 44, 13021, 128, False), (6, 7, 1490, 64, False),  # chunks, and the split-KV pass, measured faster
     (11, 78, 78, 128, False), (52, 21, 21, 64, False),    # a second round of short workgroups
+    (15, 49, 12448, 64, True), (9, 36, 10097, 128, True),  # two chunks
     (16, 20, 2048, 64, True), (5, 48, 1738, 64, True), (12, 5, 1224, 64, True), (2, 512, 5262, 128, True)])
 def test_short_form_of_paged_calls(batch, seq_q, keys, head_dim, short):
     from gqa_kernels.paged import paged_short

@@ -778,7 +778,8 @@ static hipError_t launch_fwd_t(FwdParams p, hipStream_t stream) {
   else if (PG == 0 && !p.dm.causal)
     set_item_order(p, per_bh, p.n_split > 0, p.dm.B * p.dm.Hkv);
   else
-    set_item_order(p, per_bh, total > cus && (PG > 0 || D == 64 || fixed_lists), kDealPairs(D));
+    set_item_order(p, per_bh, (PG > 0 && D == 128) || (total > cus && (PG > 0 || D == 64 || fixed_lists)),
+                   kDealPairs(D));
   p.div_mblk = make_fast_div((uint32_t)p.n_mblk);
   p.div_hkv = make_fast_div((uint32_t)p.dm.Hkv);
   p.bm_mul = (65536u + (uint32_t)p.block_m - 1) / (uint32_t)p.block_m;

@@ -38,7 +38,10 @@ namespace gqa {
 //   head_dim 64 with 25-32: 0.97, 0.94 and 0.98 (worst 295 over 10192 1.17);
 //   with more, equal lengths 1.06.
 // * At most one item per CU, all start together: paged head_dim 64, 13 pairs
-//   21.8 / 23.5, 14 pairs 20.2 / 21.7; contiguous 10 pairs 13.0 / 14.0.
+//   21.8 / 23.5, 14 pairs 20.2 / 21.7; contiguous 10 pairs 13.0 / 14.0.  Paged
+//   head_dim 128 only the spread over the XCDs counts: 8 x 200 tokens over
+//   2850-26921 keys 645 / 554, 32 batches of up to 12 pairs with unequal lengths 0.96-0.99
+//   in the mean, equal ones and more pairs within 1 %.
 // * Key chunks, paged head_dim 128: 97 tokens of [4223, 9688] keys 49.5 / 44.7,
 //   equal lengths alike; head_dim 64 35 tokens over 1981 keys 18.9 / 22.6, 127
 //   over 4834 32.9 / 35.7, so pair after pair there.

@@ -94,7 +94,9 @@ _DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 # 122.8 -> 120.0, head-major 1 -> 4 113.5 -> 116.7 (8 splits: 119.9, so the
 # workgroup cap); eight such batches 929 -> 887 us in all.  Uniform lengths
 # pay: B = 32 x 4096 head-major 82.8 -> 88.5, B = 8 x 16384 82.9 -> 84.9
-# (four uniform batches 345 -> 353 us).
+# (four uniform batches 345 -> 353 us).  These batches of one token take the flat
+# split now (paged_flat_slots); the counts are for the ones it leaves: more
+# packed rows, shorter sequences, strides it does not address.
 _BATCH_MIN_SPLITS = 8
 _BATCH_MAX_WG_PER_CU = 8
 _SPLIT_ROWS = 32
